@@ -164,7 +164,7 @@ struct fxc_plan {
     DevBuf tw_l1, tw_l2, tw_lm, d_x[2], d_y, d_z[2], d_params, d_lshifts;
     DevBuf tw_l0;   // W_64 (the fused four-step's rows at N = 16384)
     // scratch
-    DevBuf part, red_scratch, table_dev, d_raw[2], d_acc, d_raw_out, d_tmp_in, d_tmp_out,
+    DevBuf part, table_dev, d_raw[2], d_acc, d_raw_out, d_tmp_in, d_tmp_out,
         d_shifts, d_cb, d_tbuf;
     DevBuf d_chain;          // the reference's f32 phase chains of one slab/chunk of frames
     DevBuf d_fringe;         // one chunk's products for the whole-scan cross spectrum
@@ -188,7 +188,7 @@ struct fxc_plan {
     template <class Fn> void each_buf(Fn fn) {
         DevBuf *bufs[] = {&tw_fft, &tw_post, &lev_dev[0], &lev_dev[1], &out_lev, &mf_tab,
                           &tw_l1, &tw_l2, &tw_lm, &tw_l0, &d_x[0], &d_x[1], &d_y, &d_z[0], &d_z[1],
-                          &d_params, &d_lshifts, &part, &red_scratch, &table_dev, &d_raw[0],
+                          &d_params, &d_lshifts, &part, &table_dev, &d_raw[0],
                           &d_raw[1], &d_acc, &d_raw_out, &d_tmp_in, &d_tmp_out, &d_shifts,
                           &d_cb, &d_tbuf, &d_chain, &d_fringe, &d_err, &d_cacc};
         for (DevBuf *b : bufs) fn(*b);
@@ -956,7 +956,6 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
                                    : std::max(64, (cus * 1024) / p->T);
     if ((p->fft_form == 1 && p->d_cacc.ensure((size_t)p->max_wg * kMfConsumerAccBytes) != hipSuccess) ||
         p->part.ensure((size_t)p->max_wg * kNumProducts * half * sizeof(double)) != hipSuccess ||
-        p->red_scratch.ensure((size_t)64 * kNumProducts * half * sizeof(double)) != hipSuccess ||
         p->d_err.ensure(sizeof(int32_t)) != hipSuccess)
         return cleanup(fail(FXC_ERR_NOMEM, "scratch allocation failed"));
     if (hipMemset(p->d_err.p, 0, sizeof(int32_t)) != hipSuccess)
@@ -1282,6 +1281,19 @@ static bool xcf_uses_chain(const fxc_plan *p) {
 }
 constexpr size_t kChainSlabBytes = (size_t)256 << 20;   // chain scratch of the fused plain path
 
+// Frames per workgroup of the fused kernels for a launch of nf frames on at
+// most wg_cap workgroups.  Stockham kernels (one frame pair at a time per
+// workgroup): as few as the cap allows, so that a short launch spreads over
+// the chip; a frame pair alone takes about 8 us of latency at N = 1024, and a
+// 150-frame sector on 19 workgroups of 8 frames took 64 us where 150
+// workgroups take 20.  MFMA kernels: whole frames per producer wave, eight a
+// workgroup, which run side by side.
+static int64_t frames_per_wg(const fxc_plan *p, int64_t nf, int64_t wg_cap) {
+    const int64_t fpw = std::max<int64_t>(1, (nf + wg_cap - 1) / wg_cap);
+    const int64_t batch = p->fft_form == 1 ? 8 : 1;
+    return (fpw + batch - 1) / batch * batch;
+}
+
 // Long phase chains of the chunked paths (phased, large-N plain) are
 // computed for a span of whole chunks at a time, up to this much table: each
 // chain is one thread's sequential walk, so the frames of one chunk alone (a
@@ -1317,9 +1329,7 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
     const int64_t nchunks = (nf + cmax - 1) / cmax;
     const int64_t chunk = (nf + nchunks - 1) / nchunks;
     if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
-    const int batch = 8;   // whole frames per producer wave
-    int64_t fpw = (chunk + p->max_wg - 1) / p->max_wg;
-    fpw = ((fpw + batch - 1) / batch) * batch;
+    const int64_t fpw = frames_per_wg(p, chunk, p->max_wg);
     const int n_wg = (int)((chunk + fpw - 1) / fpw);
     for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
         const int64_t cn = std::min(chunk, nf - c0);
@@ -1337,8 +1347,7 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
             HIP_TRY(launch_irfft_quantise(a, (const float2 *)p->d_cb.p, cn, d_raw_out + c0 * bpf_o,
                                           p->desc.output_lsb != 0, s));
     }
-    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, d_acc,
-                          (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, base.flags, d_acc, s));
     return FXC_OK;
 }
 
@@ -1361,9 +1370,7 @@ static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf
     const int64_t span = chain_span(nf, chunk, 2 * (size_t)ld * 8, (int)half);
     if (!prec) GROW(p, p->d_chain, (size_t)span * 2 * ld * 8, s, "phased rotation chains");
     if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
-    int64_t fpw = (chunk + p->max_wg - 1) / p->max_wg;
-    fpw = ((fpw + kFrameBatch - 1) / kFrameBatch) * kFrameBatch;
-    if (fpw < kFrameBatch) fpw = kFrameBatch;
+    const int64_t fpw = frames_per_wg(p, chunk, p->max_wg);
     const int n_wg = (int)((chunk + fpw - 1) / fpw);
     int64_t span0 = -1;    // first frame (of this sector) of the computed chains
     for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
@@ -1395,8 +1402,7 @@ static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf
                                           p->desc.output_lsb != 0, s));
         }
     }
-    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, d_acc,
-                          (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, base.flags, d_acc, s));
     return FXC_OK;
 }
 
@@ -1464,8 +1470,7 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
                                          d_raw_out + c0 * bpf_o, s));
         }
     }
-    HIP_TRY(launch_reduce((const double *)p->part.p, kLargeGroups, p->half, d_acc,
-                          (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce((const double *)p->part.p, kLargeGroups, p->half, base.flags, d_acc, s));
     return FXC_OK;
 }
 
@@ -1567,8 +1572,8 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
             HIP_TRY(launch_irfft_cols_quantise(a, (const float2 *)p->d_cb.p, cn, d_raw_out + c0 * bpf_o,
                                                p->desc.output_lsb != 0, (const float2 *)p->tw_lm.p, s));
     }
-    HIP_TRY(launch_reduce_pairs((const double *)p->part.p, ng, p->half, p->M1, p->M2, d_acc,
-                                (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce_pairs((const double *)p->part.p, ng, p->half, p->M1, p->M2, base.flags,
+                                    d_acc, s));
     return FXC_OK;
 }
 
@@ -1603,8 +1608,8 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
             HIP_TRY(launch_large_pass2_mac(a, (const float2 *)p->d_z[0].p, (const float2 *)p->d_z[1].p,
                                            params, p->M1, p->M2, twl2, ng, c0 > 0 ? 1 : 0, s));
         }
-        HIP_TRY(launch_reduce_pairs((const double *)p->part.p, ng, p->half, p->M1, p->M2, d_acc,
-                                    (double *)p->red_scratch.p, 64, s));
+        HIP_TRY(launch_reduce_pairs((const double *)p->part.p, ng, p->half, p->M1, p->M2, base.flags,
+                                    d_acc, s));
         return FXC_OK;
     }
     const bool chain = xcf_uses_chain(p);
@@ -1650,8 +1655,7 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                  (const float2 *)p->d_z[1].p, params, kLargeGroups, c0 > 0 ? 1 : 0,
                                  s));
     }
-    HIP_TRY(launch_reduce((const double *)p->part.p, kLargeGroups, p->half, d_acc,
-                          (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce((const double *)p->part.p, kLargeGroups, p->half, base.flags, d_acc, s));
     return FXC_OK;
 }
 
@@ -1693,10 +1697,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         slab = std::min<int64_t>(nf, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / ((size_t)ld * 8))));
         GROW(p, p->d_chain, (size_t)slab * ld * 8, s, "phase chains");
     }
-    int64_t fpw = (slab + wg_cap - 1) / wg_cap;
-    const int batch = p->fft_form == 1 ? 8 : kFrameBatch;   // MFMA form: whole frames per wave
-    fpw = ((fpw + batch - 1) / batch) * batch;
-    if (fpw < batch) fpw = batch;
+    const int64_t fpw = frames_per_wg(p, slab, wg_cap);
     const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;
     a.part = (double *)p->part.p;
@@ -1735,8 +1736,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         HIP_TRY(hipEventRecord(ev.second, s));
         p->pending.push_back(ev);
     }
-    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, d_acc,
-                          (double *)p->red_scratch.p, 64, s));
+    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, a.flags, d_acc, s));
     return FXC_OK;
 }
 
@@ -1904,7 +1904,7 @@ extern "C" fxc_status fxc_sector_run_device(fxc_plan *p, const uint8_t *d_raw1,
 
 // The sector path of fxc_sector_run_device with every scratch buffer in
 // caller-given device memory (fxc_noalloc.hip passes its static array):
-// [geometric table | reduction chunk sums | workgroup partial slots].  Only
+// [geometric table | workgroup partial slots].  Only
 // the paths whose whole scratch is the partial slots run here: ACF/XCF plans
 // of the fused kernels without the plain form's phase-chain table.  The
 // grid is the plan's, capped by the slots that fit.  Allocates nothing and
@@ -1954,18 +1954,16 @@ extern "C" fxc_status fxc_internal_sector_noalloc(fxc_plan *p, const uint8_t *d_
         HIP_TRY(launch_fill_zero(d_acc, acc_bytes, s));
         return FXC_OK;
     }
-    const int kReduceChunks = 64;
     const size_t slot = acc_bytes;
     // per workgroup: its partial slot and, for the fused N = 1024 / 2048
     // form, its consumers' FP64 totals
     const size_t per_wg = slot + (p->fft_form == 1 ? kMfConsumerAccBytes : 0);
-    const size_t head = table_bytes + (size_t)kReduceChunks * slot + 256;   // + alignment of the totals
+    const size_t head = table_bytes + 256;   // + alignment of the totals
     const int64_t slots = scratch_bytes > head ? (int64_t)((scratch_bytes - head) / per_wg) : 0;
     if (slots < 1)
         return fail(FXC_ERR_UNSUPPORTED, "fft_len %d: %zu-byte partial slots do not fit the %zu-byte scratch",
                     p->N, slot, scratch_bytes);
-    double *red = (double *)(scratch + table_bytes);
-    double *part = red + (size_t)kReduceChunks * kNumProducts * p->half;
+    double *part = (double *)(scratch + table_bytes);
     const uintptr_t cacc_at = ((uintptr_t)(part + (size_t)slots * kNumProducts * p->half) + 255) & ~(uintptr_t)255;
     double *cacc = (double *)cacc_at;
     SectorArgs a;
@@ -1977,16 +1975,13 @@ extern "C" fxc_status fxc_internal_sector_noalloc(fxc_plan *p, const uint8_t *d_
     a.first_frame = first_frame;
     a.nf = nf;
     const int64_t wg_cap = std::min<int64_t>(std::max(1, p->max_wg / p->grid_div), slots);
-    int64_t fpw = (nf + wg_cap - 1) / wg_cap;
-    const int batch = p->fft_form == 1 ? 8 : kFrameBatch;
-    fpw = ((fpw + batch - 1) / batch) * batch;
-    if (fpw < batch) fpw = batch;
+    const int64_t fpw = frames_per_wg(p, nf, wg_cap);
     const int n_wg = (int)((nf + fpw - 1) / fpw);
     a.frames_per_wg = fpw;
     a.part = part;
     if (p->fft_form == 1) HIP_TRY(launch_sector_mfma(a, p->desc.precision, n_wg, s));
     else HIP_TRY(launch_sector(a, p->desc.precision, n_wg, s));
-    HIP_TRY(launch_reduce(part, n_wg, p->half, d_acc, red, kReduceChunks, s));
+    HIP_TRY(launch_reduce(part, n_wg, p->half, a.flags, d_acc, s));
     return FXC_OK;
 }
 

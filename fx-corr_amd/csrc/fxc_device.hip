@@ -194,7 +194,6 @@ __attribute__((amdgpu_waves_per_eu(MF && E == 8 && T == 256 ? 4 : 1))) void k_se
         const int g = tid + NT * i;
         if (g <= M) {
             const bool add = a.accumulate != 0;
-            out[P_PH * half + g] = 0.0;
             out[P_11 * half + g] = add ? out[P_11 * half + g] + acc[0][i] : acc[0][i];
             out[P_22 * half + g] = add ? out[P_22 * half + g] + acc[1][i] : acc[1][i];
             out[P_12R * half + g] = add ? out[P_12R * half + g] + acc[2][i] : acc[2][i];
@@ -204,72 +203,84 @@ __attribute__((amdgpu_waves_per_eu(MF && E == 8 && T == 256 ? 4 : 1))) void k_se
 }
 
 // ---------------------------------------------------- deterministic reduce
-__global__ void k_reduce_chunks(const double *part, int n_wg, int cols, int chunk,
-                                double *scratch) {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    const int c = blockIdx.y;
-    if (col >= cols) return;
-    const int w_begin = c * chunk;
-    int w_end = w_begin + chunk;
-    if (w_end > n_wg) w_end = n_wg;
-    double s = 0.0;
-    for (int w = w_begin; w < w_end; ++w) s += part[(size_t)w * cols + col];
-    scratch[(size_t)c * cols + col] = s;
-}
-
-__global__ void k_reduce_final(const double *scratch, int n_chunks, int cols, double *out) {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= cols) return;
-    double s = 0.0;
-    for (int c = 0; c < n_chunks; ++c) s += scratch[(size_t)c * cols + col];
-    out[col] = s;
-}
-
-hipError_t launch_reduce(const double *part, int n_wg, int half, double *out, double *scratch,
-                         int n_chunks, hipStream_t stream) {
+// Sums the workgroups' partial slots [n_wg][5][half] into out[5][half].  Only
+// the slot columns [c0, c1) are read (the plan's products); the others are
+// written as zeros.  A workgroup takes 16 adjacent columns (one 128-byte line
+// per slot): row y of its threads adds the slots y, y + R, y + 2R, ... (R =
+// blockDim / 16 rows), then the R row sums are added in LDS, both in a fixed
+// order, so the result does not depend on timing.  PAIRS: the slots hold the
+// fused four-step's pair-major order (index p 2 M2 + j: row p for j < M2, row
+// M1 - p, or M1 / 2 for p = 0, otherwise; k2 = j mod M2; bin M last), written
+// to the bins g = row + M1 k2.
+//
+// Latency-bound: every slot line is read once, and one launch with R = 64
+// rows keeps 64 x 8 loads in flight per line.  The two launches it replaces
+// (up to 64 slot groups, then 64 sums per column by one thread each) took 21
+// us behind the fused kernels at N = 256 / 1024 (the second one's 64 dependent
+// loads 16 us of it).
+constexpr int kRedCols = 16;
+template <bool PAIRS>
+__global__ __launch_bounds__(1024) void k_reduce_slots(const double *part, int n_wg, int half, int c0,
+                                                       int c1, int M1, int M2, double *out) {
+    __shared__ double rows[64][kRedCols];
+    const int x = threadIdx.x & (kRedCols - 1), y = threadIdx.x / kRedCols;
+    const int R = blockDim.x / kRedCols;
     const int cols = kNumProducts * half;
-    if (n_chunks < 1) n_chunks = 1;
-    if (n_chunks > n_wg) n_chunks = n_wg;
-    const int chunk = (n_wg + n_chunks - 1) / n_chunks;
-    n_chunks = (n_wg + chunk - 1) / chunk;
-    dim3 g1((cols + 255) / 256, n_chunks);
-    hipLaunchKernelGGL(k_reduce_chunks, g1, dim3(256), 0, stream, part, n_wg, cols, chunk, scratch);
-    hipLaunchKernelGGL(k_reduce_final, dim3((cols + 255) / 256), dim3(256), 0, stream, scratch,
-                       n_chunks, cols, out);
+    const int col = blockIdx.x * kRedCols + x;
+    double s = 0.0;
+    if (col >= c0 && col < c1) {
+        const double *p = part + col;
+#pragma unroll 8
+        for (int w = y; w < n_wg; w += R) s += p[(size_t)w * cols];
+    }
+    rows[y][x] = s;
+    __syncthreads();
+    const int R2 = R < 8 ? R : 8;
+    if (y < R2) {
+        for (int r = y + R2; r < R; r += R2) s += rows[r][x];
+        rows[y][x] = s;
+    }
+    __syncthreads();
+    if (y > 0 || col >= cols) return;
+    for (int r = 1; r < R2; ++r) s += rows[r][x];
+    int g = col;
+    if constexpr (PAIRS) {
+        const int prod = col / half, idx = col - prod * half;
+        if (idx < half - 1) {
+            const int p = idx / (2 * M2), j = idx - p * 2 * M2;
+            const int row = j < M2 ? p : (p == 0 ? M1 / 2 : M1 - p);
+            g = prod * half + row + M1 * (j % M2);
+        }
+    }
+    out[g] = s;
+}
+
+// flags: the plan's products (FLAG_*), i.e. which slot columns were written.
+static void reduce_shape(int n_wg, int half, int flags, int &c0, int &c1, dim3 &grid, dim3 &block) {
+    const bool phased = (flags & (FLAG_PHASED | FLAG_RAW_OUT)) != 0;
+    c0 = phased ? P_PH * half : P_11 * half;
+    c1 = phased ? P_11 * half : kNumProducts * half;
+    int rows = 4;   // a whole wave
+    while (rows < 64 && rows < n_wg) rows *= 2;
+    grid = dim3((kNumProducts * half + kRedCols - 1) / kRedCols);
+    block = dim3(rows * kRedCols);
+}
+
+hipError_t launch_reduce(const double *part, int n_wg, int half, int flags, double *out,
+                         hipStream_t stream) {
+    int c0, c1;
+    dim3 grid, block;
+    reduce_shape(n_wg, half, flags, c0, c1, grid, block);
+    hipLaunchKernelGGL(k_reduce_slots<false>, grid, block, 0, stream, part, n_wg, half, c0, c1, 0, 0, out);
     return hipGetLastError();
 }
 
-// The same reduce over partial slots held in the fused four-step's
-// pair-major order (index p 2 M2 + j: row p for j < M2, row M1 - p, or
-// M1 / 2 for p = 0, otherwise; k2 = j mod M2; bin M last), written to the
-// bins g = row + M1 k2.
-__global__ void k_reduce_final_pairs(const double *scratch, int n_chunks, int half, int M1,
-                                     int M2, double *out) {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= kNumProducts * half) return;
-    double s = 0.0;
-    for (int c = 0; c < n_chunks; ++c) s += scratch[(size_t)c * kNumProducts * half + col];
-    const int prod = col / half, idx = col - prod * half;
-    int g = idx;
-    if (idx < half - 1) {
-        const int p = idx / (2 * M2), j = idx - p * 2 * M2;
-        const int row = j < M2 ? p : (p == 0 ? M1 / 2 : M1 - p);
-        g = row + M1 * (j % M2);
-    }
-    out[(size_t)prod * half + g] = s;
-}
-
-hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, int M2, double *out,
-                               double *scratch, int n_chunks, hipStream_t stream) {
-    const int cols = kNumProducts * half;
-    if (n_chunks < 1) n_chunks = 1;
-    if (n_chunks > n_wg) n_chunks = n_wg;
-    const int chunk = (n_wg + n_chunks - 1) / n_chunks;
-    n_chunks = (n_wg + chunk - 1) / chunk;
-    dim3 g1((cols + 255) / 256, n_chunks);
-    hipLaunchKernelGGL(k_reduce_chunks, g1, dim3(256), 0, stream, part, n_wg, cols, chunk, scratch);
-    hipLaunchKernelGGL(k_reduce_final_pairs, dim3((cols + 255) / 256), dim3(256), 0, stream, scratch,
-                       n_chunks, half, M1, M2, out);
+hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, int M2, int flags,
+                               double *out, hipStream_t stream) {
+    int c0, c1;
+    dim3 grid, block;
+    reduce_shape(n_wg, half, flags, c0, c1, grid, block);
+    hipLaunchKernelGGL(k_reduce_slots<true>, grid, block, 0, stream, part, n_wg, half, c0, c1, M1, M2, out);
     return hipGetLastError();
 }
 

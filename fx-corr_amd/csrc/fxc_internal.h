@@ -127,8 +127,8 @@ constexpr int MFT4_BYTES = MFT4_SLUT + 2 * 4 * 256 * 4;
 // Launchers implemented in fxc_device.hip.  All enqueue on `stream`.
 hipError_t launch_sector(const SectorArgs &a, int precision, int n_wg,
                          hipStream_t stream);
-hipError_t launch_reduce(const double *part, int n_wg, int half, double *out,
-                         double *scratch, int n_chunks, hipStream_t stream);
+hipError_t launch_reduce(const double *part, int n_wg, int half, int flags, double *out,
+                         hipStream_t stream);
 int sector_threads_per_frame(int N);
 bool sector_supported(int N);
 bool sector_has_variant(int N);
@@ -216,8 +216,8 @@ hipError_t launch_rfft_mfma(const SectorArgs &a, const float *in, int64_t nframe
 hipError_t launch_large_pass1_fused(const SectorArgs &a, const int64_t *shifts, float2 *out0,
                                     float2 *out1, int M1, int M2, const float2 *tw_m,
                                     hipStream_t s);
-hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, int M2, double *out,
-                               double *scratch, int n_chunks, hipStream_t stream);
+hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, int M2, int flags,
+                               double *out, hipStream_t stream);
 hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                   const FrameParam *params, int M1, int M2, const float2 *tw_m2,
                                   int n_groups, int accumulate, hipStream_t s);

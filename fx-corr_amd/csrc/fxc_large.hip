@@ -255,7 +255,6 @@ __global__ __launch_bounds__(256) void k_mac_large(SectorArgs a, const float2 *z
                             accumulate ? out[P_22 * half + g] : 0.0,
                             accumulate ? out[P_12R * half + g] : 0.0,
                             accumulate ? out[P_12I * half + g] : 0.0};
-    out[P_PH * half + g] = 0.0;
     out[P_11 * half + g] = prev[0] + acc[0];
     out[P_22 * half + g] = prev[1] + acc[1];
     out[P_12R * half + g] = prev[2] + acc[2];
@@ -459,7 +458,6 @@ __global__ __launch_bounds__(256) void k_large_pass2_mac(SectorArgs a, const flo
                                 accumulate ? out[P_22 * half + g] : 0.0,
                                 accumulate ? out[P_12R * half + g] : 0.0,
                                 accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_PH * half + g] = 0.0;
         out[P_11 * half + g] = prev[0] + acc[i][0];
         out[P_22 * half + g] = prev[1] + acc[i][1];
         out[P_12R * half + g] = prev[2] + acc[i][2];
@@ -618,7 +616,6 @@ __global__ __launch_bounds__(256) void k_large_pass2_r16(SectorArgs a, const flo
                                 accumulate ? out[P_22 * half + g] : 0.0,
                                 accumulate ? out[P_12R * half + g] : 0.0,
                                 accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_PH * half + g] = 0.0;
         out[P_11 * half + g] = prev[0] + acc[i][0];
         out[P_22 * half + g] = prev[1] + acc[i][1];
         out[P_12R * half + g] = prev[2] + acc[i][2];
@@ -791,7 +788,6 @@ __global__ __launch_bounds__(256) void k_large_pass2_r8(SectorArgs a, const floa
                                 accumulate ? out[P_22 * half + g] : 0.0,
                                 accumulate ? out[P_12R * half + g] : 0.0,
                                 accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_PH * half + g] = 0.0;
         out[P_11 * half + g] = prev[0] + v[0];
         out[P_22 * half + g] = prev[1] + v[1];
         out[P_12R * half + g] = prev[2] + v[2];
@@ -1016,10 +1012,6 @@ __global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorAr
             v = nacc + msum;
         }
         out[P_PH * half + g] = accumulate ? out[P_PH * half + g] + v : v;
-        out[P_11 * half + g] = 0.0;
-        out[P_22 * half + g] = 0.0;
-        out[P_12R * half + g] = 0.0;
-        out[P_12I * half + g] = 0.0;
     }
 }
 

@@ -610,7 +610,6 @@ __global__ __launch_bounds__(512) void k_sector_mf2(SectorArgs a) {
     }
     double *out = a.part + (size_t)blockIdx.x * kNumProducts * H;
     for (int k = tid; k < H; k += 512) {
-        out[P_PH * H + k] = 0.0;
         out[P_11 * H + k] = red[0 * H + k];
         out[P_22 * H + k] = red[1 * H + k];
         out[P_12R * H + k] = red[2 * H + k];
@@ -1134,7 +1133,6 @@ __global__ __launch_bounds__(mf::THREADS3) void k_sector_mf3(SectorArgs a) {
     if (sh.broken && tid == 0 && a.err)   // and the plan's error word reports it to the host
         __hip_atomic_fetch_or(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int k = tid; k < H; k += NT) {
-        out[P_PH * H + k] = bad;
         out[P_11 * H + k] = red[0 * H + k] + bad;
         out[P_22 * H + k] = red[1 * H + k] + bad;
         out[P_12R * H + k] = red[2 * H + k] + bad;
@@ -1526,7 +1524,6 @@ __global__ __launch_bounds__(mf::THREADS3) void k_sector_mfs(SectorArgs a) {
     if (sh.broken && tid == 0 && a.err)
         __hip_atomic_fetch_or(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int k = tid; k < H; k += NT) {
-        out[P_PH * H + k] = bad;
         out[P_11 * H + k] = red[0 * H + k] + bad;
         out[P_22 * H + k] = red[1 * H + k] + bad;
         out[P_12R * H + k] = red[2 * H + k] + bad;
@@ -1808,15 +1805,8 @@ __global__ __launch_bounds__(mf::THREADS3) void k_phased_mf3(SectorArgs a, int a
     const double bad = sh.broken ? __builtin_nan("") : 0.0;   // NaN marks a failed hand-over
     if (sh.broken && tid == 0 && a.err)
         __hip_atomic_fetch_or(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int k = tid; k < H; k += NT) {
+    for (int k = tid; k < H; k += NT)
         out[P_PH * H + k] = (accumulate ? out[P_PH * H + k] : 0.0) + red[k] + bad;
-        if (!accumulate) {   // the other products stay zero over the later chunks
-            out[P_11 * H + k] = 0.0;
-            out[P_22 * H + k] = 0.0;
-            out[P_12R * H + k] = 0.0;
-            out[P_12I * H + k] = 0.0;
-        }
-    }
 }
 
 hipError_t launch_phased_mf3(const SectorArgs &a, int accumulate, int n_wg, hipStream_t s) {
@@ -2220,7 +2210,6 @@ __global__ __launch_bounds__(mf4::THREADS) void k_sector_mf4(SectorArgs a) {
     if (sh.broken && tid == 0 && a.err)   // and the plan's error word reports it to the host
         __hip_atomic_fetch_or(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int k = tid; k < H; k += NT) {
-        out[P_PH * H + k] = bad;
         out[P_11 * H + k] = red[0 * H + k] + bad;
         out[P_22 * H + k] = red[1 * H + k] + bad;
         out[P_12R * H + k] = red[2 * H + k] + bad;

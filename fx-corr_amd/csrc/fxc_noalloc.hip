@@ -3,8 +3,8 @@
 // For callers that cannot allocate device memory (code under HIP graph
 // capture, tight serving loops, harnesses that forbid hipMalloc): the
 // sector path of fxc_sector_run_device with its scratch -- the geometric
-// table, the workgroup partial slots and the reduction's chunk sums -- in a
-// file-scope device array instead of plan-owned buffers.  The kernels are
+// table and the workgroup partial slots -- in a file-scope device array
+// instead of plan-owned buffers.  The kernels are
 // the same; the array is reached through the address hipGetSymbolAddress
 // returns for the current device (the host-side name of a __device__ array
 // is only a stand-in, not a device address).

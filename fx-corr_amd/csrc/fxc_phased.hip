@@ -182,15 +182,7 @@ __global__ __launch_bounds__(2 * T) void k_phased(SectorArgs a, int accumulate) 
     for (int i = 0; i < NB; ++i) {
         const int g = tid + NT * i;
         if (g <= M) {
-            if (accumulate) {
-                out[P_PH * half + g] += ph[i];
-            } else {   // the other products stay zero over the later chunks
-                out[P_PH * half + g] = ph[i];
-                out[P_11 * half + g] = 0.0;
-                out[P_22 * half + g] = 0.0;
-                out[P_12R * half + g] = 0.0;
-                out[P_12I * half + g] = 0.0;
-            }
+            out[P_PH * half + g] = accumulate ? out[P_PH * half + g] + ph[i] : ph[i];
         }
     }
 }
@@ -303,10 +295,6 @@ __global__ __launch_bounds__(256) void k_phased_large(SectorArgs a, const float2
     }
     double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
     out[P_PH * half + g] = accumulate ? out[P_PH * half + g] + ph : ph;
-    out[P_11 * half + g] = 0.0;
-    out[P_22 * half + g] = 0.0;
-    out[P_12R * half + g] = 0.0;
-    out[P_12I * half + g] = 0.0;
 }
 
 size_t phased_param_bytes() { return sizeof(PhasedParam); }
