@@ -147,11 +147,12 @@ struct fxc_plan {
     StationDev st[2];
     int32_t decode_ok[2] = {1, 1};
     // device tables
-    DevBuf tw_fft, tw_post, lev_dev[2], out_lev, mf_tab;
+    DevBuf tw_fft, tw_post, lev_dev[2], out_lev, mf_tab, wk_tab;
     int fft_form = 0;  // 0: FP32 Stockham, 1: FP16/FP32-MFMA four-step (N = 256..2048),
                        // 2: four-step through HBM scratch (N = 32768, 65536)
     bool mf_b1 = false;   // fft_form 0 / 2: mf_tab holds the DFT-32 operand table (scale 1)
                           // and the FFT's first pass runs on FP16 MFMA
+    bool wave = false;    // fft_form 0: variant 0 is the wave kernel (wk_tab holds its tables)
     // large-N scratch (fft_form 2): chunk of `chunk` frames
     int M1 = 0, M2 = 0;
     int64_t chunk = 0;       // allocated chunk (frames)
@@ -167,6 +168,7 @@ struct fxc_plan {
     DevBuf part, table_dev, d_raw[2], d_acc, d_raw_out, d_tmp_in, d_tmp_out,
         d_shifts, d_cb, d_tbuf;
     DevBuf d_chain;          // the reference's f32 phase chains of one slab/chunk of frames
+    DevBuf d_wparams;        // wave kernel: one slab's per-frame parameters
     DevBuf d_fringe;         // one chunk's products for the whole-scan cross spectrum
     DevBuf d_err;            // device error word: bit 0 set by a workgroup whose hand-over wait ran out
     DevBuf d_cacc;           // fused N = 1024 form: per-consumer FP64 totals (kMfConsumerAccBytes per workgroup)
@@ -186,11 +188,11 @@ struct fxc_plan {
 
     // Every device buffer of the plan (release, byte count).
     template <class Fn> void each_buf(Fn fn) {
-        DevBuf *bufs[] = {&tw_fft, &tw_post, &lev_dev[0], &lev_dev[1], &out_lev, &mf_tab,
+        DevBuf *bufs[] = {&tw_fft, &tw_post, &lev_dev[0], &lev_dev[1], &out_lev, &mf_tab, &wk_tab,
                           &tw_l1, &tw_l2, &tw_lm, &tw_l0, &d_x[0], &d_x[1], &d_y, &d_z[0], &d_z[1],
                           &d_params, &d_lshifts, &part, &table_dev, &d_raw[0],
                           &d_raw[1], &d_acc, &d_raw_out, &d_tmp_in, &d_tmp_out, &d_shifts,
-                          &d_cb, &d_tbuf, &d_chain, &d_fringe, &d_err, &d_cacc};
+                          &d_cb, &d_tbuf, &d_chain, &d_wparams, &d_fringe, &d_err, &d_cacc};
         for (DevBuf *b : bufs) fn(*b);
     }
 };
@@ -533,6 +535,7 @@ static void fill_args(fxc_plan *p, SectorArgs &a) {
     // fused MFMA kernels: their table layout; Stockham / HBM four-step: the
     // DFT-32 operand table when the first pass runs on MFMA, else none
     a.mf_tab = (p->fft_form == 1 || p->mf_b1) ? p->mf_tab.p : nullptr;
+    a.wk_tab = p->wave ? p->wk_tab.p : nullptr;
     a.variant = p->variant;
     a.err = (int32_t *)p->d_err.p;
     a.cons_acc = (double *)p->d_cacc.p;
@@ -758,6 +761,98 @@ static std::vector<uint8_t> mfma_tables(const fxc_plan *p) {
     return tab;
 }
 
+// Two resident workgroups per CU (fxc_wave.hip).
+static int wave_wg_cap() { return 2 * num_cus(); }
+
+// The wave kernel (fxc_wave.hip) replaces the Stockham sector kernel where the
+// samples can be staged as FP16 without rounding and by whole words: ACF/XCF
+// plans at N = 256..8192 with 1/2/4/8-bit codes and levels exact in FP16 (its
+// figures against k_sector are at the kernel).
+// Other widths and levels, and N = 64 / 128, keep k_sector.
+static bool wave_eligible(const fxc_plan *p) {
+    if (p->fft_form != 0 || p->N < 256 || p->N > 8192) return false;
+    if (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) return false;
+    for (int i = 0; i < 2; ++i) {
+        const int b = p->desc.st[i].bits;
+        if (b != 1 && b != 2 && b != 4 && b != 8) return false;
+    }
+    return levels_fp16_exact(p);
+}
+
+// Whether a sector of nf frames runs on the wave kernel (variant 0 of a plan
+// that has one).  Short sectors stay on the Stockham kernel, whose workgroups
+// take one frame pair at a time: they finish sooner while the chip is not
+// full (microseconds a sector, Stockham / wave: chosen N = 4096, 64 frames 19
+// / 25, 512 frames 36 / 40, 4096 frames 105 / 90; chosen 8192, 512 frames 54 /
+// 71, 2048 frames 133 / 133; plain 1024, 256 frames 19 / 20, 2048 frames 39 /
+// 24).  Four frames per CU from N = 4096 on, one below.
+static bool wave_for(const fxc_plan *p, int64_t nf) {
+    return p->wave && p->variant == 0 && nf > (int64_t)num_cus() * (p->N <= 2048 ? 1 : 4);
+}
+
+// The wave kernel's tables (WkTables): twf holds W_M^k.
+static std::vector<uint8_t> wave_tables(const fxc_plan *p, const std::vector<float> &twf) {
+    const int M = p->M, M2 = M / 32;
+    std::vector<uint8_t> tab(wk_bytes(M), 0);
+    float *tw = (float *)tab.data();
+    for (int k1 = 0; k1 < 32; ++k1)
+        for (int m2 = 0; m2 < M2; ++m2) {
+            const int k = (m2 * k1) % M, at = p->mf_b1 ? m2 * 32 + k1 : k1 * M2 + m2;
+            tw[2 * at] = twf[2 * k];
+            tw[2 * at + 1] = twf[2 * k + 1];
+        }
+    // W_M2^i rounded to the neighbouring floats whose magnitude is closest to
+    // 1: a pass reuses a few of these for every column, so their common
+    // shortening would not average out of the summed powers
+    float *w2 = tw + 2 * M;
+    for (int i = 0; i < M2; ++i) {
+        const double c = std::cos(2.0 * M_PI * i / M2), s = -std::sin(2.0 * M_PI * i / M2);
+        const float c0 = (float)c, s0 = (float)s;
+        double best = 1e300;
+        for (int u = -1; u <= 1; ++u)
+            for (int v = -1; v <= 1; ++v) {
+                const float cf = u == 0 ? c0 : std::nextafterf(c0, u * INFINITY);
+                const float sf = v == 0 ? s0 : std::nextafterf(s0, v * INFINITY);
+                const double mag = std::hypot((double)cf, (double)sf) - 1.0;
+                const double ang = c * (sf - s) - s * (cf - c);
+                const double e = 4.0 * mag * mag + ang * ang;
+                if (e < best) {
+                    best = e;
+                    w2[2 * i] = cf;
+                    w2[2 * i + 1] = sf;
+                }
+            }
+    }
+    for (int st = 0; st < 2; ++st) {
+        uint32_t *slut = (uint32_t *)(tab.data() + wk_slut_at(M)) + st * 4 * 256;
+        uint16_t *dlut = (uint16_t *)(tab.data() + wk_dlut_at(M)) + st * kWkDlutHalves;
+        const fxc_station_desc &d = p->desc.st[st];
+        const int bits = d.bits;
+        const uint32_t mask = (1u << bits) - 1u;
+        auto lev = [&](uint32_t code, bool neg) {
+            const uint16_t h = f32_to_f16_bits((float)p->levels[st][code]);
+            return (uint16_t)(neg ? (h ^ 0x8000u) : h);
+        };
+        if (bits == 8) {
+            for (uint32_t v = 0; v < 256; ++v) {
+                dlut[v] = lev(v, false);
+                dlut[256 + v] = lev(v, d.lsb != 0);
+            }
+        } else {
+            const int n = bits == 1 ? 4 : 8 / bits, values = bits == 1 ? 16 : 256;   // samples per entry
+            for (int v = 0; v < values; ++v)
+                for (int i = 0; i < n; ++i)
+                    dlut[v * n + i] = lev(((uint32_t)v >> (bits * i)) & mask, d.lsb && (i & 1));
+        }
+        for (int i = 0; i < 32; ++i) {
+            const int src = d.shuffle_internal[i];
+            for (uint32_t v = 0; v < 256; ++v)
+                if ((v >> (src & 7)) & 1u) slut[(src >> 3) * 256 + v] |= 1u << i;
+        }
+    }
+    return tab;
+}
+
 static bool large_fused_possible(const fxc_plan *p);
 static bool phased_fused_possible(const fxc_plan *p);
 
@@ -916,6 +1011,13 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
             return cleanup(fail(FXC_ERR_HIP, "MFMA table upload failed"));
         p->mf_b1 = true;
     }
+    if (wave_eligible(p)) {
+        const std::vector<uint8_t> tab = wave_tables(p, twf);
+        if (p->wk_tab.ensure(tab.size()) != hipSuccess ||
+            hipMemcpy(p->wk_tab.p, tab.data(), tab.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(fail(FXC_ERR_HIP, "wave kernel table upload failed"));
+        p->wave = true;
+    }
     // grid: plain form about 16 waves per CU worth of workgroups (p->T
     // threads each); MFMA form one 8-wave workgroup per CU; large-N form one
     // partial per frame group.  Each workgroup runs a contiguous range of
@@ -954,8 +1056,9 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
     p->max_wg = p->fft_form == 1 ? cus
                 : p->fft_form == 2 ? kLargeGroups
                                    : std::max(64, (cus * 1024) / p->T);
+    const int slots = p->wave ? std::max(p->max_wg, wave_wg_cap()) : p->max_wg;
     if ((p->fft_form == 1 && p->d_cacc.ensure((size_t)p->max_wg * kMfConsumerAccBytes) != hipSuccess) ||
-        p->part.ensure((size_t)p->max_wg * kNumProducts * half * sizeof(double)) != hipSuccess ||
+        p->part.ensure((size_t)slots * kNumProducts * half * sizeof(double)) != hipSuccess ||
         p->d_err.ensure(sizeof(int32_t)) != hipSuccess)
         return cleanup(fail(FXC_ERR_NOMEM, "scratch allocation failed"));
     if (hipMemset(p->d_err.p, 0, sizeof(int32_t)) != hipSuccess)
@@ -1281,16 +1384,19 @@ static bool xcf_uses_chain(const fxc_plan *p) {
 }
 constexpr size_t kChainSlabBytes = (size_t)256 << 20;   // chain scratch of the fused plain path
 
+// Frames of one wave-kernel launch: its parameter table stays below 32 MB.
+constexpr int64_t kWaveSlab = (int64_t)1 << 19;
+
 // Frames per workgroup of the fused kernels for a launch of nf frames on at
 // most wg_cap workgroups.  Stockham kernels (one frame pair at a time per
 // workgroup): as few as the cap allows, so that a short launch spreads over
 // the chip; a frame pair alone takes about 8 us of latency at N = 1024, and a
 // 150-frame sector on 19 workgroups of 8 frames took 64 us where 150
 // workgroups take 20.  MFMA kernels: whole frames per producer wave, eight a
-// workgroup, which run side by side.
-static int64_t frames_per_wg(const fxc_plan *p, int64_t nf, int64_t wg_cap) {
+// workgroup, which run side by side; wave kernel: whole rounds.
+static int64_t frames_per_wg(const fxc_plan *p, int64_t nf, int64_t wg_cap, bool wave = false) {
     const int64_t fpw = std::max<int64_t>(1, (nf + wg_cap - 1) / wg_cap);
-    const int64_t batch = p->fft_form == 1 ? 8 : 1;
+    const int64_t batch = p->fft_form == 1 ? 8 : wave ? wave_frames(p->N) : 1;
     return (fpw + batch - 1) / batch * batch;
 }
 
@@ -1686,18 +1792,20 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     if (phased && phased_fused_ok(p)) return enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
     if (p->fft_form == 2 || large_fused_ok(p)) return enqueue_large(p, a, nf, d_acc, s);
-    const int wg_cap = std::max(1, p->max_wg / p->grid_div);
+    const bool wave = wave_for(p, nf);
+    const int wg_cap = std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div);
     // Plain XCF over more than kChainMinOverlap bins: slabs of frames whose
     // f32 phase chains fit the chain scratch; the slabs add into the same
     // workgroup slots in order.
     const bool chain = p->fft_form == 0 && xcf_uses_chain(p);
     const int ld = chain ? chain_ld_for(a.ov) : 0;
-    int64_t slab = nf;
+    int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
     if (chain) {
-        slab = std::min<int64_t>(nf, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / ((size_t)ld * 8))));
+        slab = std::min<int64_t>(slab, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / ((size_t)ld * 8))));
         GROW(p, p->d_chain, (size_t)slab * ld * 8, s, "phase chains");
     }
-    const int64_t fpw = frames_per_wg(p, slab, wg_cap);
+    if (wave) GROW(p, p->d_wparams, (size_t)slab * sizeof(WkParam), s, "frame parameters");
+    const int64_t fpw = frames_per_wg(p, slab, wg_cap, wave);
     const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;
     a.part = (double *)p->part.p;
@@ -1723,13 +1831,18 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         b.first_frame = a.first_frame + c0;
         b.nf = cn;
         const int wgs = (int)((cn + fpw - 1) / fpw);
+        b.accumulate = c0 > 0 ? 1 : 0;
+        if (wave) {
+            HIP_TRY(launch_wave_params(b, p->desc.precision, (WkParam *)p->d_wparams.p, s));
+            b.wk_params = p->d_wparams.p;
+        }
         if (chain) {
             b.chain = (const float2 *)p->d_chain.p;
             b.chain_ld = ld;
-            b.accumulate = c0 > 0 ? 1 : 0;
             HIP_TRY(launch_phase_chain(b, CHAIN_XCF, (float2 *)p->d_chain.p, s));
         }
         if (p->fft_form == 1) HIP_TRY(launch_sector_mfma(b, p->desc.precision, wgs, s));
+        else if (wave) HIP_TRY(launch_sector_wave(b, p->desc.precision, wgs, s));
         else HIP_TRY(launch_sector(b, p->desc.precision, wgs, s));
     }
     if (p->timing) {
@@ -1958,12 +2071,16 @@ extern "C" fxc_status fxc_internal_sector_noalloc(fxc_plan *p, const uint8_t *d_
     // per workgroup: its partial slot and, for the fused N = 1024 / 2048
     // form, its consumers' FP64 totals
     const size_t per_wg = slot + (p->fft_form == 1 ? kMfConsumerAccBytes : 0);
-    const size_t head = table_bytes + 256;   // + alignment of the totals
+    // wave kernel: one slab's frame parameters
+    const bool wave = wave_for(p, nf);
+    const int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
+    const size_t par = wave ? ((size_t)slab * sizeof(WkParam) + 255) & ~(size_t)255 : 0;
+    const size_t head = table_bytes + par + 256;   // + alignment of the totals
     const int64_t slots = scratch_bytes > head ? (int64_t)((scratch_bytes - head) / per_wg) : 0;
     if (slots < 1)
         return fail(FXC_ERR_UNSUPPORTED, "fft_len %d: %zu-byte partial slots do not fit the %zu-byte scratch",
                     p->N, slot, scratch_bytes);
-    double *part = (double *)(scratch + table_bytes);
+    double *part = (double *)(scratch + table_bytes + par);
     const uintptr_t cacc_at = ((uintptr_t)(part + (size_t)slots * kNumProducts * p->half) + 255) & ~(uintptr_t)255;
     double *cacc = (double *)cacc_at;
     SectorArgs a;
@@ -1974,13 +2091,25 @@ extern "C" fxc_status fxc_internal_sector_noalloc(fxc_plan *p, const uint8_t *d_
     a.raw2 = d_raw2;
     a.first_frame = first_frame;
     a.nf = nf;
-    const int64_t wg_cap = std::min<int64_t>(std::max(1, p->max_wg / p->grid_div), slots);
-    const int64_t fpw = frames_per_wg(p, nf, wg_cap);
-    const int n_wg = (int)((nf + fpw - 1) / fpw);
+    const int64_t wg_cap =
+        std::min<int64_t>(std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div), slots);
+    const int64_t fpw = frames_per_wg(p, slab, wg_cap, wave);
+    const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;
     a.part = part;
     if (p->fft_form == 1) HIP_TRY(launch_sector_mfma(a, p->desc.precision, n_wg, s));
-    else HIP_TRY(launch_sector(a, p->desc.precision, n_wg, s));
+    else if (!wave) HIP_TRY(launch_sector(a, p->desc.precision, n_wg, s));
+    for (int64_t c0 = 0; wave && c0 < nf; c0 += slab) {
+        SectorArgs b = a;
+        b.raw1 = a.raw1 + c0 * p->st[0].bpf;
+        b.raw2 = a.raw2 + c0 * p->st[1].bpf;
+        b.first_frame = a.first_frame + c0;
+        b.nf = std::min(slab, nf - c0);
+        b.accumulate = c0 > 0 ? 1 : 0;
+        b.wk_params = scratch + table_bytes;
+        HIP_TRY(launch_wave_params(b, p->desc.precision, (WkParam *)(scratch + table_bytes), s));
+        HIP_TRY(launch_sector_wave(b, p->desc.precision, (int)((b.nf + fpw - 1) / fpw), s));
+    }
     HIP_TRY(launch_reduce(part, n_wg, p->half, a.flags, d_acc, s));
     return FXC_OK;
 }

@@ -36,6 +36,15 @@ __device__ __forceinline__ int loop_local(int v) {
     return v;
 }
 
+// Orders this wave's LDS writes before its later LDS reads (a wave's LDS
+// operations complete in issue order; this keeps the compiler from moving
+// them across each other).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------------ delay model
 // Rust `v as i64`: truncation with saturation, NaN -> 0.
 __device__ __forceinline__ int64_t f64_to_i64_sat(double v) {
@@ -150,6 +159,29 @@ __device__ __forceinline__ double wrap_turns(double x) { return x - rint(x); }
 __device__ __forceinline__ float2 phasor_turns(double x) {
     const float r = (float)wrap_turns(x);
     return make_float2(__builtin_amdgcn_cosf(r), __builtin_amdgcn_sinf(r));
+}
+
+// (cos, sin)(2 pi r) for |r| <= 0.5 turns: quadrant reduction to
+// |t| <= 1/8 turn and Taylor polynomials through x^9 / x^8 (truncation
+// error below 3e-8 on |x| <= pi/4).
+__device__ __forceinline__ float2 sincos_turns(float r) {
+    const float q = rintf(4.0f * r);
+    const float t = r - 0.25f * q;
+    const float x = t * 6.28318530717958647692f;
+    const float x2 = x * x;
+    float s = fmaf(x2, 2.75573192e-6f, -1.98412698e-4f);
+    s = fmaf(x2, s, 8.33333333e-3f);
+    s = fmaf(x2, s, -1.66666667e-1f);
+    s = fmaf(x2 * x, s, x);
+    float c = fmaf(x2, 2.48015873e-5f, -1.38888889e-3f);
+    c = fmaf(x2, c, 4.16666667e-2f);
+    c = fmaf(x2, c, -0.5f);
+    c = fmaf(x2, c, 1.0f);
+    const int qi = ((int)q) & 3;
+    // quadrants 1..3: (-s, c), (-c, -s), (s, -c), by selects and sign bits
+    const float co = (qi & 1) ? s : c, si = (qi & 1) ? c : s;
+    return make_float2(__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, co) ^ ((uint32_t)((qi + 1) & 2) << 30)),
+                       __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, si) ^ ((uint32_t)(qi & 2) << 30)));
 }
 
 __device__ __forceinline__ float2 c_scale(float2 a, float w) { return make_float2(a.x * w, a.y * w); }

@@ -79,6 +79,8 @@ struct SectorArgs {
     int32_t bpf_out;
     uint8_t *raw_out;        // phased .raw frames (nf * bpf_out) or null
     double *part;            // [n_wg][kNumProducts][half]
+    const void *wk_tab;      // wave kernel tables (WkTables), or null
+    const void *wk_params;   // wave kernel: the launch's WkParam per frame
     const void *mf_tab;      // chosen-form MFMA tables, layout MFT_* (N = 1024) or MFT4_* (N = 2048)
     float2 *cb_out;          // phased: combined half spectra [frame][half] for the .raw output
     int32_t variant;         // FFT pass sequence of the plain kernel (autotuned; 0 default)
@@ -153,6 +155,43 @@ hipError_t launch_quantise_cplx(const SectorArgs &a, const float2 *z, int64_t nf
 hipError_t launch_quantise_frames(const SectorArgs &a, const float *in,
                                   int64_t nframes, uint8_t *out,
                                   hipStream_t stream);
+
+// fxc_wave.hip: the fused sector kernel with wave-private FFTs (N = 256..8192,
+// 1/2/4/8-bit codes with levels exact in FP16).  Its tables: the stage-1
+// twiddles W_M^{m2 k1} (rows k1, or rows m2 where stage 1 runs on MFMA), the
+// M2 = M / 32 twiddles W_M2^i, byte tables of both stations' shuffles and
+// decodes.
+constexpr int kWkDlutHalves = 1024;
+struct WkTables {
+    const float2 *tw;       // M
+    const float2 *w2;       // M / 32
+    const uint32_t *slut;   // 2 x 4 x 256
+    const uint16_t *dlut;   // 2 x kWkDlutHalves
+};
+__host__ __device__ inline size_t wk_slut_at(int M) { return (size_t)(M + M / 32) * 8; }
+__host__ __device__ inline size_t wk_dlut_at(int M) { return wk_slut_at(M) + 2 * 4 * 256 * 4; }
+__host__ __device__ inline size_t wk_bytes(int M) { return wk_dlut_at(M) + 2 * kWkDlutHalves * 2; }
+__host__ __device__ inline WkTables wk_tables(const void *tab, int M) {
+    const uint8_t *b = (const uint8_t *)tab;
+    return WkTables{(const float2 *)b, (const float2 *)b + M, (const uint32_t *)(b + wk_slut_at(M)),
+                    (const uint16_t *)(b + wk_dlut_at(M))};
+}
+inline int wave_frames(int N) { return 8192 / N; }   // frames a workgroup's round holds (N <= 8192)
+// Per-frame values: the XCF phasor of overlap index k is
+// (1 + lam0 + k lam) exp(2 pi i (phw + k dth)), the fringe phasors included
+// (chosen: lam0 = lam = 0), or frmix times the chain's link.
+struct WkParam {
+    double phw, dth;
+    float2 C;            // exp(2 pi i (2 phw + (M - 2 gs) dth)): mirror bins
+    float2 F1;           // exp(2 pi i 256 dth): a thread's next pair
+    float2 frmix;
+    float lam0, lam;
+    int16_t s1, s2;      // integer shifts clamped to [-N, N]
+    int32_t pad;
+};
+// the parameters of the launch's frames, for a.wk_params
+hipError_t launch_wave_params(const SectorArgs &a, int precision, WkParam *out, hipStream_t stream);
+hipError_t launch_sector_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t stream);
 
 hipError_t launch_sector_mfma(const SectorArgs &a, int precision, int n_wg, hipStream_t stream);
 int mfma_wg_threads();

@@ -47,15 +47,6 @@ struct MfShared {
     float2 z[mf::WAVES][2][mf::M];               // [wave][station] Z/2 in natural order
 };
 
-// Orders this wave's LDS writes before its later LDS reads (a wave's LDS
-// operations complete in issue order; this keeps the compiler from moving
-// them across each other).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ double readlane_d(double v, int lane) {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
     const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, lane);
@@ -65,31 +56,6 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
 __device__ __forceinline__ float readlane_f(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, v), lane));
 }
-
-// (cos, sin)(2 pi r) for |r| <= 0.5 turns: quadrant reduction to
-// |t| <= 1/8 turn and Taylor polynomials through x^9 / x^8 (truncation
-// error below 3e-8 on |x| <= pi/4).
-__device__ __forceinline__ float2 sincos_turns(float r) {
-    const float q = rintf(4.0f * r);
-    const float t = r - 0.25f * q;
-    const float x = t * 6.28318530717958647692f;
-    const float x2 = x * x;
-    float s = fmaf(x2, 2.75573192e-6f, -1.98412698e-4f);
-    s = fmaf(x2, s, 8.33333333e-3f);
-    s = fmaf(x2, s, -1.66666667e-1f);
-    s = fmaf(x2 * x, s, x);
-    float c = fmaf(x2, 2.48015873e-5f, -1.38888889e-3f);
-    c = fmaf(x2, c, 4.16666667e-2f);
-    c = fmaf(x2, c, -0.5f);
-    c = fmaf(x2, c, 1.0f);
-    const int qi = ((int)q) & 3;
-    float co = c, si = s;
-    if (qi == 1) { co = -s; si = c; }
-    else if (qi == 2) { co = -c; si = -s; }
-    else if (qi == 3) { co = s; si = -c; }
-    return make_float2(co, si);
-}
-
 
 // Per-frame values of the chosen form (main.rs:184-241, 133-149 restated in
 // turns): integer shifts, the fringe difference phw = w1 - w2 and the

@@ -1,0 +1,65 @@
+"""The wave kernel (N = 256..8192 off the producer/consumer kernels) against
+the oracle: every size, both stage-1 forms, code widths, shuffles and LSB
+input, shifts inside and past the staging padding and past the frame, band
+offsets on both grids, product subsets, ragged last rounds, and the frame
+counts on both sides of its line against the Stockham kernel."""
+import numpy as np
+import pytest
+
+import fxcorr as F
+import fxref as R
+from _cases import gpu_run, make_case, oracle_run, spectra_err
+
+pytestmark = pytest.mark.gpu
+LINE = {256: 256, 512: 256, 1024: 256, 2048: 256, 4096: 1024, 8192: 1024}   # frames on 256 CUs
+ACF, XCF, OV = F.PRODUCT_ACF, F.PRODUCT_XCF, F.PRODUCT_ACF_OVERLAP_ONLY
+PERM = np.random.default_rng(4).permutation(32).astype(np.int32)
+SWAP = np.arange(32, dtype=np.int32) ^ 1
+
+
+def check(c, form):
+    plain = form == "plain"
+    g = gpu_run(c, F.PRECISION_PLAIN_FP32 if plain else F.PRECISION_CHOSEN)
+    o = oracle_run(c, R.MODE_F32 if plain else R.MODE_F64)
+    errs = spectra_err(g, o)   # bars of the two forms, as everywhere in the parity tests
+    assert g["n_failed"] == 0 and all(e < (1e-5 if plain else 1e-4) for e in errs.values()), errs
+    for k in ("acc11", "acc22", "acc12"):
+        assert np.array_equal(g[k] == 0, o[k] == 0), k
+
+
+@pytest.mark.parametrize("form", ["plain", "chosen"])
+@pytest.mark.parametrize("n,extra", [(256, 0), (256, 1), (256, 70), (512, 13), (1024, 1), (1024, 260), (2048, 3),
+                                     (4096, 1), (4096, 2), (8192, 1), (8192, 0)])
+def test_wave_sizes(n, extra, form):
+    # band offset of one bin: also the chosen form leaves the producer/consumer kernels
+    c = make_case(n=n, fs=64e6, nf=LINE[n] + extra, rho=0.2, seed=n + extra, band=(1, 0, n // 2 - 1, 1),
+                  delay_user_samples=5.3, extra_delay_rate_sps=3e-8, lo1_hz=6.7e9, lo2_hz=6.7e9)
+    check(c, form)
+
+
+@pytest.mark.parametrize("form", ["plain", "chosen"])
+@pytest.mark.parametrize("n", [256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("bits,shuffles,lsb,shift,grid,delay,products", [
+    ((1, 8), (None, PERM), (False, True), 0, 0, -70.6, ACF | XCF),
+    ((8, 2), (PERM, None), (True, False), 5, 1, 33.2, ACF | XCF),
+    ((4, 1), (SWAP, PERM), (True, True), -7, 0, 64.9, ACF | XCF | OV),
+    ((2, 4), (None, SWAP), (False, False), 32, 1, -31.7, XCF),
+    ((2, 2), (None, None), (False, True), 0, 1, 129.4, ACF),
+])
+def test_wave_options(n, bits, shuffles, lsb, shift, grid, delay, products, form):
+    m = n // 2
+    a1s = max(0, -shift)
+    band = (shift, a1s, min(m, m - shift), a1s + shift)
+    c = make_case(n=n, fs=64e6, nf=LINE[n] + 9, bits=bits, shuffles=shuffles, lsb=lsb, band=band, grid=grid,
+                  products=products, rho=0.3, seed=n, delay_samples=3.0, delay_user_samples=delay,
+                  lo1_hz=1.2e9, lo2_hz=1.2e9)
+    check(c, form)
+
+
+@pytest.mark.parametrize("n", [256, 2048, 4096])
+def test_wave_shift_past_the_frame(n):
+    """Station 1 shifted out of most frames: the sweep crosses +-N."""
+    fs = 64e6
+    c = make_case(n=n, fs=fs, nf=LINE[n] + 5, rho=0.3, seed=3, delay_user_samples=-1.2 * n, lo1_hz=1e9, lo2_hz=1e9,
+                  extra_delay_rate_sps=2.4 * n / fs / ((LINE[n] + 5) * n / fs))
+    check(c, "plain")
