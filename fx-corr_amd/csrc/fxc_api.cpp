@@ -1494,10 +1494,10 @@ static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf
                 SectorArgs ca = a;
                 ca.nf = std::min(span, nf - c0);
                 ca.chain_ld = ld;
-                HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float2 *)p->d_chain.p, s));
+                HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float *)p->d_chain.p, s));
                 span0 = c0;
             }
-            a.chain = (const float2 *)p->d_chain.p + (size_t)(c0 - span0) * 2 * ld;   // rows 2f + station
+            a.chain = (const float *)p->d_chain.p + (size_t)(c0 - span0) * 4 * ld;   // rows 2f + station
             a.chain_ld = ld;
         } else {
             a.chain = nullptr;
@@ -1556,10 +1556,10 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
                 SectorArgs ca = a;
                 ca.nf = std::min(span, nf - c0);
                 ca.chain_ld = ld;
-                HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float2 *)p->d_chain.p, s));
+                HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float *)p->d_chain.p, s));
                 span0 = c0;
             }
-            a.chain = (const float2 *)p->d_chain.p + (size_t)(c0 - span0) * 2 * ld;   // rows 2f + station
+            a.chain = (const float *)p->d_chain.p + (size_t)(c0 - span0) * 4 * ld;   // rows 2f + station
             a.chain_ld = ld;
         } else {
             a.chain = nullptr;
@@ -1751,10 +1751,10 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
                 SectorArgs ca = a;
                 ca.nf = std::min(span, nf - c0);
                 ca.chain_ld = ld;
-                HIP_TRY(launch_phase_chain(ca, CHAIN_XCF, (float2 *)p->d_chain.p, s));
+                HIP_TRY(launch_phase_chain(ca, CHAIN_XCF, (float *)p->d_chain.p, s));
                 span0 = c0;
             }
-            a.chain = (const float2 *)p->d_chain.p + (size_t)(c0 - span0) * ld;
+            a.chain = (const float *)p->d_chain.p + (size_t)(c0 - span0) * 2 * ld;
             a.chain_ld = ld;
         }
         HIP_TRY(launch_mac_large(a, p->desc.precision, (const float2 *)p->d_z[0].p,
@@ -1800,8 +1800,11 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     const bool chain = p->fft_form == 0 && xcf_uses_chain(p);
     const int ld = chain ? chain_ld_for(a.ov) : 0;
     int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
-    if (chain) {
+    if (chain)
         slab = std::min<int64_t>(slab, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / ((size_t)ld * 8))));
+    // slabs of equal length (a short last one would leave most workgroups idle)
+    slab = (nf + (nf + slab - 1) / slab - 1) / ((nf + slab - 1) / slab);
+    if (chain) {
         GROW(p, p->d_chain, (size_t)slab * ld * 8, s, "phase chains");
     }
     if (wave) GROW(p, p->d_wparams, (size_t)slab * sizeof(WkParam), s, "frame parameters");
@@ -1837,9 +1840,9 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
             b.wk_params = p->d_wparams.p;
         }
         if (chain) {
-            b.chain = (const float2 *)p->d_chain.p;
+            b.chain = (const float *)p->d_chain.p;
             b.chain_ld = ld;
-            HIP_TRY(launch_phase_chain(b, CHAIN_XCF, (float2 *)p->d_chain.p, s));
+            HIP_TRY(launch_phase_chain(b, CHAIN_XCF, (float *)p->d_chain.p, s));
         }
         if (p->fft_form == 1) HIP_TRY(launch_sector_mfma(b, p->desc.precision, wgs, s));
         else if (wave) HIP_TRY(launch_sector_wave(b, p->desc.precision, wgs, s));

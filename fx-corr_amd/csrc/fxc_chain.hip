@@ -14,27 +14,40 @@
 // return exactly those, and a start one ulp away (larger band-shifted start
 // angles) moves a chain by at most ~5e-7 over 30720 links.
 //
-// One thread per chain writes its row in pairs of links (16-byte stores).
-// Blocks of one wave, so that the few long chains of a launch spread over
-// the compute units (each chain's walk is latency-bound).
+// Two adjacent lanes walk one chain, one holding its real part and the other
+// its imaginary part: a link is then own * re(step) + other * (-/+ im(step)),
+// the same products and sums, with the other lane's part read through the
+// multiply's DPP operand -- three VALU instructions and one wait state on the
+// walk's critical path.  Each chain is one sequential walk (a launch holds a
+// few hundred to a few thousand of them, far fewer than the chip's lanes), so
+// the launch time is the latency of a link.  One thread per chain with both
+// parts took 22.6 ns a link (six VALU instructions, an address and a store per
+// pair); this form takes 11..13 ns (a 128-frame FFT-2048 sector 46 -> 34 us,
+// four frames at FFT 65536 870 -> 434).  Rows are planar (chain_at): each lane
+// stores four links of its part as one 16-byte store.  Blocks of one wave, so
+// that the few long chains of a launch spread over the compute units.
 #include "fxc_dev.h"
 
 namespace fxc {
 
-__device__ __forceinline__ float2 c_mul_rust(float2 a, float2 b) {
+// The next link's part held by this lane: v * qx + other * c, other = the
+// partner lane's part (quad_perm [1, 0, 3, 2]).  Real part (c = -im step):
+// re*qx - im*qy; imaginary part (c = im step): im*qx + re*qy.
+__device__ __forceinline__ float chain_next(float v, float qx, float c) {
 #pragma clang fp contract(off)
-    const float rr = a.x * b.x;
-    const float ii = a.y * b.y;
-    const float ri = a.x * b.y;
-    const float ir = a.y * b.x;
-    return make_float2(rr - ii, ri + ir);
+    const float other = __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+    const float own = v * qx;
+    const float cross = other * c;
+    return own + cross;
 }
 
-__global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, float2 *out) {
+__global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, float *out) {
     const int nch = kind == CHAIN_XCF ? 1 : 2;
     const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.nf * nch) return;
+    const int64_t i = (int64_t)blockIdx.x * (blockDim.x / 2) + (threadIdx.x >> 1);   // chain
+    const bool im = threadIdx.x & 1;
+    if (i >= a.nf * nch) return;   // both lanes of a pair together
     const int64_t f = i / nch;
     const int s = (int)(i - f * nch);
     FrameDelayDev d;
@@ -55,21 +68,30 @@ __global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, floa
             step = polar1_f32((float)phase_step);
         }
     }
-    // row of a.chain_ld (even, >= len + (len & 1)) float2: 16-byte aligned
-    float4 *o = reinterpret_cast<float4 *>(out + i * (int64_t)a.chain_ld);
-    for (int k = 0; k < len; k += 2) {
-        const float2 q = c_mul_rust(p, step);
-        o[k >> 1] = make_float4(p.x, p.y, q.x, q.y);
-        p = c_mul_rust(q, step);
+    // this part's row: a.chain_ld floats (a multiple of 16, >= len)
+    float4 *o = reinterpret_cast<float4 *>(out + (2 * i + (im ? 1 : 0)) * (int64_t)a.chain_ld);
+    const float qx = step.x, c = im ? step.y : -step.y;
+    float v = im ? p.y : p.x;
+    for (int k = 0; k < len; k += 16, o += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float4 r;
+            r.x = v;
+            r.y = chain_next(r.x, qx, c);
+            r.z = chain_next(r.y, qx, c);
+            r.w = chain_next(r.z, qx, c);
+            o[u] = r;
+            v = chain_next(r.w, qx, c);
+        }
     }
 }
 
-hipError_t launch_phase_chain(const SectorArgs &a, int kind, float2 *out, hipStream_t s) {
+hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t s) {
     const int64_t n = a.nf * (kind == CHAIN_XCF ? 1 : 2);
     if (n <= 0) return hipSuccess;
     const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
-    if (a.chain_ld < chain_ld_for(len) || (a.chain_ld & 1)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_phase_chain, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, a, kind,
+    if (a.chain_ld < chain_ld_for(len) || (a.chain_ld & 15)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_phase_chain, dim3((unsigned)((n + 31) / 32)), dim3(64), 0, s, a, kind,
                        out);
     return hipGetLastError();
 }

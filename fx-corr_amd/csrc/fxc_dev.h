@@ -195,6 +195,12 @@ struct FrameParam {
                          // difference included) and its step per index, turns
 };
 
+// Link k of the phase chain in row `row` of a.chain.
+__device__ __forceinline__ float2 chain_at(const SectorArgs &a, int64_t row, int k) {
+    const float *r = a.chain + row * 2 * a.chain_ld;
+    return make_float2(r[k], r[a.chain_ld + k]);
+}
+
 // Per-frame parameters of the phased-array sum (k_phased_params).
 struct PhasedParam {
     int32_t s1, s2;        // integer shifts clamped to [-N, N]

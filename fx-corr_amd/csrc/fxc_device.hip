@@ -95,7 +95,7 @@ __attribute__((amdgpu_waves_per_eu(MF && E == 8 && T == 256 ? 4 : 1))) void k_se
 #pragma unroll
                     for (int i = 0; i < NB; ++i) {
                         const int g = tid + NT * i;
-                        chv[i] = (g <= M && g >= gs && g < ge) ? a.chain[f * a.chain_ld + (g - gs)]
+                        chv[i] = (g <= M && g >= gs && g < ge) ? chain_at(a, f, g - gs)
                                                                : make_float2(0.f, 0.f);
                     }
                 }
@@ -143,7 +143,7 @@ __attribute__((amdgpu_waves_per_eu(MF && E == 8 && T == 256 ? 4 : 1))) void k_se
                         const int k = g - gs;
                         float2 ph;
                         if (PREC == 0 && a.chain != nullptr) {
-                            ph = CPF ? chv[CPF ? i : 0] : a.chain[f * a.chain_ld + k];   // the reference's own chain
+                            ph = CPF ? chv[CPF ? i : 0] : chain_at(a, f, k);   // the reference's own chain
                         } else if (PREC != 0) {
                             // chosen form: the first overlap bin's phasor from
                             // the FP64 phase in turns (reduced mod 1, then the

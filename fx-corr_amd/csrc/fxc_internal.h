@@ -85,9 +85,10 @@ struct SectorArgs {
     float2 *cb_out;          // phased: combined half spectra [frame][half] for the .raw output
     int32_t variant;         // FFT pass sequence of the plain kernel (autotuned; 0 default)
     // Plain form: the reference's sequential f32 phase chains of this
-    // launch's frames, row (frame * chains_per_frame + c) of chain_ld float2
-    // (k_phase_chain); null where the kernels take FP64 powers of the step.
-    const float2 *chain;
+    // launch's frames, row (frame * chains_per_frame + c) of chain_ld real
+    // parts followed by chain_ld imaginary parts (k_phase_chain, chain_at);
+    // null where the kernels take FP64 powers of the step.
+    const float *chain;
     int32_t chain_ld;
     int32_t accumulate;      // fused plain kernel: add to the partial slots (sector in slabs)
     int32_t *err;            // plan's device error word (bit 0: a bounded hand-over wait ran out)
@@ -105,7 +106,10 @@ enum { CHAIN_XCF = 0, CHAIN_PHASED = 1 };
 // frame's bins (2.8e-6 rms; 2.6e-5 and 6.6e-6 at 1024 bins), which keeps the
 // fused N <= 1024 kernel free of a per-frame table.
 constexpr int kChainMinOverlap = 512;
-__host__ __device__ constexpr int chain_ld_for(int len) { return (len + 1) & ~1; }
+// Whole 16-link store groups, and an odd number of 64-byte lines: the chains of
+// a wave store the same link of many rows at once, and rows a power of two
+// apart would all lie on the same memory channels.
+__host__ __device__ constexpr int chain_ld_for(int len) { return ((len + 15) & ~15) | 16; }
 
 // Chosen-form MFMA tables (fxc_mfma.hip), byte offsets into one device
 // buffer.  [idx][lane] order so a wave's loads are contiguous.
@@ -207,10 +211,10 @@ hipError_t launch_add_f64(double *dst, const double *src, size_t n, hipStream_t 
 hipError_t launch_scale_add_xcf(double *ac, const double *re, const double *im, int half, double s,
                                 hipStream_t stream);
 
-// fxc_chain.hip: one thread per chain; frames [0, a.nf) of the launch,
-// rows of a.chain_ld float2 (one XCF chain of a.ov bins, or two phased
+// fxc_chain.hip: frames [0, a.nf) of the launch, rows of 2 a.chain_ld
+// floats, real parts then imaginary parts (one XCF chain of a.ov bins, or two phased
 // chains of M+1 bins, per frame).
-hipError_t launch_phase_chain(const SectorArgs &a, int kind, float2 *out, hipStream_t stream);
+hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t stream);
 
 // fxc_large.hip: N = 32768, 65536 through HBM scratch (four-step M = M1 x M2)
 struct FrameParam;

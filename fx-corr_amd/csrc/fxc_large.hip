@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_mac_large(SectorArgs a, const float2 *z
             const FrameParam &P = params[f];
             float2 phf;
             if (PREC == 0 && a.chain != nullptr) {
-                phf = a.chain[f * a.chain_ld + kk];            // the reference's own chain
+                phf = chain_at(a, f, kk);   // the reference's own chain
             } else if (PREC != 0) {
                 // chosen form: the FP64 phase in turns, reduced mod 1, then the f32 sincos
                 const float r = (float)wrap_turns(fma((double)kk, P.dth, P.phw));

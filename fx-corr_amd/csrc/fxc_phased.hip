@@ -95,15 +95,14 @@ __global__ __launch_bounds__(2 * T) void k_phased(SectorArgs a, int accumulate) 
             // rotation of bin b: the reference's own f32 chain r_b
             // (k_phase_chain, rows 2f + station of this chunk).  Loaded
             // before the decode and FFT so their latency overlaps them.
-            const float2 *chg = PREC ? nullptr : a.chain + (2 * f + gsn) * a.chain_ld;
-            const float2 *cho = PREC ? nullptr : a.chain + (2 * f + 1 - gsn) * a.chain_ld;
+            const int64_t rowg = 2 * f + gsn, rowo = 2 * f + 1 - gsn;
             float2 rg[PF ? NB : 1], ro[PF ? NB : 1];
             if constexpr (PF) {
 #pragma unroll
                 for (int i = 0; i < NB; ++i) {
                     const int g = tid + NT * i;
-                    rg[i] = g <= M ? chg[g] : make_float2(0.f, 0.f);
-                    ro[i] = (g <= M && g >= gs && g < ge) ? cho[g + sb_other] : make_float2(0.f, 0.f);
+                    rg[i] = g <= M ? chain_at(a, rowg, g) : make_float2(0.f, 0.f);
+                    ro[i] = (g <= M && g >= gs && g < ge) ? chain_at(a, rowo, g + sb_other) : make_float2(0.f, 0.f);
                 }
             }
             stage_words<T>(raw + f * st.bpf, st, ws, t);
@@ -147,14 +146,14 @@ __global__ __launch_bounds__(2 * T) void k_phased(SectorArgs a, int accumulate) 
                 }
                 if (g <= M) {
                     float2 sg = c_mul(untangle(zg, g, M, a.tw_post),
-                                      PREC ? Rg : (PF ? rg[PF ? i : 0] : chg[g]));
+                                      PREC ? Rg : (PF ? rg[PF ? i : 0] : chain_at(a, rowg, g)));
                     if (g == M) sg.y = 0.0f;                  // Nyquist (utils.rs:118-123)
                     const float2 cg = c_mul(sg, frg);
                     float2 co = make_float2(0.0f, 0.0f);
                     if (g >= gs && g < ge) {
                         const int j = g + sb_other;
                         float2 so = c_mul(untangle(zo, j, M, a.tw_post),
-                                          PREC ? Ro : (PF ? ro[PF ? i : 0] : cho[j]));
+                                          PREC ? Ro : (PF ? ro[PF ? i : 0] : chain_at(a, rowo, j)));
                         if (j == M) so.y = 0.0f;
                         co = c_mul(so, fro);
                     }
@@ -265,8 +264,8 @@ __global__ __launch_bounds__(256) void k_phased_large(SectorArgs a, const float2
         const float2 fro = gsn == 0 ? P.fr2 : P.fr1;
         float2 rg, ro = make_float2(1.f, 0.f);
         if constexpr (PREC == 0) {
-            rg = a.chain[(2 * f + gsn) * a.chain_ld + g];
-            if (in_ov) ro = a.chain[(2 * f + 1 - gsn) * a.chain_ld + j];
+            rg = chain_at(a, 2 * f + gsn, g);
+            if (in_ov) ro = chain_at(a, 2 * f + 1 - gsn, j);
         } else {
             rg = phasor_turns((double)g * (gsn == 0 ? P.th1 : P.th2));
             if (in_ov) ro = phasor_turns((double)j * (gsn == 0 ? P.th2 : P.th1));

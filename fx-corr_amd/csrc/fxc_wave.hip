@@ -33,8 +33,8 @@
 // SIMD, because 32 points, the FP64 sums and the twiddles of a lane take
 // 180..256 VGPRs.  2^27 samples per station, 2-bit, Stockham kernel -> this
 // one (microseconds; plain from N = 2048 with the phase chains): plain 256:
-// 1051 -> 369, 512: 973 -> 362, 1024: 776 -> 359, 2048: 1454 -> 909, 4096: 1600
-// -> 1078, 8192: 1335 -> 942; chosen 4096: 709 -> 498, 8192: 908 -> 730.
+// 1051 -> 369, 512: 973 -> 362, 1024: 776 -> 359, 2048: 1146 -> 638, 4096: 1510
+// -> 748, 8192: 1695 -> 911; chosen 4096: 709 -> 498, 8192: 908 -> 730.
 #include "fxc_dev.h"
 
 namespace fxc {
@@ -651,9 +651,8 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                         float2 Pp, Pm;
                         if (chain) {
                             const int kp = p - gs, km = M - p - gs;
-                            const float2 *row = a.chain + (fr + f) * a.chain_ld;
-                            Pp = c_mul(P.frmix, row[kp < 0 ? 0 : (kp >= a.ov ? a.ov - 1 : kp)]);
-                            Pm = c_mul(P.frmix, row[km < 0 ? 0 : (km >= a.ov ? a.ov - 1 : km)]);
+                            Pp = c_mul(P.frmix, chain_at(a, fr + f, kp < 0 ? 0 : (kp >= a.ov ? a.ov - 1 : kp)));
+                            Pm = c_mul(P.frmix, chain_at(a, fr + f, km < 0 ? 0 : (km >= a.ov ? a.ov - 1 : km)));
                         } else {
                             Pp = U;
                             Pm = c_mul(P.C, c_conj(U));
@@ -692,7 +691,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                 if (do_xcf && k >= 0 && k < a.ov) {
                     float2 ph;
                     if (a.chain != nullptr) {
-                        ph = c_mul(P.frmix, a.chain[(fr + f) * a.chain_ld + k]);
+                        ph = c_mul(P.frmix, chain_at(a, fr + f, k));
                     } else {
                         ph = sincos_turns((float)wrap_turns(fma((double)k, P.dth, P.phw)));
                         ph = c_scale(ph, 1.0f + fmaf((float)k, P.lam, P.lam0));
