@@ -764,14 +764,13 @@ static std::vector<uint8_t> mfma_tables(const fxc_plan *p) {
 // Two resident workgroups per CU (fxc_wave.hip).
 static int wave_wg_cap() { return 2 * num_cus(); }
 
-// The wave kernel (fxc_wave.hip) replaces the Stockham sector kernel where the
-// samples can be staged as FP16 without rounding and by whole words: ACF/XCF
-// plans at N = 256..8192 with 1/2/4/8-bit codes and levels exact in FP16 (its
+// The wave kernel (fxc_wave.hip) replaces the Stockham sector and phased
+// kernels where the samples can be staged as FP16 without rounding and by whole
+// words: plans at N = 256..8192 with 1/2/4/8-bit codes and levels exact in FP16 (its
 // figures against k_sector are at the kernel).
 // Other widths and levels, and N = 64 / 128, keep k_sector.
 static bool wave_eligible(const fxc_plan *p) {
     if (p->fft_form != 0 || p->N < 256 || p->N > 8192) return false;
-    if (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) return false;
     for (int i = 0; i < 2; ++i) {
         const int b = p->desc.st[i].bits;
         if (b != 1 && b != 2 && b != 4 && b != 8) return false;
@@ -780,14 +779,17 @@ static bool wave_eligible(const fxc_plan *p) {
 }
 
 // Whether a sector of nf frames runs on the wave kernel (variant 0 of a plan
-// that has one).  Short sectors stay on the Stockham kernel, whose workgroups
-// take one frame pair at a time: they finish sooner while the chip is not
-// full (microseconds a sector, Stockham / wave: chosen N = 4096, 64 frames 19
-// / 25, 512 frames 36 / 40, 4096 frames 105 / 90; chosen 8192, 512 frames 54 /
-// 71, 2048 frames 133 / 133; plain 1024, 256 frames 19 / 20, 2048 frames 39 /
-// 24).  Four frames per CU from N = 4096 on, one below.
+// that has one).  Short sectors stay on the Stockham kernels, whose workgroups
+// take one frame pair at a time, with no parameter launch: they finish sooner
+// while the chip is not full (microseconds a sector, Stockham / wave: chosen N
+// = 4096, 64 frames 19 / 25, 512 frames 36 / 40, 4096 frames 105 / 90; chosen
+// 8192, 512 frames 54 / 71, 2048 frames 133 / 133; plain 512, 512 frames 18 /
+// 20; plain 1024, 256 frames 19 / 20, 2048 frames 39 / 24; phased plain 512,
+// 512 frames 21 / 28, 4096 frames 45 / 33).  Four frames per CU for the phased
+// sum and from N = 4096 on, two otherwise.
 static bool wave_for(const fxc_plan *p, int64_t nf) {
-    return p->wave && p->variant == 0 && nf > (int64_t)num_cus() * (p->N <= 2048 ? 1 : 4);
+    const bool phased = (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) != 0;
+    return p->wave && p->variant == 0 && nf > (int64_t)num_cus() * (p->N <= 2048 && !phased ? 2 : 4);
 }
 
 // The wave kernel's tables (WkTables): twf holds W_M^k.
@@ -1457,9 +1459,61 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
     return FXC_OK;
 }
 
+// Phased sum on the wave kernel: equal chunks whose combined spectra (.raw) and
+// rotation chains (plain) fit kPhasedWaveBytes, so that the kernels after them
+// read both from the Infinity Cache.  A delay model with the geometric table
+// gives station 2 no delay (main.rs:184-207): its chain is all ones and is
+// neither computed nor read.
+constexpr size_t kPhasedWaveBytes = (size_t)192 << 20;
+
+static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64_t nf,
+                                      uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
+    const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
+    const size_t half = (size_t)p->half;
+    const int64_t bpf_o = plan_bpf_out(p);
+    const int prec = p->desc.precision == FXC_PRECISION_CHOSEN ? 1 : 0;
+    const int nch = prec ? 0 : (base.dly.table != nullptr ? 1 : 2);
+    const int ld = chain_ld_for((int)half);
+    const size_t per_frame = (raw ? half * 8 : 0) + (size_t)nch * ld * 8;
+    int64_t chunk = std::min(nf, kWaveSlab);
+    if (per_frame) chunk = std::min<int64_t>(chunk, (int64_t)(kPhasedWaveBytes / per_frame));
+    const int64_t nchunks = (nf + chunk - 1) / chunk;
+    chunk = (nf + nchunks - 1) / nchunks;
+    if (nch) GROW(p, p->d_chain, (size_t)chunk * nch * ld * 8, s, "phased rotation chains");
+    if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
+    GROW(p, p->d_wparams, (size_t)chunk * sizeof(WkPhased), s, "frame parameters");
+    const int64_t fpw = frames_per_wg(p, chunk, wave_wg_cap(), true);
+    const int n_wg = (int)((chunk + fpw - 1) / fpw);
+    for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
+        const int64_t cn = std::min(chunk, nf - c0);
+        SectorArgs a = base;
+        a.raw1 = base.raw1 + c0 * p->st[0].bpf;
+        a.raw2 = base.raw2 + c0 * p->st[1].bpf;
+        a.first_frame = base.first_frame + c0;
+        a.nf = cn;
+        a.frames_per_wg = fpw;
+        a.part = (double *)p->part.p;
+        a.cb_out = raw ? (float2 *)p->d_cb.p : nullptr;
+        a.accumulate = c0 > 0 ? 1 : 0;
+        a.chain = nch ? (const float *)p->d_chain.p : nullptr;
+        a.chain_ld = ld;
+        a.chains = nch;
+        HIP_TRY(launch_wave_phased_params(a, prec, (WkPhased *)p->d_wparams.p, s));
+        a.wk_params = p->d_wparams.p;
+        if (nch) HIP_TRY(launch_phase_chain(a, CHAIN_PHASED, (float *)p->d_chain.p, s));
+        HIP_TRY(launch_phased_wave(a, p->desc.precision, (int)((cn + fpw - 1) / fpw), s));
+        if (raw)
+            HIP_TRY(launch_irfft_quantise(a, (const float2 *)p->d_cb.p, cn, d_raw_out + c0 * bpf_o,
+                                          p->desc.output_lsb != 0, s));
+    }
+    HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, base.flags, d_acc, s));
+    return FXC_OK;
+}
+
 static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                  uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
     if (p->fft_form == 1) return enqueue_phased_mf3(p, base, nf, d_raw_out, d_acc, s);
+    if (wave_for(p, nf)) return enqueue_phased_wave(p, base, nf, d_raw_out, d_acc, s);
     const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
     const size_t half = (size_t)p->half;
     const int64_t bpf_o = plan_bpf_out(p);
@@ -1494,6 +1548,7 @@ static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf
                 SectorArgs ca = a;
                 ca.nf = std::min(span, nf - c0);
                 ca.chain_ld = ld;
+                ca.chains = 2;
                 HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float *)p->d_chain.p, s));
                 span0 = c0;
             }
@@ -1556,6 +1611,7 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
                 SectorArgs ca = a;
                 ca.nf = std::min(span, nf - c0);
                 ca.chain_ld = ld;
+                ca.chains = 2;
                 HIP_TRY(launch_phase_chain(ca, CHAIN_PHASED, (float *)p->d_chain.p, s));
                 span0 = c0;
             }

@@ -43,7 +43,7 @@ __device__ __forceinline__ float chain_next(float v, float qx, float c) {
 }
 
 __global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, float *out) {
-    const int nch = kind == CHAIN_XCF ? 1 : 2;
+    const int nch = kind == CHAIN_XCF ? 1 : a.chains;
     const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
     const int64_t i = (int64_t)blockIdx.x * (blockDim.x / 2) + (threadIdx.x >> 1);   // chain
     const bool im = threadIdx.x & 1;
@@ -87,7 +87,8 @@ __global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, floa
 }
 
 hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t s) {
-    const int64_t n = a.nf * (kind == CHAIN_XCF ? 1 : 2);
+    if (kind == CHAIN_PHASED && a.chains != 1 && a.chains != 2) return hipErrorInvalidValue;
+    const int64_t n = a.nf * (kind == CHAIN_XCF ? 1 : a.chains);
     if (n <= 0) return hipSuccess;
     const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
     if (a.chain_ld < chain_ld_for(len) || (a.chain_ld & 15)) return hipErrorInvalidValue;

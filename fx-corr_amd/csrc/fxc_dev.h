@@ -255,6 +255,28 @@ __device__ void make_frame_param(int64_t idx, const SectorArgs &a, int logm, Fra
     for (int b = 1; b < logm; ++b) p.pw[b] = d_mul(p.pw[b - 1], p.pw[b - 1]);
 }
 
+template <int PREC>
+__device__ void make_phased_param(int64_t idx, const SectorArgs &a, PhasedParam &p) {
+    FrameDelayDev d;
+    compute_frame_delay(idx, a.dly, d, nullptr, nullptr);
+    p.s1 = clamp_shift(d.int1, a.N);
+    p.s2 = clamp_shift(d.int2, a.N);
+    if constexpr (PREC == 0) {
+        p.fr1 = make_float2(d.fr1[0], d.fr1[1]);
+        p.fr2 = make_float2(d.fr2[0], d.fr2[1]);
+        p.th1 = p.th2 = 0.0;
+    } else {
+        double tau1, tau2, tf1, tf2;
+        frame_taus(idx, a.dly, tau1, tau2, tf1, tf2);
+        const float w1 = a.dly.lo1 == 0.0 ? 0.0f : (float)wrap_turns(-a.dly.lo1 * tf1);
+        const float w2 = a.dly.lo2 == 0.0 ? 0.0f : (float)wrap_turns(-a.dly.lo2 * tf2);
+        p.fr1 = make_float2(__builtin_amdgcn_cosf(w1), __builtin_amdgcn_sinf(w1));
+        p.fr2 = make_float2(__builtin_amdgcn_cosf(w2), __builtin_amdgcn_sinf(w2));
+        p.th1 = -a.df * d.frac1;
+        p.th2 = -a.df * d.frac2;
+    }
+}
+
 // ------------------------------------------------------------- decode
 __device__ __forceinline__ uint32_t shuffle_word(uint32_t w, const StationDev &st) {
     if (st.shuffle_kind == SHUF_PAIRSWAP) {

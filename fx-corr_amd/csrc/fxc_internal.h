@@ -90,6 +90,7 @@ struct SectorArgs {
     // null where the kernels take FP64 powers of the step.
     const float *chain;
     int32_t chain_ld;
+    int32_t chains;          // phased: chains per frame (2; 1: station 2 has no delay, its links are all 1)
     int32_t accumulate;      // fused plain kernel: add to the partial slots (sector in slabs)
     int32_t *err;            // plan's device error word (bit 0: a bounded hand-over wait ran out)
     // N = 1024 producer/consumer kernel: per-consumer FP64 totals,
@@ -193,7 +194,17 @@ struct WkParam {
     int16_t s1, s2;      // integer shifts clamped to [-N, N]
     int32_t pad;
 };
+// The phased sum's: rotation per bin th (turns, chosen form), fringe phasors,
+// and rotations of M and of 256 bins, per station.
+struct WkPhased {
+    double th[2];
+    float2 fr[2], RM[2], F1[2];
+    int16_t s1, s2;
+    int32_t pad;
+};
 // the parameters of the launch's frames, for a.wk_params
+hipError_t launch_wave_phased_params(const SectorArgs &a, int precision, WkPhased *out, hipStream_t stream);
+hipError_t launch_phased_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t stream);
 hipError_t launch_wave_params(const SectorArgs &a, int precision, WkParam *out, hipStream_t stream);
 hipError_t launch_sector_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t stream);
 

@@ -1,6 +1,7 @@
 // Fused sector kernel with wave-private FFTs, N = 256..8192: the plain form,
 // and the chosen form off the producer/consumer kernels (N = 4096 / 8192, or
-// stations on different band starts).
+// stations on different band starts; phased sums from N = 2048 on); ACF / XCF
+// products or the phased sum.
 //
 // M = N / 2 complex points per station-frame, split M = 32 x M2:
 //   m = M2 m1 + m2,  k = k1 + 32 k2
@@ -34,7 +35,11 @@
 // 180..256 VGPRs.  2^27 samples per station, 2-bit, Stockham kernel -> this
 // one (microseconds; plain from N = 2048 with the phase chains): plain 256:
 // 1051 -> 369, 512: 973 -> 362, 1024: 776 -> 359, 2048: 1146 -> 638, 4096: 1510
-// -> 748, 8192: 1695 -> 911; chosen 4096: 709 -> 498, 8192: 908 -> 730.
+// -> 748, 8192: 1695 -> 911; chosen 4096: 709 -> 498, 8192: 908 -> 730; phased
+// power, plain 256: 1675 -> 656, 1024: 1264 -> 632, 4096: 1559 -> 809; chosen
+// 2048: 694 -> 468, 4096: 792 -> 548, 8192: 1067 -> 584.
+#include <type_traits>
+
 #include "fxc_dev.h"
 
 namespace fxc {
@@ -61,14 +66,14 @@ struct Shape {
 
 }  // namespace wk
 
-template <int LOGM>
+template <int LOGM, typename P>
 struct WkShared {
     using S = wk::Shape<LOGM>;
     alignas(16) float2 z[2][S::F][S::M];
     uint32_t slut[2][4 * 256];
     alignas(16) uint16_t dlut[2][kWkDlutHalves];
     float2 w2[S::A > 1 ? S::M2 : 1];
-    WkParam pp[S::F];   // this round's frames
+    P pp[S::F];   // this round's frames
 };
 
 // Slot of element (row k1, position a B + b) of the wave's station-frame q.
@@ -495,6 +500,30 @@ __global__ __launch_bounds__(64) void k_wave_params(SectorArgs a, int precision,
     out[f] = p;
 }
 
+// The phased sum's parameters (make_phased_param), and for the chosen form the
+// rotations of bin M and of a step of 256 bins.
+template <int PREC>
+__global__ __launch_bounds__(64) void k_wave_phased_params(SectorArgs a, WkPhased *out) {
+    const int64_t f = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (f >= a.nf) return;
+    PhasedParam p;
+    make_phased_param<PREC>(a.first_frame + f, a, p);
+    WkPhased o;
+    o.th[0] = p.th1;
+    o.th[1] = p.th2;
+    o.fr[0] = p.fr1;
+    o.fr[1] = p.fr2;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        o.RM[s] = sincos_turns((float)wrap_turns((double)a.M * o.th[s]));
+        o.F1[s] = sincos_turns((float)wrap_turns(256.0 * o.th[s]));
+    }
+    o.s1 = (int16_t)p.s1;
+    o.s2 = (int16_t)p.s2;
+    o.pad = 0;
+    out[f] = o;
+}
+
 // X[p] and X[M - p] (times 2) from Z[p], Z[M - p]; w = W_N^p.
 __device__ __forceinline__ void wk_untangle(float2 a, float2 b, float2 w, float2 &xp, float2 &xm) {
     const float ex = a.x + b.x, ey = a.y - b.y;
@@ -511,14 +540,18 @@ __device__ __forceinline__ float2 wk_untangle1(float2 a, float2 b, float2 w) {
 }
 
 // SHIFT: the stations' band starts differ, so the other station's bins of a
-// pair are p + sb and M - p + sb, untangled one by one.
-template <int LOGM, bool MF, bool SHIFT>
+// pair are p + sb and M - p + sb, untangled one by one.  PH: the phased sum
+// in place of the ACF / XCF products: per bin the stations' rotations (the
+// reference's f32 chains, or phasors of the FP64 phases), fringe phasors, the
+// weighted sum cb, |cb|^2 and, for the .raw output, cb.
+template <int LOGM, bool MF, bool SHIFT, bool PH>
 __global__ __launch_bounds__(wk::Shape<LOGM>::NT)
 __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
+    using Par = std::conditional_t<PH, WkPhased, WkParam>;
     using S = wk::Shape<LOGM>;
     constexpr int M = S::M, H = M + 1, NT = S::NT, F = S::F, PPT = S::PPT, G = S::G;
     extern __shared__ __align__(16) uint8_t smem[];
-    WkShared<LOGM> &sh = *reinterpret_cast<WkShared<LOGM> *>(smem);
+    WkShared<LOGM, Par> &sh = *reinterpret_cast<WkShared<LOGM, Par> *>(smem);
     const int tid = threadIdx.x, l = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int s = wv / (S::WAVES / 2), ws = wv % (S::WAVES / 2);   // station, wave of the station
@@ -539,13 +572,16 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
         const float2 v = a.tw_post[k];
         return make_float2(v.x, -v.y);
     };
-    double acc[PPT][2][4], mid[4] = {0.0, 0.0, 0.0, 0.0};
+    constexpr int NP = PH ? 1 : 4;   // sums per bin
+    double acc[PPT][2][NP], mid[NP];
+#pragma unroll
+    for (int c = 0; c < NP; ++c) mid[c] = 0.0;
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
 #pragma unroll
         for (int e = 0; e < 2; ++e)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[j][e][c] = 0.0;
+            for (int c = 0; c < NP; ++c) acc[j][e][c] = 0.0;
 
     const int64_t f_begin = (int64_t)blockIdx.x * a.frames_per_wg;
     int64_t f_end = f_begin + a.frames_per_wg;
@@ -565,7 +601,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
     wk_load<LOGM>(raw + (f_begin + fw) * bpf, nvalid(f_begin), bits, t, w);
     float2 *zw = &sh.z[s][fw][0];
 
-    const WkParam *params = reinterpret_cast<const WkParam *>(a.wk_params);
+    const Par *params = reinterpret_cast<const Par *>(a.wk_params);
     for (int64_t fr = f_begin; fr < f_end; fr += F) {
         {
             const int nf = (int)((f_end - fr) < F ? (f_end - fr) : F);   // frames of this round
@@ -575,12 +611,12 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
             for (int tp = 0; tp < (MF ? 4 : 1); ++tp) {
                 int q = fw;
                 if constexpr (S::WPS == 1) q += (MF ? 16 * tp + (lr & 15) : lr) / S::M2;
-                const WkParam &P = params[fr + (q < nf ? q : nf - 1)];
+                const Par &P = params[fr + (q < nf ? q : nf - 1)];
                 sht[tp] = s ? P.s2 : P.s1;
             }
             // the round's parameters (read after the barrier below)
             {
-                constexpr int PW = sizeof(WkParam) / 4;
+                constexpr int PW = sizeof(Par) / 4;
                 const uint32_t *src = reinterpret_cast<const uint32_t *>(params + fr);
                 uint32_t *dst = reinterpret_cast<uint32_t *>(sh.pp);
                 for (int i = tid; i < nf * PW; i += NT) dst[i] = src[i];
@@ -618,87 +654,196 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                 }
             }
             __syncthreads();
-            // ---- products of the round's frames (main.rs:2491-2568)
-#pragma unroll 1
-            for (int f = grp; f < nf; f += G) {
-                const WkParam &P = sh.pp[f];
-                const float2 *zg = &sh.z[gst][f][0], *zo = &sh.z[gst ^ 1][f][0];
-                // rows of the wave's station-frame q are XORed by q in the
-                // single-pass swizzle
-                const int qx = S::A == 1 ? ((f % S::SPW) & (S::RB - 1)) * S::M2 : 0;
-                float2 U = make_float2(1.f, 0.f);
+            if constexpr (PH) {
+                // ---- phased sum of the round's frames (main.rs:2238-2302)
+                const float wg = 0.5f * (float)(gst == 0 ? a.w1 : a.w2);   // 1/2: the untangle's factor
+                const float wo = 0.5f * (float)(gst == 0 ? a.w2 : a.w1);
                 const bool chain = a.chain != nullptr;
-                if (do_xcf && !chain)
-                    U = sincos_turns((float)wrap_turns(fma((double)(pt - gs), P.dth, P.phw)));
+                const bool write_cb = (a.flags & FLAG_RAW_OUT) != 0 && a.cb_out != nullptr;
+                // cb of grid bin g from both stations' bins X (times 2) and
+                // rotations R; the Nyquist bins lose their imaginary part
+                // after the rotation (utils.rs:118-123)
+                auto combine = [&](int g, float2 Xg, float2 Rg, float2 frg, float2 Xo, float2 Ro, float2 fro) {
+                    float2 sg = c_mul(Xg, Rg);
+                    if (g == M) sg.y = 0.0f;
+                    const float2 cg = c_mul(sg, frg);
+                    float2 co = make_float2(0.f, 0.f);
+                    if (g >= gs && g < ge) {
+                        float2 so = c_mul(Xo, Ro);
+                        if (g + sb == M) so.y = 0.0f;
+                        co = c_mul(so, fro);
+                    }
+                    const float2 c1 = gst == 0 ? cg : co, c2 = gst == 0 ? co : cg;
+                    const float u1 = gst == 0 ? wg : wo, u2 = gst == 0 ? wo : wg;
+                    float2 cb;
+                    {
+#pragma clang fp contract(off)
+                        const float2 a1 = c_scale(c1, u1), a2 = c_scale(c2, u2);
+                        cb = make_float2(a1.x + a2.x, a1.y + a2.y);
+                    }
+                    return cb;
+                };
+                auto put_cb = [&](int64_t f, int g, float2 cb) {
+                    if (g == 0 || g == M) cb.y = 0.0f;   // main.rs:2283-2284
+                    a.cb_out[f * (M + 1) + g] = cb;
+                };
+                auto clampo = [&](int g) { const int o = g + sb; return o < 0 ? 0 : (o > M ? M : o); };
+                auto link = [&](int64_t f, int st, int b) {   // station st's chain, all ones without a delay
+                    if (st == 1 && a.chains == 1) return make_float2(1.f, 0.f);
+                    return chain_at(a, f * a.chains + st, b);
+                };
+#pragma unroll 1
+                for (int f = grp; f < nf; f += G) {
+                    const Par &P = sh.pp[f];
+                    const float2 *zg = &sh.z[gst][f][0], *zo = &sh.z[gst ^ 1][f][0];
+                    const int qx = S::A == 1 ? ((f % S::SPW) & (S::RB - 1)) * S::M2 : 0;
+                    const float2 frg = P.fr[gst], fro = P.fr[gst ^ 1];
+                    float2 Ug = make_float2(1.f, 0.f), Uo = Ug, Uom = Ug;   // rotations of p, p + sb, M - p + sb
+                    if (!chain) {
+                        Ug = sincos_turns((float)wrap_turns((double)pt * P.th[gst]));
+                        Uo = sincos_turns((float)wrap_turns((double)(pt + sb) * P.th[gst ^ 1]));
+                        if constexpr (SHIFT)
+                            Uom = sincos_turns((float)wrap_turns((double)(M - pt + sb) * P.th[gst ^ 1]));
+                    }
 #pragma unroll
-                for (int j = 0; j < PPT; ++j) {
-                    const int p = pt + NT * j;
-                    float2 gp, gm, xp, xm;   // grid station, other station
-                    wk_untangle(zg[zp[j] ^ qx], zg[zm[j] ^ qx], wp[j], gp, gm);
-                    if constexpr (SHIFT) {
-                        xp = wk_untangle1(zo[op[j][0] ^ qx], zo[op[j][1] ^ qx], ow[j][0]);
-                        xm = wk_untangle1(zo[op[j][2] ^ qx], zo[op[j][3] ^ qx], ow[j][1]);
-                    } else {
-                        wk_untangle(zo[zp[j] ^ qx], zo[zm[j] ^ qx], wp[j], xp, xm);
-                    }
-                    if (do_acf) {
-                        acc[j][0][0] += (double)norm_sqr(gp);
-                        acc[j][0][1] += (double)norm_sqr(xp);
-                        acc[j][1][0] += (double)norm_sqr(gm);
-                        acc[j][1][1] += (double)norm_sqr(xm);
-                    }
-                    if (do_xcf) {
-                        float2 Pp, Pm;
-                        if (chain) {
-                            const int kp = p - gs, km = M - p - gs;
-                            Pp = c_mul(P.frmix, chain_at(a, fr + f, kp < 0 ? 0 : (kp >= a.ov ? a.ov - 1 : kp)));
-                            Pm = c_mul(P.frmix, chain_at(a, fr + f, km < 0 ? 0 : (km >= a.ov ? a.ov - 1 : km)));
+                    for (int j = 0; j < PPT; ++j) {
+                        const int p = pt + NT * j;
+                        float2 gp, gm, xp, xm;   // grid station, other station
+                        wk_untangle(zg[zp[j] ^ qx], zg[zm[j] ^ qx], wp[j], gp, gm);
+                        if constexpr (SHIFT) {
+                            xp = wk_untangle1(zo[op[j][0] ^ qx], zo[op[j][1] ^ qx], ow[j][0]);
+                            xm = wk_untangle1(zo[op[j][2] ^ qx], zo[op[j][3] ^ qx], ow[j][1]);
                         } else {
-                            Pp = U;
-                            Pm = c_mul(P.C, c_conj(U));
-                            if constexpr (!MF) {   // plain form: the f32 step's magnitude
-                                Pp = c_scale(Pp, 1.0f + fmaf((float)(p - gs), P.lam, P.lam0));
-                                Pm = c_scale(Pm, 1.0f + fmaf((float)(M - p - gs), P.lam, P.lam0));
-                            }
-                            if (j + 1 < PPT) U = c_mul(U, P.F1);
+                            wk_untangle(zo[zp[j] ^ qx], zo[zm[j] ^ qx], wp[j], xp, xm);
                         }
-                        // station 1 times conj(station 2)
-                        const float2 vp = c_mul(gst == 0 ? c_mul(gp, c_conj(xp)) : c_mul(xp, c_conj(gp)), Pp);
-                        const float2 vm = c_mul(gst == 0 ? c_mul(gm, c_conj(xm)) : c_mul(xm, c_conj(gm)), Pm);
-                        acc[j][0][2] += (double)vp.x;
-                        acc[j][0][3] += (double)vp.y;
-                        acc[j][1][2] += (double)vm.x;
-                        acc[j][1][3] += (double)vm.y;
+                        float2 Rgp, Rgm, Rop, Rom;
+                        if (chain) {
+                            Rgp = link(fr + f, gst, p);
+                            Rgm = link(fr + f, gst, M - p);
+                            Rop = link(fr + f, gst ^ 1, clampo(p));
+                            Rom = link(fr + f, gst ^ 1, clampo(M - p));
+                        } else {
+                            Rgp = Ug;
+                            Rgm = c_mul(P.RM[gst], c_conj(Ug));
+                            Rop = Uo;
+                            Rom = SHIFT ? Uom : c_mul(P.RM[gst ^ 1], c_conj(Uo));
+                            if (j + 1 < PPT) {
+                                Ug = c_mul(Ug, P.F1[gst]);
+                                Uo = c_mul(Uo, P.F1[gst ^ 1]);
+                                if constexpr (SHIFT) Uom = c_mul(Uom, c_conj(P.F1[gst ^ 1]));
+                            }
+                        }
+                        const float2 cp = combine(p, gp, Rgp, frg, xp, Rop, fro);
+                        const float2 cm = combine(M - p, gm, Rgm, frg, xm, Rom, fro);
+                        acc[j][0][0] += (double)norm_sqr(cp);
+                        acc[j][1][0] += (double)norm_sqr(cm);
+                        if (write_cb) {
+                            put_cb(fr + f, p, cp);
+                            put_cb(fr + f, M - p, cm);
+                        }
                     }
                 }
-            }
-            // bin M / 2 pairs with itself; thread f takes frame f's
-            if (tid < nf) {
-                const int f = tid;
-                const WkParam &P = sh.pp[f];
-                const int qf = S::WPS == 1 ? f % S::SPW : 0;
-                const float2 zg = sh.z[gst][f][wk_zslot<LOGM>(qf, M / 2)];
-                const float2 g2 = make_float2(2.0f * zg.x, -2.0f * zg.y);
-                int o = M / 2 + (SHIFT ? sb : 0);
-                o = o < 0 ? 0 : (o > M ? M : o);
-                const float2 x2 = wk_untangle1(sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, o & (M - 1))],
-                                               sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, (M - o) & (M - 1))], wn(o));
-                if (do_acf) {
-                    mid[0] += (double)norm_sqr(g2);
-                    mid[1] += (double)norm_sqr(x2);
+                // bin M / 2 pairs with itself; thread f takes frame f's
+                if (tid < nf) {
+                    const int f = tid, g = M / 2;
+                    const Par &P = sh.pp[f];
+                    const int qf = S::WPS == 1 ? f % S::SPW : 0;
+                    const float2 zg = sh.z[gst][f][wk_zslot<LOGM>(qf, g)];
+                    const float2 g2 = make_float2(2.0f * zg.x, -2.0f * zg.y);
+                    const int o = clampo(g);
+                    const float2 x2 = wk_untangle1(sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, o & (M - 1))],
+                                                   sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, (M - o) & (M - 1))], wn(o));
+                    const float2 Rg = chain ? link(fr + f, gst, g)
+                                            : sincos_turns((float)wrap_turns((double)g * P.th[gst]));
+                    const float2 Ro = chain ? link(fr + f, gst ^ 1, o)
+                                            : sincos_turns((float)wrap_turns((double)o * P.th[gst ^ 1]));
+                    const float2 cb = combine(g, g2, Rg, P.fr[gst], x2, Ro, P.fr[gst ^ 1]);
+                    mid[0] += (double)norm_sqr(cb);
+                    if (write_cb) put_cb(fr + f, g, cb);
                 }
-                const int k = M / 2 - gs;
-                if (do_xcf && k >= 0 && k < a.ov) {
-                    float2 ph;
-                    if (a.chain != nullptr) {
-                        ph = c_mul(P.frmix, chain_at(a, fr + f, k));
-                    } else {
-                        ph = sincos_turns((float)wrap_turns(fma((double)k, P.dth, P.phw)));
-                        ph = c_scale(ph, 1.0f + fmaf((float)k, P.lam, P.lam0));
+            } else {
+                // ---- products of the round's frames (main.rs:2491-2568)
+    #pragma unroll 1
+                for (int f = grp; f < nf; f += G) {
+                    const Par &P = sh.pp[f];
+                    const float2 *zg = &sh.z[gst][f][0], *zo = &sh.z[gst ^ 1][f][0];
+                    // rows of the wave's station-frame q are XORed by q in the
+                    // single-pass swizzle
+                    const int qx = S::A == 1 ? ((f % S::SPW) & (S::RB - 1)) * S::M2 : 0;
+                    float2 U = make_float2(1.f, 0.f);
+                    const bool chain = a.chain != nullptr;
+                    if (do_xcf && !chain)
+                        U = sincos_turns((float)wrap_turns(fma((double)(pt - gs), P.dth, P.phw)));
+    #pragma unroll
+                    for (int j = 0; j < PPT; ++j) {
+                        const int p = pt + NT * j;
+                        float2 gp, gm, xp, xm;   // grid station, other station
+                        wk_untangle(zg[zp[j] ^ qx], zg[zm[j] ^ qx], wp[j], gp, gm);
+                        if constexpr (SHIFT) {
+                            xp = wk_untangle1(zo[op[j][0] ^ qx], zo[op[j][1] ^ qx], ow[j][0]);
+                            xm = wk_untangle1(zo[op[j][2] ^ qx], zo[op[j][3] ^ qx], ow[j][1]);
+                        } else {
+                            wk_untangle(zo[zp[j] ^ qx], zo[zm[j] ^ qx], wp[j], xp, xm);
+                        }
+                        if (do_acf) {
+                            acc[j][0][0] += (double)norm_sqr(gp);
+                            acc[j][0][1] += (double)norm_sqr(xp);
+                            acc[j][1][0] += (double)norm_sqr(gm);
+                            acc[j][1][1] += (double)norm_sqr(xm);
+                        }
+                        if (do_xcf) {
+                            float2 Pp, Pm;
+                            if (chain) {
+                                const int kp = p - gs, km = M - p - gs;
+                                Pp = c_mul(P.frmix, chain_at(a, fr + f, kp < 0 ? 0 : (kp >= a.ov ? a.ov - 1 : kp)));
+                                Pm = c_mul(P.frmix, chain_at(a, fr + f, km < 0 ? 0 : (km >= a.ov ? a.ov - 1 : km)));
+                            } else {
+                                Pp = U;
+                                Pm = c_mul(P.C, c_conj(U));
+                                if constexpr (!MF) {   // plain form: the f32 step's magnitude
+                                    Pp = c_scale(Pp, 1.0f + fmaf((float)(p - gs), P.lam, P.lam0));
+                                    Pm = c_scale(Pm, 1.0f + fmaf((float)(M - p - gs), P.lam, P.lam0));
+                                }
+                                if (j + 1 < PPT) U = c_mul(U, P.F1);
+                            }
+                            // station 1 times conj(station 2)
+                            const float2 vp = c_mul(gst == 0 ? c_mul(gp, c_conj(xp)) : c_mul(xp, c_conj(gp)), Pp);
+                            const float2 vm = c_mul(gst == 0 ? c_mul(gm, c_conj(xm)) : c_mul(xm, c_conj(gm)), Pm);
+                            acc[j][0][2] += (double)vp.x;
+                            acc[j][0][3] += (double)vp.y;
+                            acc[j][1][2] += (double)vm.x;
+                            acc[j][1][3] += (double)vm.y;
+                        }
                     }
-                    const float2 v = c_mul(gst == 0 ? c_mul(g2, c_conj(x2)) : c_mul(x2, c_conj(g2)), ph);
-                    mid[2] += (double)v.x;
-                    mid[3] += (double)v.y;
+                }
+                // bin M / 2 pairs with itself; thread f takes frame f's
+                if (tid < nf) {
+                    const int f = tid;
+                    const Par &P = sh.pp[f];
+                    const int qf = S::WPS == 1 ? f % S::SPW : 0;
+                    const float2 zg = sh.z[gst][f][wk_zslot<LOGM>(qf, M / 2)];
+                    const float2 g2 = make_float2(2.0f * zg.x, -2.0f * zg.y);
+                    int o = M / 2 + (SHIFT ? sb : 0);
+                    o = o < 0 ? 0 : (o > M ? M : o);
+                    const float2 x2 = wk_untangle1(sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, o & (M - 1))],
+                                                   sh.z[gst ^ 1][f][wk_zslot<LOGM>(qf, (M - o) & (M - 1))], wn(o));
+                    if (do_acf) {
+                        mid[0] += (double)norm_sqr(g2);
+                        mid[1] += (double)norm_sqr(x2);
+                    }
+                    const int k = M / 2 - gs;
+                    if (do_xcf && k >= 0 && k < a.ov) {
+                        float2 ph;
+                        if (a.chain != nullptr) {
+                            ph = c_mul(P.frmix, chain_at(a, fr + f, k));
+                        } else {
+                            ph = sincos_turns((float)wrap_turns(fma((double)k, P.dth, P.phw)));
+                            ph = c_scale(ph, 1.0f + fmaf((float)k, P.lam, P.lam0));
+                        }
+                        const float2 v = c_mul(gst == 0 ? c_mul(g2, c_conj(x2)) : c_mul(x2, c_conj(g2)), ph);
+                        mid[2] += (double)v.x;
+                        mid[3] += (double)v.y;
+                    }
                 }
             }
             __syncthreads();
@@ -710,33 +855,36 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
     const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
     double *out = a.part + (size_t)blockIdx.x * kNumProducts * H;
     auto put = [&](int c, int g, double v) {   // c 0 / 1: grid / other station's ACF; 2 / 3: XCF
-        const bool in_ov = g >= gs && g < ge;
-        v = in_ov || (c == 0 && !ov_only) ? 0.25 * v : 0.0;
-        const int prod = c >= 2 ? P_12R + (c - 2) : ((c == 0) == (gst == 0) ? P_11 : P_22);
+        int prod = P_PH;
+        if constexpr (!PH) {
+            const bool in_ov = g >= gs && g < ge;
+            v = in_ov || (c == 0 && !ov_only) ? 0.25 * v : 0.0;
+            prod = c >= 2 ? P_12R + (c - 2) : ((c == 0) == (gst == 0) ? P_11 : P_22);
+        }
         double *o = out + prod * H + g;
         *o = a.accumulate ? *o + v : v;
     };
-    double *red = reinterpret_cast<double *>(&sh.z[0][0][0]);   // [F][4] mids, then G > 1: [G - 1][4][M + 2]
+    double *red = reinterpret_cast<double *>(&sh.z[0][0][0]);   // [F][NP] mids, then G > 1: [G - 1][NP][M + 2]
     if (tid < F)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) red[tid * 4 + c] = mid[c];
+        for (int c = 0; c < NP; ++c) red[tid * NP + c] = mid[c];
     if constexpr (G > 1) {
-        static_assert(PPT == 1 && (4 * F + (G - 1) * 4 * (M + 2)) * 8 <= (int)sizeof(sh.z), "group sums");
-        double *gr = red + 4 * F;
+        static_assert(PPT == 1 && (NP * F + (G - 1) * NP * (M + 2)) * 8 <= (int)sizeof(sh.z), "group sums");
+        double *gr = red + NP * F;
         const int p = tid % (M / 2);
         if (grp > 0)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                gr[((grp - 1) * 4 + c) * (M + 2) + p] = acc[0][0][c];
-                gr[((grp - 1) * 4 + c) * (M + 2) + M - p] = acc[0][1][c];
+            for (int c = 0; c < NP; ++c) {
+                gr[((grp - 1) * NP + c) * (M + 2) + p] = acc[0][0][c];
+                gr[((grp - 1) * NP + c) * (M + 2) + M - p] = acc[0][1][c];
             }
         __syncthreads();
         if (grp == 0)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+            for (int c = 0; c < NP; ++c)
                 for (int k = 0; k < G - 1; ++k) {
-                    acc[0][0][c] += gr[(k * 4 + c) * (M + 2) + p];
-                    acc[0][1][c] += gr[(k * 4 + c) * (M + 2) + M - p];
+                    acc[0][0][c] += gr[(k * NP + c) * (M + 2) + p];
+                    acc[0][1][c] += gr[(k * NP + c) * (M + 2) + M - p];
                 }
     } else {
         __syncthreads();
@@ -746,26 +894,26 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
         for (int j = 0; j < PPT; ++j) {
             const int p = (G > 1 ? tid % (M / 2) : tid) + NT * j;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < NP; ++c) {
                 put(c, p, acc[j][0][c]);
                 put(c, M - p, acc[j][1][c]);
             }
         }
     }
-    if (tid < 4) {
+    if (tid < NP) {
         double v = 0.0;
-        for (int f = 0; f < F; ++f) v += red[f * 4 + tid];
+        for (int f = 0; f < F; ++f) v += red[f * NP + tid];
         put(tid, M / 2, v);
     }
 }
 
-template <int LOGM, bool MF>
+template <int LOGM, bool MF, bool PH>
 static hipError_t launch_wave_t(const SectorArgs &a, int n_wg, hipStream_t s) {
-    constexpr size_t lds = sizeof(WkShared<LOGM>);
+    constexpr size_t lds = sizeof(WkShared<LOGM, std::conditional_t<PH, WkPhased, WkParam>>);
     static_assert(2 * lds <= 160 * 1024 && wk::Shape<LOGM>::NT == 256, "two workgroups per CU");
     const dim3 grid(n_wg), block(wk::Shape<LOGM>::NT);
-    if (a.a1s == a.a2s) hipLaunchKernelGGL((k_sector_wave<LOGM, MF, false>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((k_sector_wave<LOGM, MF, true>), grid, block, lds, s, a);
+    if (a.a1s == a.a2s) hipLaunchKernelGGL((k_sector_wave<LOGM, MF, false, PH>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((k_sector_wave<LOGM, MF, true, PH>), grid, block, lds, s, a);
     return hipGetLastError();
 }
 
@@ -775,18 +923,35 @@ hipError_t launch_wave_params(const SectorArgs &a, int precision, WkParam *out, 
     return hipGetLastError();
 }
 
-hipError_t launch_sector_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t s) {
-    if (a.wk_tab == nullptr || a.wk_params == nullptr || a.frames_per_wg % wave_frames(a.N) != 0) return hipErrorInvalidValue;
+hipError_t launch_wave_phased_params(const SectorArgs &a, int precision, WkPhased *out, hipStream_t s) {
+    if (a.nf <= 0) return hipSuccess;
+    const dim3 grid((unsigned)((a.nf + 63) / 64));
+    if (precision == 0) hipLaunchKernelGGL(k_wave_phased_params<0>, grid, dim3(64), 0, s, a, out);
+    else hipLaunchKernelGGL(k_wave_phased_params<1>, grid, dim3(64), 0, s, a, out);
+    return hipGetLastError();
+}
+
+template <bool PH>
+static hipError_t launch_wave_n(const SectorArgs &a, int precision, int n_wg, hipStream_t s) {
+    if (a.wk_tab == nullptr || a.wk_params == nullptr || a.frames_per_wg % wave_frames(a.N) != 0)
+        return hipErrorInvalidValue;
     const bool mf = precision != 0 && a.mf_tab != nullptr;   // the DFT-32 operand table (scale 1)
     switch (a.N) {
-    case 256: return launch_wave_t<7, false>(a, n_wg, s);
-    case 512: return launch_wave_t<8, false>(a, n_wg, s);
-    case 1024: return mf ? launch_wave_t<9, true>(a, n_wg, s) : launch_wave_t<9, false>(a, n_wg, s);
-    case 2048: return mf ? launch_wave_t<10, true>(a, n_wg, s) : launch_wave_t<10, false>(a, n_wg, s);
-    case 4096: return mf ? launch_wave_t<11, true>(a, n_wg, s) : launch_wave_t<11, false>(a, n_wg, s);
-    case 8192: return mf ? launch_wave_t<12, true>(a, n_wg, s) : launch_wave_t<12, false>(a, n_wg, s);
+    case 256: return launch_wave_t<7, false, PH>(a, n_wg, s);
+    case 512: return launch_wave_t<8, false, PH>(a, n_wg, s);
+    case 1024: return mf ? launch_wave_t<9, true, PH>(a, n_wg, s) : launch_wave_t<9, false, PH>(a, n_wg, s);
+    case 2048: return mf ? launch_wave_t<10, true, PH>(a, n_wg, s) : launch_wave_t<10, false, PH>(a, n_wg, s);
+    case 4096: return mf ? launch_wave_t<11, true, PH>(a, n_wg, s) : launch_wave_t<11, false, PH>(a, n_wg, s);
+    case 8192: return mf ? launch_wave_t<12, true, PH>(a, n_wg, s) : launch_wave_t<12, false, PH>(a, n_wg, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_sector_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t s) {
+    return launch_wave_n<false>(a, precision, n_wg, s);
+}
+hipError_t launch_phased_wave(const SectorArgs &a, int precision, int n_wg, hipStream_t s) {
+    return launch_wave_n<true>(a, precision, n_wg, s);
 }
 
 }  // namespace fxc

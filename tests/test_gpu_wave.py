@@ -11,7 +11,7 @@ import fxref as R
 from _cases import gpu_run, make_case, oracle_run, spectra_err
 
 pytestmark = pytest.mark.gpu
-LINE = {256: 256, 512: 256, 1024: 256, 2048: 256, 4096: 1024, 8192: 1024}   # frames on 256 CUs
+LINE = {256: 512, 512: 512, 1024: 512, 2048: 512, 4096: 1024, 8192: 1024}   # frames on 256 CUs
 ACF, XCF, OV = F.PRODUCT_ACF, F.PRODUCT_XCF, F.PRODUCT_ACF_OVERLAP_ONLY
 PERM = np.random.default_rng(4).permutation(32).astype(np.int32)
 SWAP = np.arange(32, dtype=np.int32) ^ 1
@@ -63,3 +63,31 @@ def test_wave_shift_past_the_frame(n):
     c = make_case(n=n, fs=fs, nf=LINE[n] + 5, rho=0.3, seed=3, delay_user_samples=-1.2 * n, lo1_hz=1e9, lo2_hz=1e9,
                   extra_delay_rate_sps=2.4 * n / fs / ((LINE[n] + 5) * n / fs))
     check(c, "plain")
+
+
+@pytest.mark.parametrize("form", ["plain", "chosen"])
+@pytest.mark.parametrize("n,nf,shift,grid", [(256, 3001, 3, 0), (512, 1300, -5, 1), (1024, 30_000, 0, 0),
+                                             (2048, 1025, -1, 1), (4096, 6001, 0, 1), (8192, 1500, 7, 0)])
+def test_wave_phased_both_stations_delayed(n, nf, shift, grid, form):
+    """The analytic delay model gives both stations a delay (two rotation
+    chains per frame in the plain form); the larger sectors take two chunks."""
+    m, fs = n // 2, 64e6
+    a1s = max(0, -shift)
+    c = make_case(n=n, fs=fs, nf=nf, bits=(2, 4), shuffles=(None, PERM), lsb=(True, False),
+                  band=(shift, a1s, min(m, m - shift), a1s + shift), grid=grid, rho=0.4, delay_samples=3.0,
+                  products=F.PRODUCT_PHASED | F.PRODUCT_RAW_OUT, seed=n, no_table=True, net_d1_base=4.4 / fs,
+                  total_rate1_base=1e-9, net_d2_base=-2.7 / fs, total_rate2_base=-2e-9, lo1_hz=1.5e9, lo2_hz=1.4e9)
+    w, plain = (0.8, 1.1), form == "plain"
+    p = F.Plan(n, bits=c["bits"], levels=c["levels"], shuffles=c["shuffles"], lsb=c["lsb"], band=c["band"],
+               df_hz=fs / n, products=c["products"], out_grid=grid, w=w, bit_out=4,
+               precision=F.PRECISION_PLAIN_FP32 if plain else F.PRECISION_CHOSEN)
+    g = p.sector_run(c["raw1"], c["raw2"], 0, nf, F.make_delay_cfg(c["table"], **c["delay"]))
+    desc = dict(fft_len=n, bits1=2, bits2=4, levels1=c["levels"][0], levels2=c["levels"][1],
+                shuffle1=c["shuffles"][0], shuffle2=c["shuffles"][1], lsb1=1, lsb2=0, a1s=c["band"][1],
+                a1e=c["band"][2], a2s=c["band"][3], out_grid=grid, df_hz=fs / n, need_acf=0, need_xcf=0,
+                need_phased=1, write_raw=1, w1=w[0], w2=w[1], bit_out=4, output_lsb=0, cpu_threads=8)
+    o = R.sector_run(desc, c["raw1"], c["raw2"], 0, nf, R.make_delay_cfg(c["table"], **c["delay"]),
+                     mode=R.MODE_F32 if plain else R.MODE_F64, threads=8)
+    # power: the forms' bars; codes: a byte holds two, each may flip at a decision boundary (1e-4 of codes)
+    assert np.max(np.abs(g["acc_ph"] / o["acc_ph"] - 1)) < (1e-5 if plain else 1e-4)
+    assert np.count_nonzero(g["raw_out"] != o["raw_out"]) <= 2e-4 * o["raw_out"].size + 2
