@@ -1623,13 +1623,11 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
         HIP_TRY(launch_phased_large(a, prec, (const float2 *)p->d_z[0].p, (const float2 *)p->d_z[1].p,
                                     p->d_params.p, kLargeGroups, c0 > 0 ? 1 : 0, s));
         if (raw) {
-            // d_x[0]: conj(Z'), d_z[0]: its FFT, quantised straight from there
+            // d_x[0]: conj(Z'), quantised in its FFT's last pass
             HIP_TRY(launch_irfft_large((const float2 *)p->d_cb.p, cn, p->M1, p->M2, twl1, twl2, twm,
                                        (const float2 *)p->tw_post.p, (float2 *)p->d_x[0].p,
-                                       (float2 *)p->d_y.p, (float2 *)p->d_z[0].p,
-                                       p->desc.output_lsb != 0, nullptr, s));
-            HIP_TRY(launch_quantise_cplx(a, (const float2 *)p->d_z[0].p, cn, p->desc.output_lsb != 0,
-                                         d_raw_out + c0 * bpf_o, s));
+                                       (float2 *)p->d_y.p, nullptr, p->desc.output_lsb != 0, nullptr,
+                                       &a, d_raw_out + c0 * bpf_o, s));
         }
     }
     HIP_TRY(launch_reduce((const double *)p->part.p, kLargeGroups, p->half, base.flags, d_acc, s));
@@ -1666,14 +1664,15 @@ static int64_t fused_param_span(const fxc_plan *p) {
     return std::max<int64_t>(1, p->param_cap / p->chunk_use) * p->chunk_use;
 }
 
-// The phased sum at N = 16384 on the fused four-step (chosen form): the
+// The phased sum at N >= 16384 on the fused four-step (chosen form): the
 // same first pass, the phased bin in the second pass; as for the products,
 // both stations' bins of a pair on the same rows (band shift a multiple of
-// M1) and code widths of at most 16 bits.
+// M1) and code widths of at most 16 bits.  Variant 0 is the four-step
+// through HBM (N = 16384: the wave or Stockham kernel).
 static bool phased_fused_possible(const fxc_plan *p) {
     const int64_t sb = p->desc.a2s - p->desc.a1s;
-    return p->fft_form == 0 && p->N == 16384 && p->desc.precision == FXC_PRECISION_CHOSEN &&
-           p->mf_b1 && (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) &&
+    const bool shape = p->fft_form == 2 || (p->fft_form == 0 && p->N == 16384);
+    return shape && p->desc.precision == FXC_PRECISION_CHOSEN && p->mf_b1 && (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) &&
            (sb % 128) == 0 && p->st[0].bits <= 16 && p->st[1].bits <= 16;
 }
 
@@ -1682,29 +1681,32 @@ static bool phased_fused_ok(const fxc_plan *p) {
 }
 
 // Frame groups of the fused second pass: enough workgroups (M1 / 2 row
-// pairs x groups) for one resident round at the kernel's occupancy (three
-// workgroups per CU at M2 = 256, five at M2 = 64 / 128), at most the plan's
+// pairs x groups) for one resident round at the kernel's occupancy (five
+// workgroups per CU at M2 = 64, four at 128 and 256), at most the plan's
 // partial slots.
 static int large_fused_groups(const fxc_plan *p) {
-    const int per_cu = p->M2 == 256 ? 3 : 5;
+    const int per_cu = p->M2 == 64 ? 5 : 4;
     return std::max(1, std::min(p->max_wg, num_cus() * per_cu / (p->M1 / 2)));
 }
 
-// Phased sum at N = 16384 on the fused four-step: per chunk the phased
-// parameters and shifts, the fused first pass of both stations, the second
-// pass with the phased bin into the frame-group partial slots (pair-major)
-// and, for the .raw output, the inverse real FFT as a four-step too: the
+// Phased sum on the fused four-step: per chunk the phased parameters and
+// shifts, the fused first pass of both stations, the second pass with the
+// phased bin into the frame-group partial slots (pair-major) and, for the
+// .raw output, the inverse real FFT as a four-step too.  N = 16384: the
 // second pass forms the half-length spectrum of each pair's rows and their
 // DFT-64 (rows of 128 x 64 per frame), the column kernel the DFT-128 over
-// the rows and the quantiser.
+// the rows and the quantiser.  N = 32768 / 65536: the second pass leaves the
+// phased spectra as rows, the inverse's first pass takes the rows as they
+// are, its second ends in natural order with the quantiser.
 static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                        uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
     const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
     const int64_t bpf_o = plan_bpf_out(p);
     // the .raw second pass holds four waves per SIMD (the power-only one
     // five): one resident round of workgroups at that occupancy
-    const int ng = raw ? std::max(1, std::min(p->max_wg, num_cus() * 4 / (p->M1 / 2)))
-                       : large_fused_groups(p);
+    const int ng = raw && p->M2 == 64 ? std::max(1, std::min(p->max_wg, num_cus() * 4 / (p->M1 / 2)))
+                                      : large_fused_groups(p);
+    const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
     if (raw) GROW(p, p->d_cb, (size_t)p->chunk_use * p->half * 8, s, "phased spectra");
     const int64_t span = fused_param_span(p);
     int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
@@ -1728,9 +1730,14 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
         HIP_TRY(launch_large_pass1_fused(a, shifts, (float2 *)p->d_z[0].p, (float2 *)p->d_z[1].p,
                                          p->M1, p->M2, (const float2 *)p->tw_lm.p, s));
         HIP_TRY(launch_large_pass2_phased(a, (const float2 *)p->d_z[0].p, (const float2 *)p->d_z[1].p,
-                                          pp, p->M1, p->M2, (const float2 *)p->tw_l0.p,
+                                          pp, p->M1, p->M2, twl2,
                                           (const float2 *)p->tw_lm.p, raw, ng, c0 > 0 ? 1 : 0, s));
-        if (raw)   // the inverse FFT's row half done: columns and quantiser
+        if (raw && p->M2 != 64) {
+            HIP_TRY(launch_irfft_rows_quantise(a, (const float2 *)p->d_cb.p, cn, p->M1, p->M2,
+                                               (const float2 *)p->tw_l1.p, twl2, (const float2 *)p->tw_lm.p,
+                                               (float2 *)p->d_y.p, d_raw_out + c0 * bpf_o,
+                                               p->desc.output_lsb != 0, s));
+        } else if (raw)   // the inverse FFT's row half done: columns and quantiser
             HIP_TRY(launch_irfft_cols_quantise(a, (const float2 *)p->d_cb.p, cn, d_raw_out + c0 * bpf_o,
                                                p->desc.output_lsb != 0, (const float2 *)p->tw_lm.p, s));
     }
@@ -1844,8 +1851,8 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     a.raw2 = d_raw2;
     a.first_frame = first_frame;
     a.nf = nf;
-    if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased && phased_fused_ok(p)) return enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s);
+    if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
     if (p->fft_form == 2 || large_fused_ok(p)) return enqueue_large(p, a, nf, d_acc, s);
     const bool wave = wave_for(p, nf);
@@ -2350,7 +2357,7 @@ static fxc_status run_fft(fxc_plan *p, const float *in, int64_t nframes, float *
                                        (const float2 *)(p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p),
                                        (const float2 *)p->tw_lm.p, (const float2 *)p->tw_post.p,
                                        (float2 *)p->d_x[0].p, (float2 *)p->d_y.p, (float2 *)p->d_z[0].p,
-                                       false, (float *)p->d_tmp_out.p + c0 * p->N, s));
+                                       false, (float *)p->d_tmp_out.p + c0 * p->N, nullptr, nullptr, s));
         }
     } else if (p->fft_form == 2) {
         for (int64_t c0 = 0; c0 < nframes; c0 += p->chunk) {   // through the chunk scratch
@@ -2550,7 +2557,7 @@ extern "C" fxc_status fxc_synth_spectral_pair_device(const fxc_synth_spectral_de
                                            (const float2 *)(p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p),
                                            (const float2 *)p->tw_lm.p, (const float2 *)p->tw_post.p,
                                            (float2 *)p->d_x[0].p, (float2 *)p->d_y.p,
-                                           (float2 *)p->d_z[0].p, false, x, s));
+                                           (float2 *)p->d_z[0].p, false, x, nullptr, nullptr, s));
             else
                 HIP_TRY(launch_irfft_frames(a, spec, cn, x, false, s));
             HIP_TRY(launch_synth_pack(x, cn * N, d->bits[stn], d->lsb[stn], d->shuffle_internal[stn],

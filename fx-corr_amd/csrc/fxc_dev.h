@@ -556,6 +556,16 @@ __device__ __forceinline__ float2 untangle_np(const float2 *zs, int k, int M, co
     return make_float2(ex + (w.x * dy - w.y * dx), ey - (w.x * dx + w.y * dy));
 }
 
+// One bin pair of the inverse's half-length spectrum: X[k], X[M - k], and
+// w = W_N^{-k}
+__device__ __forceinline__ float2 irfft_pre_pair(float2 A, float2 Bc, float2 w) {
+    const float er = A.x + Bc.x, ei = A.y - Bc.y;
+    const float dr = A.x - Bc.x, di = A.y + Bc.y;
+    const float orr = dr * w.x - di * w.y;
+    const float oi = dr * w.y + di * w.x;
+    return make_float2(er - oi, ei + orr);
+}
+
 // The inverse real FFT's input element k (< M) of the half spectrum X
 // (M + 1 bins): Z'[k] = E' + i O' (the split method run backwards), returned
 // conjugated for IFFT = conj(FFT(conj(.))).  DC/Nyquist imaginary parts are
@@ -566,13 +576,7 @@ __device__ __forceinline__ float2 irfft_pre_elem(const float2 *X, int k, int M,
     if (k == 0) {
         z = make_float2(X[0].x + X[M].x, X[0].x - X[M].x);
     } else {
-        const float2 A = X[k], Bc = X[M - k];
-        const float er = A.x + Bc.x, ei = A.y - Bc.y;
-        const float dr = A.x - Bc.x, di = A.y + Bc.y;
-        const float2 w = tw_post[k];
-        const float orr = dr * w.x - di * w.y;
-        const float oi = dr * w.y + di * w.x;
-        z = make_float2(er - oi, ei + orr);
+        z = irfft_pre_pair(X[k], X[M - k], tw_post[k]);
     }
     return c_conj(z);
 }

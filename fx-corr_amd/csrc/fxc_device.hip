@@ -939,44 +939,72 @@ hipError_t launch_irfft_quantise(const SectorArgs &a, const float2 *in, int64_t 
     }
 }
 
-// The quantiser reading the inverse FFT's complex output z (M = N/2 points
-// per frame, natural order) of the HBM four-step path: sample 2m is
-// z[m].x * scale, sample 2m + 1 is odd_sign * (z[m].y * scale), the floats
-// the staged finish kernel writes, so the words match.
-// One word per thread over a (frame, 256-word tile) grid: a frame of
-// N = 65536 samples has up to 16,384 words, and a chunk's few hundred frames
-// alone would leave the GPU at about two waves per SIMD.
-__global__ __launch_bounds__(256) void k_quantise_cplx(SectorArgs a, const float2 *z,
-                                                       int64_t nframes, int negate_odd,
-                                                       uint8_t *out) {
+// The last pass of the four-step inverse (N = 32768 / 65536) with the
+// quantiser in it: a batch of 16 columns' L-point FFTs (L = E T; k_fft_pass's
+// form), whose results k are elements c0 + c + cols k of the series, so the
+// block holds 16 consecutive elements (32 samples, a.bit_out whole words) for
+// each k.  Sample 2 m is z[m].x * scale, sample 2 m + 1 odd_sign * (z[m].y *
+// scale), the floats the staged finish kernel writes, so the words match.
+// The separate quantiser kernel read the series (8 bytes per element) back
+// from memory: 50 us per 512 frames of 32768 samples next to the pass's 35,
+// 70 in one.
+template <int E, int T>
+__global__ __launch_bounds__(16 * T) void k_fft_cols_quantise(SectorArgs a, const float2 *in, int64_t nframes,
+                                                              int cols, int64_t ics, int64_t ims,
+                                                              const float2 *tw_l, uint8_t *out,
+                                                              int negate_odd) {
+    constexpr int CB = 16, L = E * T, LP = L + L / 16 + 2;
+    __shared__ float2 buf[CB][LP];
     __shared__ float lv[256];
+    const int tid = threadIdx.x;
+    const int bpf = cols / CB;
+    const int64_t f = blockIdx.x / bpf;
+    const int c0 = (int)(blockIdx.x % bpf) * CB;
+    if (f >= nframes) return;   // uniform per workgroup
     const int nl = a.out_nlevels < 256 ? a.out_nlevels : 256;
-    for (int i = threadIdx.x; i < nl; i += blockDim.x) lv[i] = a.out_levels[i];
+    for (int i = tid; i < nl; i += CB * T) lv[i] = a.out_levels[i];
+    const float2 *src = in + f * a.M;
+    for (int i = tid; i < CB * L; i += CB * T) {
+        int c, m;
+        if (ics == 1) { c = i % CB; m = i / CB; }
+        else { m = i % L; c = i / L; }
+        buf[c][pad(m)] = src[(c0 + c) * ics + m * ims];
+    }
     __syncthreads();
-    const int nwo = a.bpf_out / 4;
-    const int w = (int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x;
-    if (w >= nwo) return;
-    const uint32_t mask = (a.bit_out >= 32) ? 0xFFFFFFFFu : ((1u << a.bit_out) - 1u);
-    const int64_t f = blockIdx.x;
-    const float2 *zf = z + f * (a.N / 2);
+    const int c = tid / T, t = tid % T;
+    float2 v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) v[r] = buf[c][pad(t + T * r)];
+    __syncthreads();
+    fft_forward<E, T>(buf[c], v, tw_l, t);   // ends with a barrier
+    const int bits = a.bit_out;
+    const uint32_t mask = (bits >= 32) ? 0xFFFFFFFFu : ((1u << bits) - 1u);
+    const QLev ql = out_qlev(a, lv);
     const float scale = 1.0f / (float)a.N;
     const float odd_sign = negate_odd ? 1.0f : -1.0f;   // main.rs:2290-2292
-    const uint32_t word = quant_word(
-        [zf, scale, odd_sign](int i) {
-            const float2 v = zf[i >> 1];
-            return (i & 1) ? odd_sign * (v.y * scale) : v.x * scale;
-        },
-        a.N, w, a.bit_out, out_qlev(a, lv), mask);
-    reinterpret_cast<uint32_t *>(out + f * a.bpf_out)[w] =
-        a.out_shuffle_ident ? word : shuffle_out_word(word, a.out_shifts);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(out + f * a.bpf_out);
+    for (int i = tid; i < L * bits; i += CB * T) {
+        const int k = i % L, w = i / L;   // word w of the 32 samples of result k
+        const uint32_t word = quant_word_any(
+            [&](int x) {
+                const float2 z = buf[x >> 1][pad(k)];
+                return (x & 1) ? odd_sign * (z.y * scale) : z.x * scale;
+            },
+            2 * CB, w, bits, ql, mask);
+        dst[(k * cols + c0) / CB * bits + w] =
+            a.out_shuffle_ident ? word : shuffle_out_word(word, a.out_shifts);
+    }
 }
 
-hipError_t launch_quantise_cplx(const SectorArgs &a, const float2 *z, int64_t nframes,
-                                bool negate_odd, uint8_t *out, hipStream_t s) {
+hipError_t launch_fft_cols_quantise(const SectorArgs &a, const float2 *in, int64_t nframes, int cols, int L,
+                                    int64_t ics, int64_t ims, const float2 *tw_l, uint8_t *out,
+                                    bool negate_odd, hipStream_t s) {
     if (nframes <= 0) return hipSuccess;
-    const int nwo = a.bpf_out / 4;
-    hipLaunchKernelGGL(k_quantise_cplx, dim3((unsigned)nframes, (unsigned)((nwo + 255) / 256)), dim3(256),
-                       0, s, a, z, nframes, negate_odd ? 1 : 0, out);
+    if ((L != 128 && L != 256) || cols % 16 != 0 || (int64_t)cols * L != a.M || a.bpf_out != a.N / 32 * a.bit_out * 4)
+        return hipErrorInvalidValue;
+    auto kern = L == 128 ? k_fft_cols_quantise<4, 32> : k_fft_cols_quantise<8, 32>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(nframes * (cols / 16))), dim3(512), 0, s, a, in, nframes, cols,
+                       ics, ims, tw_l, out, negate_odd ? 1 : 0);
     return hipGetLastError();
 }
 

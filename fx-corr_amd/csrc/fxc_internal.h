@@ -155,8 +155,6 @@ hipError_t launch_delay_eval(const DelayDev &d, int64_t first, int64_t n,
 hipError_t launch_irfft_quantise(const SectorArgs &a, const float2 *in, int64_t nframes,
                                  uint8_t *out, bool negate_odd, hipStream_t s);
 // Quantiser over the HBM four-step inverse's complex output (N >= 32768).
-hipError_t launch_quantise_cplx(const SectorArgs &a, const float2 *z, int64_t nframes,
-                                bool negate_odd, uint8_t *out, hipStream_t s);
 hipError_t launch_quantise_frames(const SectorArgs &a, const float *in,
                                   int64_t nframes, uint8_t *out,
                                   hipStream_t stream);
@@ -241,12 +239,23 @@ hipError_t launch_fft_large(const void *x, bool x_fp16, float2 *ybuf, float2 *z,
 hipError_t launch_fft_pass1_mfma(const void *in, bool in_fp16, float2 *out, int64_t nbatch, int M1,
                                  int M2, const void *b1, const float2 *tw_m, hipStream_t stream);
 // inverse real FFT of nframes half spectra X through the HBM four-step:
-// zc (M complex per frame), ybuf, z scratch; out nframes*N floats, or null
-// to leave the unscaled transform (conj-FFT input, M per frame) in z.
+// zc (M complex per frame), ybuf, z scratch; out nframes*N floats, or, with
+// q, quantised words to q_out (z and out are not used).
 hipError_t launch_irfft_large(const float2 *X, int64_t nframes, int M1, int M2, const float2 *tw1,
                               const float2 *tw2, const float2 *twm, const float2 *tw_post,
                               float2 *zc, float2 *ybuf, float2 *z, bool negate_odd, float *out,
-                              hipStream_t stream);
+                              const SectorArgs *q, uint8_t *q_out, hipStream_t stream);
+// spectra kept as the four-step's rows (M1 rows X[k1][k2] of bin k1 + M1 k2,
+// then bin M, per frame) to quantised words
+hipError_t launch_irfft_rows_quantise(const SectorArgs &a, const float2 *X, int64_t nframes, int M1, int M2,
+                                      const float2 *tw1, const float2 *tw2, const float2 *twm, float2 *ybuf,
+                                      uint8_t *out, bool negate_odd, hipStream_t stream);
+// the last pass of a four-step inverse with the quantiser in it
+// (fxc_device.hip): result k (< L) of column c (< cols, input in[c ics + k
+// ims]) is element c + cols k of the frame's M = cols L
+hipError_t launch_fft_cols_quantise(const SectorArgs &a, const float2 *in, int64_t nframes, int cols, int L,
+                                    int64_t ics, int64_t ims, const float2 *tw_l, uint8_t *out,
+                                    bool negate_odd, hipStream_t stream);
 // phased-array sum at N >= 32768 (fxc_phased.hip); pp: phased_param_bytes()
 // per frame of the chunk
 size_t phased_param_bytes();
@@ -275,10 +284,11 @@ hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, i
 hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                   const FrameParam *params, int M1, int M2, const float2 *tw_m2,
                                   int n_groups, int accumulate, hipStream_t s);
-// the phased sum on the fused second pass (N = 16384, M2 = 64); pp: the
-// chunk's phased parameters (launch_phased_params); raw: also the first
-// half of the inverse FFT into a.cb_out (M per frame), finished by
-// launch_irfft_cols_quantise (tw_m: W_M table)
+// the phased sum on the fused second pass; pp: the chunk's phased parameters
+// (launch_phased_params).  raw, M2 = 64 (N = 16384): also the first half of
+// the inverse FFT into a.cb_out (M per frame), finished by
+// launch_irfft_cols_quantise (tw_m: W_M table); M2 = 128 / 256: the spectra
+// as rows into a.cb_out (M + 1 per frame), for launch_irfft_rows
 hipError_t launch_large_pass2_phased(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                      const void *pp, int M1, int M2, const float2 *tw_m2,
                                      const float2 *tw_m, bool raw, int n_groups, int accumulate,

@@ -45,12 +45,33 @@ hipError_t launch_frame_params(const SectorArgs &a, int precision, FrameParam *p
 // at in[c*ics + m*ims] (m < L), result k written to out[c*ocs + k*oks],
 // multiplied by W_M^{(c0 + c) k} when `twiddle` (tw_m = W_M^j, j < M).
 // Loads and stores walk the unit-stride index across the threads.
-template <int E, int T, int CB>
+// ROWS (the inverse of spectra kept as four-step rows): in holds per frame
+// the M1 = cols rows X[k1][k2] of bin k1 + M1 k2 and then bin M; element
+// (column k1, k2) is conj(Z'[k1 + M1 k2]) of the half-length inverse,
+// irfft_pre_elem's arithmetic formed on the way in (bins k and M - k are in
+// rows k1 and M1 - k1, row 0 its own mirror).
+template <bool ROWS>
+__device__ __forceinline__ float2 pass_input(const float2 *src, int64_t c, int64_t m, int64_t ics, int64_t ims,
+                                             int64_t cols, int L, const float2 *tw_post) {
+    if constexpr (!ROWS) return src[c * ics + m * ims];
+    const int M1 = (int)cols, M = M1 * L, k1 = (int)c, k2 = (int)m;
+    float2 z;
+    if (k1 == 0 && k2 == 0) {
+        z = make_float2(src[0].x + src[M].x, src[0].x - src[M].x);
+    } else {
+        const int km = k1 == 0 ? L - k2 : L - 1 - k2, rm = k1 == 0 ? 0 : M1 - k1;
+        z = irfft_pre_pair(src[k1 * L + k2], src[rm * L + km], tw_post[k1 + M1 * k2]);
+    }
+    return c_conj(z);
+}
+
+template <int E, int T, int CB, bool ROWS>
 __global__ __launch_bounds__(CB *T) void k_fft_pass(const float2 *in, float2 *out, int64_t nbatch,
                                                     int64_t cols, int64_t ics, int64_t ims,
                                                     int64_t ocs, int64_t oks, int64_t frame_in,
                                                     int64_t frame_out, const float2 *tw_l,
-                                                    const float2 *tw_m, int M, int twiddle) {
+                                                    const float2 *tw_m, int M, int twiddle,
+                                                    const float2 *tw_post) {
     constexpr int L = E * T;
     constexpr int LP = L + L / 16 + 2;
     __shared__ float2 buf[CB][LP];
@@ -64,9 +85,10 @@ __global__ __launch_bounds__(CB *T) void k_fft_pass(const float2 *in, float2 *ou
     // load: unit stride along c (ics == 1) or along m (ims == 1)
     for (int i = tid; i < CB * L; i += CB * T) {
         int c, m;
-        if (ics == 1) { c = i % CB; m = i / CB; }
+        // (rows of a spectrum: along c, where the W_N^{-k} table is contiguous)
+        if (ics == 1 || ROWS) { c = i % CB; m = i / CB; }
         else { m = i % L; c = i / L; }
-        buf[c][pad(m)] = src[(c0 + c) * ics + (int64_t)m * ims];
+        buf[c][pad(m)] = pass_input<ROWS>(src, c0 + c, m, ics, ims, cols, L, tw_post);
     }
     __syncthreads();
     const int c = tid / T, t = tid % T;
@@ -89,25 +111,27 @@ template <int E, int T>
 static hipError_t launch_pass_t(const float2 *in, float2 *out, int64_t nbatch, int64_t cols,
                                 int64_t ics, int64_t ims, int64_t ocs, int64_t oks,
                                 int64_t frame_in, int64_t frame_out, const float2 *tw_l,
-                                const float2 *tw_m, int M, int twiddle, hipStream_t s) {
+                                const float2 *tw_m, int M, int twiddle, hipStream_t s,
+                                const float2 *rows_tw_post) {
     constexpr int CB = 16;
     if (cols % CB != 0) return hipErrorInvalidValue;
     const int64_t grid = nbatch * (cols / CB);
-    hipLaunchKernelGGL((k_fft_pass<E, T, CB>), dim3((unsigned)grid), dim3(CB * T), 0, s, in, out,
-                       nbatch, cols, ics, ims, ocs, oks, frame_in, frame_out, tw_l, tw_m, M,
-                       twiddle);
+    auto kern = rows_tw_post ? k_fft_pass<E, T, CB, true> : k_fft_pass<E, T, CB, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(CB * T), 0, s, in, out, nbatch, cols, ics, ims,
+                       ocs, oks, frame_in, frame_out, tw_l, tw_m, M, twiddle, rows_tw_post);
     return hipGetLastError();
 }
 
 static hipError_t launch_pass(int L, const float2 *in, float2 *out, int64_t nbatch, int64_t cols,
                               int64_t ics, int64_t ims, int64_t ocs, int64_t oks,
                               int64_t frame_in, int64_t frame_out, const float2 *tw_l,
-                              const float2 *tw_m, int M, int twiddle, hipStream_t s) {
+                              const float2 *tw_m, int M, int twiddle, hipStream_t s,
+                              const float2 *rows_tw_post = nullptr) {
     switch (L) {
     case 128: return launch_pass_t<4, 32>(in, out, nbatch, cols, ics, ims, ocs, oks, frame_in,
-                                          frame_out, tw_l, tw_m, M, twiddle, s);
+                                          frame_out, tw_l, tw_m, M, twiddle, s, rows_tw_post);
     case 256: return launch_pass_t<8, 32>(in, out, nbatch, cols, ics, ims, ocs, oks, frame_in,
-                                          frame_out, tw_l, tw_m, M, twiddle, s);
+                                          frame_out, tw_l, tw_m, M, twiddle, s, rows_tw_post);
     default: return hipErrorInvalidValue;
     }
 }
@@ -177,7 +201,7 @@ __global__ void k_irfft_finish_large(const float2 *z, int64_t nframes, int M, in
 hipError_t launch_irfft_large(const float2 *X, int64_t nframes, int M1, int M2, const float2 *tw1,
                               const float2 *tw2, const float2 *twm, const float2 *tw_post,
                               float2 *zc, float2 *ybuf, float2 *z, bool negate_odd, float *out,
-                              hipStream_t s) {
+                              const SectorArgs *q, uint8_t *q_out, hipStream_t s) {
     const int M = M1 * M2;
     const int64_t n = nframes * M;
     if (n <= 0) return hipSuccess;
@@ -185,11 +209,30 @@ hipError_t launch_irfft_large(const float2 *X, int64_t nframes, int M1, int M2, 
     hipLaunchKernelGGL(k_irfft_prepare_large, grid, dim3(256), 0, s, X, nframes, M, tw_post, zc);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    if (q != nullptr) {   // rows c = k1: result n1 = k2 of row k1 is element k1 + M1 k2 of the series
+        e = launch_pass(M1, zc, ybuf, nframes, M2, 1, M2, 1, M2, M, M, tw1, twm, M, 1, s);
+        return e != hipSuccess ? e : launch_fft_cols_quantise(*q, ybuf, nframes, M1, M2, M2, 1, tw2, q_out, negate_odd, s);
+    }
     e = launch_fft_large(zc, false, ybuf, z, nframes, M1, M2, tw1, tw2, twm, nullptr, s);
-    if (e != hipSuccess || out == nullptr) return e;   // no out: the caller reads z
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_irfft_finish_large, grid, dim3(256), 0, s, z, nframes, M, negate_odd ? 1 : 0,
                        out);
     return hipGetLastError();
+}
+
+// The same transform of spectra kept as the four-step's rows (M1 rows of M2
+// bins, then bin M, per frame), quantised: y[k1 + M1 k2] = conj(Z'[k1 + M1
+// k2]) is row k1's entry k2, so the first pass is the rows' DFT-M2 over k2
+// (formed on the way in, no pass of its own) times W_M^{n2 k1}, the second
+// the columns' DFT-M1 over k1 into n2 + M2 n1.
+hipError_t launch_irfft_rows_quantise(const SectorArgs &a, const float2 *X, int64_t nframes, int M1, int M2,
+                                      const float2 *tw1, const float2 *tw2, const float2 *twm, float2 *ybuf,
+                                      uint8_t *out, bool negate_odd, hipStream_t s) {
+    const int M = M1 * M2;
+    if (nframes <= 0) return hipSuccess;
+    hipError_t e = launch_pass(M2, X, ybuf, nframes, M1, M2, 1, M2, 1, M + 1, M, tw2, twm, M, 1, s, a.tw_post);
+    if (e != hipSuccess) return e;
+    return launch_fft_cols_quantise(a, ybuf, nframes, M2, M1, 1, M2, tw1, out, negate_odd, s);
 }
 
 // ---------------------------------------------------------- untangle + MAC
@@ -270,56 +313,21 @@ __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int L, int R, int NS>
-__device__ __forceinline__ void wave_stockham_pass(float2 *z, const float2 *tw, int lane) {
-    if constexpr (NS < L) {
-        constexpr int RR = (L / NS < R) ? (L / NS) : R;
-        constexpr int BPT = L / (64 * RR);   // butterflies per lane
-        float2 a[BPT][RR];
-#pragma unroll
-        for (int u = 0; u < BPT; ++u) {
-            const int j = lane + 64 * u;
-#pragma unroll
-            for (int r = 0; r < RR; ++r) a[u][r] = z[pad(j + r * (L / RR))];
-            if constexpr (NS > 1) {
-                const int jm = j % NS;
-#pragma unroll
-                for (int r = 1; r < RR; ++r) a[u][r] = c_mul(a[u][r], tw[r * jm * (L / (NS * RR))]);
-            }
-            dftR<RR>(a[u]);
-        }
-        wave_sync_lds();
-#pragma unroll
-        for (int u = 0; u < BPT; ++u) {
-            const int j = lane + 64 * u;
-            const int base = (j / NS) * NS * RR + (j % NS);
-#pragma unroll
-            for (int r = 0; r < RR; ++r) z[pad(base + r * NS)] = a[u][r];
-        }
-        wave_sync_lds();
-        wave_stockham_pass<L, R, NS * RR>(z, tw, lane);
-    }
-}
-
 // ------------------------------------ second pass fused with the products
 // Chosen form, both stations' bins on the same rows of the four-step (the
 // band shift a multiple of M1).  Z[k1 + M1 k2] is row k1's DFT over m2 of
 // Y[k1][m2], and bin M - k lies in row M1 - k1 (row 0 and row M1/2 are their
 // own mirrors), so the untangle of a bin needs only its row pair.
 // Workgroup (pair p, frame group): rows ra = p, rb = M1 - p (p = 0: rows 0
-// and M1/2) of both stations; the pair's post twiddles W_N^{-g} and the
-// DFT-M2 twiddles are staged in LDS once.  Per frame, wave q loads row q of
-// [grid ra, grid rb, other ra, other rb] (the next two frames' rows are
-// loaded into registers while this one is worked on) and runs its DFT-M2 in LDS
-// with wave-level syncs; after one workgroup barrier each thread takes bins
-// g = row + M1 k2 of the pair (and bin M in pair 0): the split-method
-// untangle of both stations, the ACF/XCF products with the XCF phasor from
-// the frame's FP64 phase (k_mac_large's arithmetic) and FP64 sums.  The
-// rows are double-buffered in LDS, so a frame needs only that one barrier:
-// a wave rewrites a buffer two frames later, after every thread has passed
-// the next frame's barrier and so finished this frame's bins.  The frame
-// group's partial slot holds the pair's bins contiguously (coalesced
-// stores); the reduce over the slots puts them back in bin order.
+// and M1/2) of both stations; the pair's post twiddles W_N^{-g} are staged
+// in LDS once.  The four rows of a frame are transformed by one wave (its
+// next frames' rows are loaded into registers meanwhile); after a barrier
+// each thread takes bins g = row + M1 k2 of the pair (and bin M in pair 0):
+// the split-method untangle of both stations, then the ACF/XCF products with
+// the XCF phasor from the frame's FP64 phase (k_mac_large's arithmetic) or
+// the phased bin, and FP64 sums.  The frame group's partial slot holds the
+// pair's bins contiguously (coalesced stores); the reduce over the slots
+// puts them back in bin order.
 __device__ __forceinline__ float2 untangle_ab(float2 A, float2 B, int k, int M, float2 w) {
     if (k == 0 || k == M) return make_float2(k == 0 ? A.x + A.y : A.x - A.y, 0.0f);
     const float ex = 0.5f * (A.x + B.x), ey = 0.5f * (A.y - B.y);
@@ -327,305 +335,29 @@ __device__ __forceinline__ float2 untangle_ab(float2 A, float2 B, int k, int M, 
     return make_float2(ex + (w.x * dy - w.y * dx), ey - (w.x * dx + w.y * dy));
 }
 
-template <int M2>
-__global__ __launch_bounds__(256) void k_large_pass2_mac(SectorArgs a, const float2 *y1,
-                                                         const float2 *y2, const FrameParam *params,
-                                                         int M1, const float2 *tw_m2, int64_t fpg,
-                                                         int accumulate) {
-    constexpr int E = M2 / 64;
-    constexpr int LP = M2 + M2 / 16 + 2;
-    constexpr int BPT = (2 * M2) / 256;   // bins per thread (plus bin M for thread 0 of pair 0)
-    __shared__ float2 zr[2][4][LP];       // [buffer][grid ra, grid rb, other ra, other rb]
-    __shared__ float2 twm[M2];
-    __shared__ float2 twp[2][M2];         // tw_post[row + M1 k2], rows ra / rb
-    const int M = a.M;
-    const int half = M + 1;
-    const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int p = blockIdx.x;
-    const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
-    for (int i = tid; i < M2; i += 256) twm[i] = tw_m2[i];
-    for (int i = tid; i < 2 * M2; i += 256)
-        twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
-    const int64_t g0 = (int64_t)blockIdx.y * fpg;
-    int64_t g1 = g0 + fpg;
-    if (g1 > a.nf) g1 = a.nf;
-    const bool do_acf = (a.flags & FLAG_ACF) != 0;
-    const bool do_xcf = (a.flags & FLAG_XCF) != 0;
-    const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
-    const int gs = (a.grid == 0) ? a.a1s : a.a2s;
-    const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
-    const int jo = sbo / M1;   // the other station's k2 offset (sbo is a multiple of M1)
-    // this wave's row: q = w
-    const float2 *src_row = ((w & 2) ? (a.grid == 0 ? y2 : y1) : (a.grid == 0 ? y1 : y2)) +
-                            (int64_t)((w & 1) ? rb : ra) * M2;
-    const bool nyq = p == 0 && tid == 0;
-    double acc[BPT + 1][4];
+// What a second pass forms of its bins: the products; the phased power; the
+// power and the phased spectra, rows of M2 as they come (a.cb_out, per frame
+// M1 rows, then bin M).
+enum { P2_PRODUCTS = 0, P2_PHASED = 1, P2_PHASED_CB = 2 };
+
+// A thread's sums into its entry of the partial slot (phased: the power
+// alone, the other products are not read)
+template <int NA>
+__device__ __forceinline__ void store_pair_sums(double *out, int half, int g, const double (&acc)[NA],
+                                                int accumulate) {
+    if constexpr (NA == 1) {
+        out[P_PH * half + g] = accumulate ? out[P_PH * half + g] + acc[0] : acc[0];
+    } else {
+        const int prod[4] = {P_11, P_22, P_12R, P_12I};
 #pragma unroll
-    for (int i = 0; i <= BPT; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[i][c] = 0.0;
-    // rows of frames f (cur), f + 1 and f + 2 in flight
-    float2 cur[E], nx1[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        cur[e] = g0 < g1 ? src_row[g0 * (int64_t)M + lane + 64 * e] : make_float2(0.f, 0.f);
-        nx1[e] = g0 + 1 < g1 ? src_row[(g0 + 1) * (int64_t)M + lane + 64 * e] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();   // twiddles staged
-    int b = 0;
-    for (int64_t f = g0; f < g1; ++f, b ^= 1) {
-        float2 nx2[E];
-        const bool more = f + 2 < g1;
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-            nx2[e] = more ? src_row[(f + 2) * (int64_t)M + lane + 64 * e] : make_float2(0.f, 0.f);
-        float2 *z = zr[b][w];
-        dftR<E>(cur);
-#pragma unroll
-        for (int r = 0; r < E; ++r) z[pad(lane * E + r)] = cur[r];
-        wave_sync_lds();
-        wave_stockham_pass<M2, E, E>(z, twm, lane);
-        __syncthreads();   // the four rows of frame f are ready
-        const double dth = params[f].dth, phw = params[f].phw;
-        const float2(*zb)[LP] = zr[b];
-#pragma unroll
-        for (int i = 0; i <= BPT; ++i) {
-            int g, row, k2;
-            if (i < BPT) {
-                const int j = tid + 256 * i;
-                row = j < M2 ? ra : rb;
-                k2 = j % M2;
-                g = row + M1 * k2;
-            } else {
-                if (!nyq) continue;
-                row = 0;
-                k2 = M2;
-                g = M;
-            }
-            const int bg = row == ra ? 0 : 1;
-            // mirror M - g: row 0 -> row 0, k2' = M2 - k2; else row M1 - row, k2' = M2 - 1 - k2
-            const int bm = (row == 0 ? row : M1 - row) == ra ? 0 : 1;
-            const int km = row == 0 ? (M2 - k2) & (M2 - 1) : M2 - 1 - k2;
-            const float2 Zg = zb[bg][pad(k2 & (M2 - 1))], Zm = zb[bm][pad(km)];
-            const float2 Xg = untangle_ab(Zg, Zm, g, M, twp[bg][k2 & (M2 - 1)]);
-            const bool in_ov = g >= gs && g < gs + a.ov;
-            float2 Xo = make_float2(0.0f, 0.0f);
-            if (in_ov) {
-                const int h = g + sbo, kh = k2 + jo;   // same row, k2 shifted
-                const int khm = row == 0 ? (M2 - kh) & (M2 - 1) : M2 - 1 - kh;
-                const float2 Oh = zb[2 + bg][pad(kh & (M2 - 1))];
-                const float2 Om = zb[2 + bm][pad(khm & (M2 - 1))];
-                Xo = untangle_ab(Oh, Om, h, M, twp[bg][kh & (M2 - 1)]);
-            }
-            if (do_acf) {
-                const float pgrid = (!ov_only || in_ov) ? norm_sqr(Xg) : 0.0f;
-                const float poth = in_ov ? norm_sqr(Xo) : 0.0f;
-                acc[i][0] += (double)(a.grid == 0 ? pgrid : poth);
-                acc[i][1] += (double)(a.grid == 0 ? poth : pgrid);
-            }
-            if (in_ov && do_xcf) {
-                const float r = (float)wrap_turns(fma((double)(g - gs), dth, phw));
-                const float2 phf = make_float2(__builtin_amdgcn_cosf(r), __builtin_amdgcn_sinf(r));
-                const float2 X1 = (a.grid == 0) ? Xg : Xo;
-                const float2 X2 = (a.grid == 0) ? Xo : Xg;
-                const float2 v2 = c_mul(c_mul(X1, c_conj(X2)), phf);
-                acc[i][2] += (double)v2.x;
-                acc[i][3] += (double)v2.y;
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            cur[e] = nx1[e];
-            nx1[e] = nx2[e];
-        }
-    }
-    // partial slot in pair-major order: index p 2 M2 + j (j < M2: row ra,
-    // k2 = j; else row rb, k2 = j - M2), bin M last; launch_reduce_pairs
-    // restores bin order
-    double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
-#pragma unroll
-    for (int i = 0; i <= BPT; ++i) {
-        int g;
-        if (i < BPT) {
-            g = p * 2 * M2 + tid + 256 * i;
-        } else {
-            if (!nyq) continue;
-            g = M;
-        }
-        const double prev[4] = {accumulate ? out[P_11 * half + g] : 0.0,
-                                accumulate ? out[P_22 * half + g] : 0.0,
-                                accumulate ? out[P_12R * half + g] : 0.0,
-                                accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_11 * half + g] = prev[0] + acc[i][0];
-        out[P_22 * half + g] = prev[1] + acc[i][1];
-        out[P_12R * half + g] = prev[2] + acc[i][2];
-        out[P_12I * half + g] = prev[3] + acc[i][3];
+        for (int c = 0; c < 4; ++c)
+            out[prod[c] * half + g] = (accumulate ? out[prod[c] * half + g] : 0.0) + acc[c];
     }
 }
 
-// The same second pass at M2 = 256 with two radix-16 passes per row: each
-// wave transforms one frame's four rows (lane = 16 q + j: row q, butterfly
-// j) -- the first pass from registers, its outputs multiplied by the second
-// pass's twiddles W_256^{j r} (held per lane) and transposed through LDS,
-// the second pass writing X[j + 16 r] -- so a frame costs 48 LDS accesses
-// per lane instead of the radix-4 passes' 112 over four waves.  The four
-// waves transform four frames, then after a barrier every thread forms its
-// bins of all four (k_large_pass2_mac's bin code), and a second barrier
-// frees the rows.
-__device__ __forceinline__ void pair_bins(const float2 (*zb)[274], const float2 (*twp)[256],
-                                          int tid, int M, int M1, int ra, int rb, int gs, int ov,
-                                          int sbo, int jo, int grid, bool do_acf, bool do_xcf,
-                                          bool ov_only, bool nyq, double dth, double phw,
-                                          double (&acc)[3][4]) {
-    constexpr int M2 = 256;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        int g, row, k2;
-        if (i < 2) {
-            row = i == 0 ? ra : rb;
-            k2 = tid;
-            g = row + M1 * k2;
-        } else {
-            if (!nyq) continue;
-            row = 0;
-            k2 = M2;
-            g = M;
-        }
-        const int bg = row == ra ? 0 : 1;
-        const int bm = (row == 0 ? row : M1 - row) == ra ? 0 : 1;
-        const int km = row == 0 ? (M2 - k2) & (M2 - 1) : M2 - 1 - k2;
-        const float2 Zg = zb[bg][pad(k2 & (M2 - 1))], Zm = zb[bm][pad(km)];
-        const float2 Xg = untangle_ab(Zg, Zm, g, M, twp[bg][k2 & (M2 - 1)]);
-        const bool in_ov = g >= gs && g < gs + ov;
-        float2 Xo = make_float2(0.0f, 0.0f);
-        if (in_ov) {
-            const int h = g + sbo, kh = k2 + jo;
-            const int khm = row == 0 ? (M2 - kh) & (M2 - 1) : M2 - 1 - kh;
-            const float2 Oh = zb[2 + bg][pad(kh & (M2 - 1))];
-            const float2 Om = zb[2 + bm][pad(khm & (M2 - 1))];
-            Xo = untangle_ab(Oh, Om, h, M, twp[bg][kh & (M2 - 1)]);
-        }
-        if (do_acf) {
-            const float pgrid = (!ov_only || in_ov) ? norm_sqr(Xg) : 0.0f;
-            const float poth = in_ov ? norm_sqr(Xo) : 0.0f;
-            acc[i][0] += (double)(grid == 0 ? pgrid : poth);
-            acc[i][1] += (double)(grid == 0 ? poth : pgrid);
-        }
-        if (in_ov && do_xcf) {
-            const float r = (float)wrap_turns(fma((double)(g - gs), dth, phw));
-            const float2 phf = make_float2(__builtin_amdgcn_cosf(r), __builtin_amdgcn_sinf(r));
-            const float2 X1 = (grid == 0) ? Xg : Xo;
-            const float2 X2 = (grid == 0) ? Xo : Xg;
-            const float2 v2 = c_mul(c_mul(X1, c_conj(X2)), phf);
-            acc[i][2] += (double)v2.x;
-            acc[i][3] += (double)v2.y;
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_large_pass2_r16(SectorArgs a, const float2 *y1,
-                                                         const float2 *y2, const FrameParam *params,
-                                                         int M1, const float2 *tw_m2, int64_t fpg,
-                                                         int accumulate) {
-    constexpr int M2 = 256, LP = M2 + M2 / 16 + 2;
-    __shared__ float2 zr[4][4][LP];   // [frame of the iteration = wave][grid ra, grid rb, other ra, other rb]
-    __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
-    static_assert(LP == 274, "pair_bins row pitch");
-    const int M = a.M;
-    const int half = M + 1;
-    const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int q = lane >> 4, j = lane & 15;
-    const int p = blockIdx.x;
-    const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
-    for (int i = tid; i < 2 * M2; i += 256)
-        twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
-    float2 tw[16];   // W_256^{j r}
-#pragma unroll
-    for (int r = 1; r < 16; ++r) tw[r] = tw_m2[(j * r) & (M2 - 1)];
-    const int64_t g0 = (int64_t)blockIdx.y * fpg;
-    int64_t g1 = g0 + fpg;
-    if (g1 > a.nf) g1 = a.nf;
-    const bool do_acf = (a.flags & FLAG_ACF) != 0;
-    const bool do_xcf = (a.flags & FLAG_XCF) != 0;
-    const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
-    const int gs = (a.grid == 0) ? a.a1s : a.a2s;
-    const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
-    const int jo = sbo / M1;
-    const float2 *src_row = ((q & 2) ? (a.grid == 0 ? y2 : y1) : (a.grid == 0 ? y1 : y2)) +
-                            (int64_t)((q & 1) ? rb : ra) * M2 + j;
-    const bool nyq = p == 0 && tid == 0;
-    double acc[3][4];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[i][c] = 0.0;
-    float2 cur[16];
-    {
-        const int64_t f = g0 + w;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            cur[r] = f < g1 ? src_row[f * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();   // twiddles staged
-    float2 *z = zr[w][q];
-    for (int64_t it = g0; it < g1; it += 4) {
-        const int64_t f = it + w, fn = f + 4;
-        float2 nxt[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
-        if (f < g1) {
-            dft16(cur);                                  // pass 1: inputs j + 16 r
-#pragma unroll
-            for (int r = 1; r < 16; ++r) cur[r] = c_mul(cur[r], tw[r]);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) z[pad(16 * j + r)] = cur[r];
-            wave_sync_lds();
-#pragma unroll
-            for (int r = 0; r < 16; ++r) cur[r] = z[pad(j + 16 * r)];
-            dft16(cur);                                  // pass 2
-            wave_sync_lds();
-#pragma unroll
-            for (int r = 0; r < 16; ++r) z[pad(j + 16 * r)] = cur[r];   // X[j + 16 r]
-        }
-        __syncthreads();   // the iteration's rows are ready
-        const int nfr = (int)((g1 - it) < 4 ? (g1 - it) : 4);
-        for (int s2 = 0; s2 < nfr; ++s2)
-            pair_bins(zr[s2], twp, tid, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid, do_acf, do_xcf,
-                      ov_only, nyq, params[it + s2].dth, params[it + s2].phw, acc);
-        __syncthreads();   // every thread is done with the rows
-#pragma unroll
-        for (int r = 0; r < 16; ++r) cur[r] = nxt[r];
-    }
-    // partial slot in pair-major order (as k_large_pass2_mac)
-    double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        int g;
-        if (i < 2) {
-            g = p * 2 * M2 + tid + 256 * i;
-        } else {
-            if (!nyq) continue;
-            g = M;
-        }
-        const double prev[4] = {accumulate ? out[P_11 * half + g] : 0.0,
-                                accumulate ? out[P_22 * half + g] : 0.0,
-                                accumulate ? out[P_12R * half + g] : 0.0,
-                                accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_11 * half + g] = prev[0] + acc[i][0];
-        out[P_22 * half + g] = prev[1] + acc[i][1];
-        out[P_12R * half + g] = prev[2] + acc[i][2];
-        out[P_12I * half + g] = prev[3] + acc[i][3];
-    }
-}
-
-// One bin of a row pair for the second pass at any M2: bin g = row + M1 k2
+// One bin of a row pair for the second pass: bin g = row + M1 k2
 // of row ra (rb_sel false) or rb, or bin M (nyq: row 0, k2 = M2); the
-// untangle of both stations and the ACF/XCF products (pair_bins' arithmetic).
+// untangle of both stations and the ACF/XCF products (k_mac_large's arithmetic).
 template <int M2, int LP>
 __device__ __forceinline__ void row_bin(const float2 (*zb)[LP], const float2 (*twp)[M2], bool rb_sel,
                                         int k2, bool nyq, int M, int M1, int ra, int rb, int gs, int ov,
@@ -665,148 +397,16 @@ __device__ __forceinline__ void row_bin(const float2 (*zb)[LP], const float2 (*t
     }
 }
 
-// The second pass at M2 = 64 (N = 16384, M1 = 128) with two radix-8 passes
-// per row: lane 8 q + j of wave w takes row slot q (frame 2 w + q / 4 of the
-// iteration, row q % 4 of [grid ra, grid rb, other ra, other rb]) and
-// butterfly j -- the first pass from registers (inputs j + 8 r), its outputs
-// multiplied by W_64^{j r} and transposed through LDS, the second pass
-// writing X[j + 8 r] -- so the four waves transform eight frames per
-// iteration.  After a barrier thread t forms bin t % 128 of the pair (row ra
-// for t % 128 < 64, else rb; k2 = t % 64) for frames t / 128, + 2, + 4, + 6
-// of the eight, and a second barrier frees the rows.  Threads t and t + 128
-// hold the same bin; their sums are added in that order at the end (bin M,
-// pair 0: threads 0 and 128).
-__global__ __launch_bounds__(256) void k_large_pass2_r8(SectorArgs a, const float2 *y1,
-                                                        const float2 *y2, const FrameParam *params,
-                                                        int M1, const float2 *tw_m2, int64_t fpg,
-                                                        int accumulate) {
-    constexpr int M2 = 64, LP = M2 + M2 / 16 + 2;
-    __shared__ float2 zr[8][4][LP];   // [frame of the iteration][grid ra, grid rb, other ra, other rb]
-    __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
-    __shared__ double hsum[128][4];   // threads 128..255's sums
-    __shared__ double msum[4];        // thread 128's bin-M sums (pair 0)
-    const int M = a.M;
-    const int half = M + 1;
-    const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int q = lane >> 3, j = lane & 7;
-    const int fw = q >> 2, rk = q & 3;
-    const int p = blockIdx.x;
-    const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
-    for (int i = tid; i < 2 * M2; i += 256)
-        twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
-    float2 tw[8];
-#pragma unroll
-    for (int r = 1; r < 8; ++r) tw[r] = tw_m2[(j * r) & (M2 - 1)];
-    const int64_t g0 = (int64_t)blockIdx.y * fpg;
-    int64_t g1 = g0 + fpg;
-    if (g1 > a.nf) g1 = a.nf;
-    const bool do_acf = (a.flags & FLAG_ACF) != 0;
-    const bool do_xcf = (a.flags & FLAG_XCF) != 0;
-    const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
-    const int gs = (a.grid == 0) ? a.a1s : a.a2s;
-    const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
-    const int jo = sbo / M1;
-    const float2 *src_row = ((rk & 2) ? (a.grid == 0 ? y2 : y1) : (a.grid == 0 ? y1 : y2)) +
-                            (int64_t)((rk & 1) ? rb : ra) * M2 + j;
-    const int bsel = tid & 127, fsel = tid >> 7;
-    const bool rb_sel = bsel >= M2;
-    const int k2 = bsel & (M2 - 1);
-    const bool nyq = p == 0 && bsel == 0;   // threads 0 and 128 also take bin M
-    double acc[4] = {0.0, 0.0, 0.0, 0.0}, nacc[4] = {0.0, 0.0, 0.0, 0.0};
-    const int slot = 2 * w + fw;   // this lane's frame of the iteration
-    float2 cur[8];
-    {
-        const int64_t f = g0 + slot;
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-            cur[r] = f < g1 ? src_row[f * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();   // twiddles staged
-    float2 *z = zr[slot][rk];
-    for (int64_t it = g0; it < g1; it += 8) {
-        const int64_t f = it + slot, fn = f + 8;
-        float2 nxt[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-            nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
-        if (f < g1) {
-            dftR<8>(cur);                                // pass 1: inputs j + 8 r
-#pragma unroll
-            for (int r = 1; r < 8; ++r) cur[r] = c_mul(cur[r], tw[r]);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) z[pad(8 * j + r)] = cur[r];
-            wave_sync_lds();
-#pragma unroll
-            for (int r = 0; r < 8; ++r) cur[r] = z[pad(j + 8 * r)];
-            dftR<8>(cur);                                // pass 2
-            wave_sync_lds();
-#pragma unroll
-            for (int r = 0; r < 8; ++r) z[pad(j + 8 * r)] = cur[r];   // X[j + 8 r]
-        }
-        __syncthreads();   // the iteration's rows are ready
-        const int nfr = (int)((g1 - it) < 8 ? (g1 - it) : 8);
-        for (int s2 = fsel; s2 < nfr; s2 += 2) {
-            const double dth = params[it + s2].dth, phw = params[it + s2].phw;
-            row_bin<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                            do_acf, do_xcf, ov_only, dth, phw, acc);
-            if (nyq)
-                row_bin<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                                do_acf, do_xcf, ov_only, dth, phw, nacc);
-        }
-        __syncthreads();   // every thread is done with the rows
-#pragma unroll
-        for (int r = 0; r < 8; ++r) cur[r] = nxt[r];
-    }
-    if (tid >= 128) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) hsum[bsel][c] = acc[c];
-        if (nyq)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) msum[c] = nacc[c];
-    }
-    __syncthreads();
-    if (tid >= 128) return;
-    // partial slot in pair-major order (as k_large_pass2_mac)
-    double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int g;
-        double v[4];
-        if (i == 0) {
-            g = p * 2 * M2 + bsel;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = acc[c] + hsum[bsel][c];
-        } else {
-            if (!nyq) continue;
-            g = M;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = nacc[c] + msum[c];
-        }
-        const double prev[4] = {accumulate ? out[P_11 * half + g] : 0.0,
-                                accumulate ? out[P_22 * half + g] : 0.0,
-                                accumulate ? out[P_12R * half + g] : 0.0,
-                                accumulate ? out[P_12I * half + g] : 0.0};
-        out[P_11 * half + g] = prev[0] + v[0];
-        out[P_22 * half + g] = prev[1] + v[1];
-        out[P_12R * half + g] = prev[2] + v[2];
-        out[P_12I * half + g] = prev[3] + v[3];
-    }
-}
-
 // One bin of a row pair for the phased sum (k_phased_large's per-bin
 // arithmetic, main.rs:2264-2302): both stations' untangled bins, each
 // rotated by exp(2 pi i b th) from the FP64 phase and by its fringe phasor,
-// cb = w1 c1 + w2 c2, |cb|^2 into the FP64 sum and, with cbl, cb (DC and
-// Nyquist imaginary parts zeroed) into the frame's pair rows in LDS
-// (cbl[row ra / rb][k2], bin M in *cbn).
+// cb = w1 c1 + w2 c2, |cb|^2 into the FP64 sum.  Returns cb as the inverse
+// FFT takes it (DC and Nyquist imaginary parts zeroed).
 template <int M2, int LP>
-__device__ __forceinline__ void row_bin_ph(const float2 (*zb)[LP], const float2 (*twp)[M2], bool rb_sel,
-                                           int k2, bool nyq, int M, int M1, int ra, int rb, int gs,
-                                           int ov, int sbo, int jo, int grid, const PhasedParam &P,
-                                           float w1, float w2, float2 (*cbl)[M2], float2 *cbn,
-                                           double &acc) {
+__device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float2 (*twp)[M2], bool rb_sel,
+                                             int k2, bool nyq, int M, int M1, int ra, int rb, int gs,
+                                             int ov, int sbo, int jo, int grid, const PhasedParam &P,
+                                             float w1, float w2, double &acc) {
     const int row = nyq ? 0 : (rb_sel ? rb : ra);
     if (nyq) k2 = M2;
     const int g = nyq ? M : row + M1 * k2;
@@ -839,16 +439,288 @@ __device__ __forceinline__ void row_bin_ph(const float2 (*zb)[LP], const float2 
         cb = make_float2(a1.x + a2.x, a1.y + a2.y);
     }
     acc += (double)norm_sqr(cb);
-    if (cbl) {
-        if (g == 0 || g == M) cb.y = 0.0f;                // main.rs:2283-2284
-        if (nyq) *cbn = cb;
-        else cbl[bg][k2] = cb;
+    if (g == 0 || g == M) cb.y = 0.0f;                    // main.rs:2283-2284
+    return cb;
+}
+
+// The same second pass at M2 = 256 with two radix-16 passes per row: each
+// wave transforms one frame's four rows (lane = 16 q + j: row q, butterfly
+// j) -- the first pass from registers, its outputs multiplied by the second
+// pass's twiddles W_256^{j r} and transposed through LDS, the second pass
+// writing X[j + 16 r].  The four waves transform four frames, then after a
+// barrier every thread forms two bins of all four, and a second barrier
+// frees the rows.  The twiddles are read from LDS, which leaves registers
+// (and, with rows of 271 entries, LDS) for four workgroups per CU instead of
+// three: 2^27 samples 703 -> 683 us.
+template <int MODE>
+__global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const float2 *y1,
+                                                         const float2 *y2, const void *params, int M1, const float2 *tw_m2, int64_t fpg,
+                                                         int accumulate) {
+    constexpr int M2 = 256, LP = 271;   // pad(255) + 1
+    constexpr int NA = MODE == P2_PRODUCTS ? 4 : 1;
+    __shared__ float2 zr[4][4][LP];   // [frame of the iteration = wave][grid ra, grid rb, other ra, other rb]
+    __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
+    __shared__ float2 twj[16][16];    // W_256^{j r}
+    const int M = a.M;
+    const int half = M + 1;
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int q = lane >> 4, j = lane & 15;
+    const int p = blockIdx.x;
+    const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
+    for (int i = tid; i < 2 * M2; i += 256)
+        twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
+    twj[tid >> 4][tid & 15] = tw_m2[(tid >> 4) * (tid & 15)];
+    const int64_t g0 = (int64_t)blockIdx.y * fpg;
+    int64_t g1 = g0 + fpg;
+    if (g1 > a.nf) g1 = a.nf;
+    const bool do_acf = (a.flags & FLAG_ACF) != 0;
+    const bool do_xcf = (a.flags & FLAG_XCF) != 0;
+    const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
+    const int gs = (a.grid == 0) ? a.a1s : a.a2s;
+    const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
+    const int jo = sbo / M1;
+    const float2 *src_row = ((q & 2) ? (a.grid == 0 ? y2 : y1) : (a.grid == 0 ? y1 : y2)) +
+                            (int64_t)((q & 1) ? rb : ra) * M2 + j;
+    const bool nyq = p == 0 && tid == 0;
+    const float w1 = (float)a.w1, w2 = (float)a.w2;   // phased sum
+    double acc[3][NA];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int c = 0; c < NA; ++c) acc[i][c] = 0.0;
+    float2 cur[16];
+    {
+        const int64_t f = g0 + w;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            cur[r] = f < g1 ? src_row[f * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();   // twiddles staged
+    float2 *z = zr[w][q];
+    for (int64_t it = g0; it < g1; it += 4) {
+        const int64_t f = it + w, fn = f + 4;
+        float2 nxt[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
+        if (f < g1) {
+            dft16(cur);                                  // pass 1: inputs j + 16 r
+#pragma unroll
+            for (int r = 1; r < 16; ++r) cur[r] = c_mul(cur[r], twj[r][loop_local(j)]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[pad(16 * j + r)] = cur[r];
+            wave_sync_lds();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) cur[r] = z[pad(j + 16 * r)];
+            dft16(cur);                                  // pass 2
+            wave_sync_lds();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[pad(j + 16 * r)] = cur[r];   // X[j + 16 r]
+        }
+        __syncthreads();   // the iteration's rows are ready
+        const int nfr = (int)((g1 - it) < 4 ? (g1 - it) : 4);
+        for (int s2 = 0; s2 < nfr; ++s2) {
+            if constexpr (MODE != P2_PRODUCTS) {
+                const PhasedParam P = static_cast<const PhasedParam *>(params)[it + s2];
+                float2 *cbo = MODE == P2_PHASED_CB ? a.cb_out + (it + s2) * half : nullptr;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov,
+                                                         sbo, jo, a.grid, P, w1, w2, acc[i][0]);
+                    if constexpr (MODE == P2_PHASED_CB) cbo[(i ? rb : ra) * M2 + tid] = cb;
+                }
+                if (nyq) {
+                    const float2 cn = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov,
+                                                         sbo, jo, a.grid, P, w1, w2, acc[2][0]);
+                    if constexpr (MODE == P2_PHASED_CB) cbo[M] = cn;
+                }
+            } else {
+                const FrameParam &F = static_cast<const FrameParam *>(params)[it + s2];
+                const double dth = F.dth, phw = F.phw;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    row_bin<M2, LP>(zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
+                                    do_acf, do_xcf, ov_only, dth, phw, acc[i]);
+                if (nyq)
+                    row_bin<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
+                                    do_acf, do_xcf, ov_only, dth, phw, acc[2]);
+            }
+        }
+        __syncthreads();   // every thread is done with the rows
+#pragma unroll
+        for (int r = 0; r < 16; ++r) cur[r] = nxt[r];
+    }
+    // partial slot in pair-major order (as k_large_pass2_r8)
+    double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        int g;
+        if (i < 2) {
+            g = p * 2 * M2 + tid + 256 * i;
+        } else {
+            if (!nyq) continue;
+            g = M;
+        }
+        store_pair_sums<NA>(out, half, g, acc[i], accumulate);
     }
 }
 
-// The phased sum on the second pass at M2 = 64 (N = 16384): k_large_pass2_r8
-// with the phased bin in place of the ACF/XCF products.  RAW (the .raw
-// output): the first half of the inverse real FFT as well.  The pair's cb
+// The second pass at M2 = 64 (N = 16384) and 128 (N = 32768) with two radix
+// passes per row, E = M2 / 8 points each lane: lane 8 q + j of wave w takes
+// row slot q (frame 2 w + q / 4 of the iteration, row q % 4 of [grid ra, grid
+// rb, other ra, other rb]) -- first the DFT-E of inputs j + 8 r from
+// registers, its outputs e multiplied by W_M2^{j e} and transposed through
+// LDS, then lane j the DFT-8 for e = j (and j + 8), writing X[e + E b] -- so
+// the four waves transform eight frames per iteration.  After a barrier each
+// thread forms one bin of the pair (bin t % (2 M2): row ra for the first M2,
+// else rb) of every frame (M2 = 64: of every second, threads t and t + 128
+// hold the same bin and their sums are added in that order at the end; bin M,
+// pair 0: the threads of bin 0), and a second barrier frees the rows.
+// The E-point registers cost a row two LDS round trips.  M2 = 128 had seven
+// radix-2 passes (two points per lane, one row per wave), fourteen LDS
+// accesses per point: 512 frames 65 us (products) and 75 us (phased power),
+// here 48 and 53.  M2 = 128 keeps the twiddles in LDS: in registers they
+// spill at four waves per SIMD (746 us for 2^27 samples against 699; 735
+// with three waves and no spill).
+template <int M2, int MODE>
+__global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
+    SectorArgs a, const float2 *y1, const float2 *y2, const void *params, int M1, const float2 *tw_m2,
+    int64_t fpg, int accumulate) {
+    constexpr int E = M2 / 8, LP = M2 + M2 / 16 + 2;
+    constexpr int FS = 128 / M2;                        // threads per bin
+    constexpr int NA = MODE == P2_PRODUCTS ? 4 : 1;
+    __shared__ float2 zr[8][4][LP];   // [frame of the iteration][grid ra, grid rb, other ra, other rb]
+    __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
+    __shared__ double hsum[FS > 1 ? 128 : 1][NA];   // FS = 2: threads 128..255's sums
+    __shared__ double msum[NA];                     // and thread 128's bin-M sums (pair 0)
+    const int M = a.M;
+    const int half = M + 1;
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int q = lane >> 3, j = lane & 7;
+    const int fw = q >> 2, rk = q & 3;
+    const int p = blockIdx.x;
+    const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
+    for (int i = tid; i < 2 * M2; i += 256)
+        twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
+    __shared__ float2 twj[M2 == 128 ? E : 1][8];   // W_M2^{j e}, M2 = 128 (M2 = 64: registers)
+    float2 tw[E];
+#pragma unroll
+    for (int r = 1; r < E; ++r) tw[r] = M2 == 64 ? tw_m2[(j * r) & (M2 - 1)] : make_float2(0.f, 0.f);
+    if (M2 == 128 && tid < 8 * E) twj[tid >> 3][tid & 7] = tw_m2[((tid & 7) * (tid >> 3)) & (M2 - 1)];
+    const int64_t g0 = (int64_t)blockIdx.y * fpg;
+    int64_t g1 = g0 + fpg;
+    if (g1 > a.nf) g1 = a.nf;
+    const bool do_acf = (a.flags & FLAG_ACF) != 0;
+    const bool do_xcf = (a.flags & FLAG_XCF) != 0;
+    const bool ov_only = (a.flags & FLAG_ACF_OVERLAP) != 0;
+    const float w1 = (float)a.w1, w2 = (float)a.w2;   // phased sum
+    const int gs = (a.grid == 0) ? a.a1s : a.a2s;
+    const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
+    const int jo = sbo / M1;   // the other station's k2 offset (sbo is a multiple of M1)
+    const float2 *src_row = ((rk & 2) ? (a.grid == 0 ? y2 : y1) : (a.grid == 0 ? y1 : y2)) +
+                            (int64_t)((rk & 1) ? rb : ra) * M2 + j;
+    const int bsel = tid % (2 * M2), fsel = tid / (2 * M2);
+    const bool rb_sel = bsel >= M2;
+    const int k2 = bsel & (M2 - 1);
+    const bool nyq = p == 0 && bsel == 0;   // these threads also take bin M
+    double acc[NA], nacc[NA];
+#pragma unroll
+    for (int c = 0; c < NA; ++c) acc[c] = nacc[c] = 0.0;
+    const int slot = 2 * w + fw;   // this lane's frame of the iteration
+    float2 cur[E];
+    {
+        const int64_t f = g0 + slot;
+#pragma unroll
+        for (int r = 0; r < E; ++r)
+            cur[r] = f < g1 ? src_row[f * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();   // twiddles staged
+    float2 *z = zr[slot][rk];
+    for (int64_t it = g0; it < g1; it += 8) {
+        const int64_t f = it + slot, fn = f + 8;
+        float2 nxt[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r)
+            nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
+        if (f < g1) {
+            dftR<E>(cur);                                // pass 1: inputs j + 8 r
+#pragma unroll
+            for (int r = 1; r < E; ++r) cur[r] = c_mul(cur[r], M2 == 64 ? tw[r] : twj[r][loop_local(j)]);
+#pragma unroll
+            for (int r = 0; r < E; ++r) z[pad(8 * r + j)] = cur[r];
+            wave_sync_lds();
+            float2 u[E / 8][8];
+#pragma unroll
+            for (int h = 0; h < E / 8; ++h)
+#pragma unroll
+                for (int r = 0; r < 8; ++r) u[h][r] = z[pad(8 * (j + 8 * h) + r)];
+            wave_sync_lds();
+#pragma unroll
+            for (int h = 0; h < E / 8; ++h) {
+                dftR<8>(u[h]);                           // pass 2
+#pragma unroll
+                for (int r = 0; r < 8; ++r) z[pad(j + 8 * h + E * r)] = u[h][r];   // X[e + E b]
+            }
+        }
+        __syncthreads();   // the iteration's rows are ready
+        const int nfr = (int)((g1 - it) < 8 ? (g1 - it) : 8);
+        for (int s2 = fsel; s2 < nfr; s2 += FS) {
+            if constexpr (MODE == P2_PRODUCTS) {
+                const FrameParam &F = static_cast<const FrameParam *>(params)[it + s2];
+                const double dth = F.dth, phw = F.phw;
+                row_bin<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
+                                do_acf, do_xcf, ov_only, dth, phw, acc);
+                if (nyq)
+                    row_bin<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
+                                    do_acf, do_xcf, ov_only, dth, phw, nacc);
+            } else {
+                const PhasedParam P = static_cast<const PhasedParam *>(params)[it + s2];
+                float2 *cbo = MODE == P2_PHASED_CB ? a.cb_out + (it + s2) * half : nullptr;
+                const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov,
+                                                     sbo, jo, a.grid, P, w1, w2, acc[0]);
+                if constexpr (MODE == P2_PHASED_CB) cbo[(rb_sel ? rb : ra) * M2 + k2] = cb;
+                if (nyq) {
+                    const float2 cn = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov,
+                                                         sbo, jo, a.grid, P, w1, w2, nacc[0]);
+                    if constexpr (MODE == P2_PHASED_CB) cbo[M] = cn;
+                }
+            }
+        }
+        __syncthreads();   // every thread is done with the rows
+#pragma unroll
+        for (int r = 0; r < E; ++r) cur[r] = nxt[r];
+    }
+    if constexpr (FS > 1) {
+        if (tid >= 128) {
+#pragma unroll
+            for (int c = 0; c < NA; ++c) hsum[bsel][c] = acc[c];
+            if (nyq)
+#pragma unroll
+                for (int c = 0; c < NA; ++c) msum[c] = nacc[c];
+        }
+        __syncthreads();
+        if (tid >= 128) return;
+#pragma unroll
+        for (int c = 0; c < NA; ++c) {
+            acc[c] += hsum[bsel][c];
+            if (nyq) nacc[c] += msum[c];
+        }
+    }
+    // partial slot in pair-major order: index p 2 M2 + i (i < M2: row ra,
+    // k2 = i; else row rb, k2 = i - M2), bin M last (phased: the power alone,
+    // the other products are not read); launch_reduce_pairs restores bin order
+    double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
+    store_pair_sums<NA>(out, half, p * 2 * M2 + bsel, acc, accumulate);
+    if (nyq) store_pair_sums<NA>(out, half, M, nacc, accumulate);
+}
+
+// The phased sum with the .raw output on the second pass at M2 = 64 (N =
+// 16384): k_large_pass2_r8 with the phased bin and the first half of the
+// inverse real FFT as well.  The pair's cb
 // rows of the iteration's frames are kept in LDS; after the barrier that
 // ends the bins, lanes 0..31 of wave w take (frame, row) tasks 4 w ..
 // 4 w + 3 (frame task / 2, row ra or rb), 8 lanes each: y[k] = conj(Z'[k])
@@ -857,8 +729,7 @@ __device__ __forceinline__ void row_bin_ph(const float2 (*zb)[LP], const float2 
 // the wave's own row buffers as scratch), times W_M^{n2 k1}, stored as row
 // k1 of the frame's 128 x 64 block in a.cb_out (M entries per frame).
 // k_irfft_cols_quantise finishes the transform over k1 and quantises.
-template <bool RAW>
-__global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorArgs a, const float2 *y1,
+__global__ __launch_bounds__(256, 4) void k_large_pass2_r8_ph(SectorArgs a, const float2 *y1,
                                                            const float2 *y2, const PhasedParam *pp,
                                                            int M1, const float2 *tw_m2,
                                                            const float2 *tw_m, int64_t fpg,
@@ -868,9 +739,9 @@ __global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorAr
     __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
     __shared__ double hsum[128];      // threads 128..255's sums
     __shared__ double msum;           // thread 128's bin-M sum (pair 0)
-    __shared__ float2 cbl[RAW ? 8 : 1][2][M2];   // cb of the pair's rows, per frame
+    __shared__ float2 cbl[8][2][M2];   // cb of the pair's rows, per frame
     __shared__ float2 cbn[8];                    // cb of bin M (pair 0)
-    __shared__ float2 twr[RAW ? 2 : 1][M2];      // W_M^{n2 row}, rows ra / rb
+    __shared__ float2 twr[2][M2];      // W_M^{n2 row}, rows ra / rb
     const int M = a.M;
     const int half = M + 1;
     const int tid = threadIdx.x;
@@ -882,7 +753,7 @@ __global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorAr
     const int ra = p, rb = p == 0 ? M1 / 2 : M1 - p;
     for (int i = tid; i < 2 * M2; i += 256) {
         twp[i / M2][i % M2] = a.tw_post[(i < M2 ? ra : rb) + M1 * (i % M2)];
-        if constexpr (RAW) twr[i / M2][i % M2] = tw_m[((i % M2) * (i < M2 ? ra : rb)) & (M - 1)];
+        twr[i / M2][i % M2] = tw_m[((i % M2) * (i < M2 ? ra : rb)) & (M - 1)];
     }
     float2 tw[8];
 #pragma unroll
@@ -935,15 +806,15 @@ __global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorAr
         const int nfr = (int)((g1 - it) < 8 ? (g1 - it) : 8);
         for (int s2 = fsel; s2 < nfr; s2 += 2) {
             const PhasedParam P = pp[it + s2];
-            float2(*cbf)[M2] = RAW ? cbl[RAW ? s2 : 0] : nullptr;
-            row_bin_ph<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov, sbo, jo,
-                               a.grid, P, w1, w2, cbf, cbn + s2, acc);
+            const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov,
+                                                 sbo, jo, a.grid, P, w1, w2, acc);
+            cbl[s2][rb_sel][k2] = cb;
             if (nyq)
-                row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo,
-                                   a.grid, P, w1, w2, cbf, cbn + s2, nacc);
+                cbn[s2] = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo,
+                                             a.grid, P, w1, w2, nacc);
         }
         __syncthreads();   // every thread is done with the rows; cb complete
-        if constexpr (RAW) {
+        {
             // the wave's row buffers zr[2 w][*] are scratch here: the next
             // frames' rows are written to them by this wave only
             const int task = 4 * w + (lane >> 3);
@@ -996,7 +867,7 @@ __global__ __launch_bounds__(256, RAW ? 4 : 5) void k_large_pass2_r8_ph(SectorAr
     }
     __syncthreads();
     if (tid >= 128) return;
-    // partial slot in pair-major order (as k_large_pass2_mac); the other
+    // partial slot in pair-major order (as k_large_pass2_r8); the other
     // products stay zero
     double *out = a.part + (size_t)blockIdx.y * kNumProducts * half;
 #pragma unroll
@@ -1020,16 +891,20 @@ hipError_t launch_large_pass2_phased(const SectorArgs &a, const float2 *y1, cons
                                      const float2 *tw_m, bool raw, int n_groups, int accumulate,
                                      hipStream_t s) {
     const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
-    if (M1 * M2 != a.M || sbo % M1 != 0 || M2 != 64 || M1 != 128 || (raw && !a.cb_out))
+    if (M1 * M2 != a.M || sbo % M1 != 0 || (M2 != 64 && M2 != 128 && M2 != 256) || M1 != 128 ||
+        (raw && !a.cb_out))
         return hipErrorInvalidValue;
     const int64_t fpg = (a.nf + n_groups - 1) / n_groups;
     const dim3 grid((unsigned)(M1 / 2), (unsigned)n_groups);
-    if (raw)
-        hipLaunchKernelGGL(k_large_pass2_r8_ph<true>, grid, dim3(256), 0, s, a, y1, y2,
-                           (const PhasedParam *)pp, M1, tw_m2, tw_m, fpg, accumulate);
-    else
-        hipLaunchKernelGGL(k_large_pass2_r8_ph<false>, grid, dim3(256), 0, s, a, y1, y2,
-                           (const PhasedParam *)pp, M1, tw_m2, tw_m, fpg, accumulate);
+    if (raw && M2 == 64) {
+        hipLaunchKernelGGL(k_large_pass2_r8_ph, grid, dim3(256), 0, s, a, y1, y2, (const PhasedParam *)pp,
+                           M1, tw_m2, tw_m, fpg, accumulate);
+        return hipGetLastError();
+    }
+    auto kern = M2 == 64    ? k_large_pass2_r8<64, P2_PHASED>
+                : M2 == 128 ? (raw ? k_large_pass2_r8<128, P2_PHASED_CB> : k_large_pass2_r8<128, P2_PHASED>)
+                            : (raw ? k_large_pass2_r16<P2_PHASED_CB> : k_large_pass2_r16<P2_PHASED>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, y1, y2, pp, M1, tw_m2, fpg, accumulate);
     return hipGetLastError();
 }
 
@@ -1040,15 +915,11 @@ hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const f
     if (M1 * M2 != a.M || sbo % M1 != 0 || (M2 != 64 && M2 != 128 && M2 != 256)) return hipErrorInvalidValue;
     const int64_t fpg = (a.nf + n_groups - 1) / n_groups;
     const dim3 grid((unsigned)(M1 / 2), (unsigned)n_groups);
-    if (M2 == 64)
-        hipLaunchKernelGGL(k_large_pass2_r8, grid, dim3(256), 0, s, a, y1, y2, params, M1, tw_m2, fpg,
-                           accumulate);
-    else if (M2 == 128)
-        hipLaunchKernelGGL(k_large_pass2_mac<128>, grid, dim3(256), 0, s, a, y1, y2, params, M1, tw_m2,
-                           fpg, accumulate);
-    else
-        hipLaunchKernelGGL(k_large_pass2_r16, grid, dim3(256), 0, s, a, y1, y2, params, M1, tw_m2,
-                           fpg, accumulate);
+    auto kern = M2 == 64    ? k_large_pass2_r8<64, P2_PRODUCTS>
+                : M2 == 128 ? k_large_pass2_r8<128, P2_PRODUCTS>
+                            : k_large_pass2_r16<P2_PRODUCTS>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, y1, y2, (const void *)params, M1, tw_m2, fpg,
+                       accumulate);
     return hipGetLastError();
 }
 
