@@ -164,6 +164,7 @@ struct fxc_plan {
     int grid_div = 1;        // workgroups = max_wg / grid_div
     DevBuf tw_l1, tw_l2, tw_lm, d_x[2], d_y, d_z[2], d_params, d_lshifts;
     DevBuf tw_l0;   // W_64 (the fused four-step's rows at N = 16384)
+    DevBuf tw_ly;   // W_M^{m2 k1} at [k1][m2] (the fused four-step's FP32 first pass)
     // scratch
     DevBuf part, table_dev, d_raw[2], d_acc, d_raw_out, d_tmp_in, d_tmp_out,
         d_shifts, d_cb, d_tbuf;
@@ -189,7 +190,7 @@ struct fxc_plan {
     // Every device buffer of the plan (release, byte count).
     template <class Fn> void each_buf(Fn fn) {
         DevBuf *bufs[] = {&tw_fft, &tw_post, &lev_dev[0], &lev_dev[1], &out_lev, &mf_tab, &wk_tab,
-                          &tw_l1, &tw_l2, &tw_lm, &tw_l0, &d_x[0], &d_x[1], &d_y, &d_z[0], &d_z[1],
+                          &tw_l1, &tw_l2, &tw_lm, &tw_l0, &tw_ly, &d_x[0], &d_x[1], &d_y, &d_z[0], &d_z[1],
                           &d_params, &d_lshifts, &part, &table_dev, &d_raw[0],
                           &d_raw[1], &d_acc, &d_raw_out, &d_tmp_in, &d_tmp_out, &d_shifts,
                           &d_cb, &d_tbuf, &d_chain, &d_wparams, &d_fringe, &d_err, &d_cacc};
@@ -1034,7 +1035,9 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
             // (or phased) parameters and shifts, the W_M and W_64 tables
             const size_t pb = std::max(frame_param_bytes(), phased_param_bytes());
             const int64_t per_frame = 2 * (int64_t)M * 8 + 16 + (int64_t)pb;
-            p->chunk = std::max<int64_t>(16, ((int64_t)512 << 20) / per_frame);
+            // (plain: half as much, the largest chunk that is timed)
+            const int64_t budget = (int64_t)(desc->precision == FXC_PRECISION_CHOSEN ? 512 : 256) << 20;
+            p->chunk = std::max<int64_t>(16, budget / per_frame);
             const size_t C = (size_t)p->chunk;
             auto table = [](DevBuf &b, int n) {
                 std::vector<float> t(2 * (size_t)n);
@@ -1053,6 +1056,15 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
                 p->d_lshifts.ensure(param_frames(C) * 16) != hipSuccess)
                 return cleanup(fail(FXC_ERR_NOMEM, "fused four-step scratch allocation failed"));
             p->param_cap = (int64_t)param_frames(C);
+        }
+        if (desc->precision == FXC_PRECISION_PLAIN_FP32) {
+            std::vector<float> t(2 * (size_t)M);
+            for (int k1 = 0; k1 < p->M1; ++k1)
+                for (int m2 = 0; m2 < p->M2; ++m2)
+                    std::memcpy(&t[2 * ((size_t)k1 * p->M2 + m2)], &twf[2 * (size_t)((m2 * k1) & (M - 1))], 8);
+            if (p->tw_ly.ensure(t.size() * 4) != hipSuccess ||
+                hipMemcpy(p->tw_ly.p, t.data(), t.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
+                return cleanup(fail(FXC_ERR_NOMEM, "fused four-step table upload failed"));
         }
     }
     p->max_wg = p->fft_form == 1 ? cus
@@ -1644,13 +1656,21 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
 // The fused four-step runs at M1 = 128 (variant 1 of the large form).
 // The fused four-step (M1 = 128): N = 32768 / 65536 (the large form's
 // default), and N = 16384 (M2 = 64) as variant 1 of the Stockham form.
+// The plain form takes it with an FP32 first pass and, for the XCF, the
+// phase chains link-major (an XCF over few bins, which uses no chains, stays
+// on the Stockham kernel / the four-step through HBM): 2^27 samples of both
+// stations 1808 -> 978 us at N = 16384, 2468 -> 1228 at 32768, 2699 -> 1523
+// at 65536; the phased sum 1853 -> 1005, 2640 -> 1208 and 2798 -> 1480, with
+// the .raw output 2633 -> 1537, 3970 -> 2524 and 4112 -> 2758.
 static bool large_fused_possible(const fxc_plan *p) {
     const int64_t sb = p->desc.a2s - p->desc.a1s;
     const bool shape = (p->fft_form == 2 && (p->M / 128 == 128 || p->M / 128 == 256)) ||
                        (p->fft_form == 0 && p->N == 16384);
-    return shape && p->desc.precision == FXC_PRECISION_CHOSEN && p->mf_b1 &&
-           !(p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) && (sb % 128) == 0 &&
-           p->st[0].bits <= 16 && p->st[1].bits <= 16;
+    const bool form = p->desc.precision == FXC_PRECISION_CHOSEN
+                          ? p->mf_b1
+                          : !(p->desc.products & FXC_PRODUCT_XCF) || xcf_uses_chain(p);
+    return shape && form && !(p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) &&
+           (sb % 128) == 0 && p->st[0].bits <= 16 && p->st[1].bits <= 16;
 }
 
 static bool large_fused_ok(const fxc_plan *p) {
@@ -1664,7 +1684,7 @@ static int64_t fused_param_span(const fxc_plan *p) {
     return std::max<int64_t>(1, p->param_cap / p->chunk_use) * p->chunk_use;
 }
 
-// The phased sum at N >= 16384 on the fused four-step (chosen form): the
+// The phased sum at N >= 16384 on the fused four-step: the
 // same first pass, the phased bin in the second pass; as for the products,
 // both stations' bins of a pair on the same rows (band shift a multiple of
 // M1) and code widths of at most 16 bits.  Variant 0 is the four-step
@@ -1672,7 +1692,8 @@ static int64_t fused_param_span(const fxc_plan *p) {
 static bool phased_fused_possible(const fxc_plan *p) {
     const int64_t sb = p->desc.a2s - p->desc.a1s;
     const bool shape = p->fft_form == 2 || (p->fft_form == 0 && p->N == 16384);
-    return shape && p->desc.precision == FXC_PRECISION_CHOSEN && p->mf_b1 && (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) &&
+    return shape && (p->desc.precision == FXC_PRECISION_PLAIN_FP32 || p->mf_b1) &&
+           (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) &&
            (sb % 128) == 0 && p->st[0].bits <= 16 && p->st[1].bits <= 16;
 }
 
@@ -1681,13 +1702,32 @@ static bool phased_fused_ok(const fxc_plan *p) {
 }
 
 // Frame groups of the fused second pass: enough workgroups (M1 / 2 row
-// pairs x groups) for one resident round at the kernel's occupancy (five
-// workgroups per CU at M2 = 64, four at 128 and 256), at most the plan's
+// pairs x groups) for one resident round at the kernel's occupancy (chosen:
+// five workgroups per CU at M2 = 64, four at 128 and 256; plain: four, and
+// three at 256 and with the .raw output), at most the plan's
 // partial slots.
 static int large_fused_groups(const fxc_plan *p) {
-    const int per_cu = p->M2 == 64 ? 5 : 4;
+    const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) != 0;
+    const int per_cu = p->desc.precision == FXC_PRECISION_CHOSEN ? (p->M2 == 64 ? 5 : 4)
+                                                                 : (p->M2 == 256 || raw ? 3 : 4);
     return std::max(1, std::min(p->max_wg, num_cus() * per_cu / (p->M1 / 2)));
 }
+
+// The plain form takes the fused four-step from 512 frames on.  A sector of
+// few frames is one serial walk of the phase chains (N / 2 links), which the
+// rows of the general path take in 12.7 ns a link and the link-major table in
+// 16; the passes' gain over the general path grows with the frames, so the
+// line is a frame count whatever N (16 / 128 / 512 / 1024 frames at N = 16384:
+// 139 / 151 / 207 / 287 us general, 163 / 167 / 194 / 227 fused; 512 frames at
+// 32768: 428 and 367; 256 at 65536: 588 and 618, 2048: 2699 and 1523).
+constexpr int64_t kPlainFusedFrames = 512;
+static bool fused_for(const fxc_plan *p, int64_t nf) {
+    return p->desc.precision == FXC_PRECISION_CHOSEN || nf >= kPlainFusedFrames;
+}
+
+// Link-major chains: a link's row holds the span's frames and eight more (the
+// last iteration's reads), on an odd number of 64-byte lines.
+static int64_t chain_links_ld(int64_t frames) { return ((frames + 8 + 15) & ~(int64_t)15) | 8; }
 
 // Phased sum on the fused four-step: per chunk the phased parameters and
 // shifts, the fused first pass of both stations, the second pass with the
@@ -1704,8 +1744,16 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
     const int64_t bpf_o = plan_bpf_out(p);
     // the .raw second pass holds four waves per SIMD (the power-only one
     // five): one resident round of workgroups at that occupancy
-    const int ng = raw && p->M2 == 64 ? std::max(1, std::min(p->max_wg, num_cus() * 4 / (p->M1 / 2)))
-                                      : large_fused_groups(p);
+    const bool plain = p->desc.precision == FXC_PRECISION_PLAIN_FP32;
+    const int ng = raw && p->M2 == 64 && !plain ? std::max(1, std::min(p->max_wg, num_cus() * 4 / (p->M1 / 2)))
+                                                : large_fused_groups(p);
+    // plain: the rotation chains of whole chunks, link-major, one per frame
+    // where the delay model gives station 2 none (as enqueue_phased_wave)
+    const int nch = base.dly.table != nullptr ? 1 : 2;
+    const int64_t cspan = plain ? chain_span(nf, p->chunk_use, (size_t)nch * p->half * 8, (int)p->half) : 0;
+    const int64_t cld = chain_links_ld(std::min(cspan, nf));
+    if (plain) GROW(p, p->d_chain, (((size_t)p->half + 7) & ~(size_t)7) * nch * cld * 8, s, "phased rotation chains");
+    int64_t cspan0 = -1;
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
     if (raw) GROW(p, p->d_cb, (size_t)p->chunk_use * p->half * 8, s, "phased spectra");
     const int64_t span = fused_param_span(p);
@@ -1722,16 +1770,30 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
         if (span0 < 0 || c0 >= span0 + span) {
             SectorArgs pa = a;
             pa.nf = std::min(span, nf - c0);
-            HIP_TRY(launch_phased_params(pa, 1, p->d_params.p, (int64_t *)p->d_lshifts.p, s));
+            HIP_TRY(launch_phased_params(pa, plain ? 0 : 1, p->d_params.p, (int64_t *)p->d_lshifts.p, s));
             span0 = c0;
+        }
+        if (plain) {
+            a.chain_ld = (int)cld;
+            a.chains = nch;
+            if (cspan0 < 0 || c0 >= cspan0 + cspan) {
+                SectorArgs ca = a;
+                ca.nf = std::min(cspan, nf - c0);
+                HIP_TRY(launch_phase_chain_links(ca, CHAIN_PHASED, (float *)p->d_chain.p, s));
+                cspan0 = c0;
+            }
+            a.chain = (const float *)p->d_chain.p + 2 * (c0 - cspan0);
         }
         const uint8_t *pp = (const uint8_t *)p->d_params.p + (size_t)(c0 - span0) * phased_param_bytes();
         const int64_t *shifts = (const int64_t *)p->d_lshifts.p + 2 * (c0 - span0);
-        HIP_TRY(launch_large_pass1_fused(a, shifts, (float2 *)p->d_z[0].p, (float2 *)p->d_z[1].p,
-                                         p->M1, p->M2, (const float2 *)p->tw_lm.p, s));
-        HIP_TRY(launch_large_pass2_phased(a, (const float2 *)p->d_z[0].p, (const float2 *)p->d_z[1].p,
-                                          pp, p->M1, p->M2, twl2,
-                                          (const float2 *)p->tw_lm.p, raw, ng, c0 > 0 ? 1 : 0, s));
+        float2 *y1 = (float2 *)p->d_z[0].p, *y2 = (float2 *)p->d_z[1].p;
+        const float2 *twm = (const float2 *)p->tw_lm.p;
+        if (plain)
+            HIP_TRY(launch_large_pass1_f32(a, shifts, y1, y2, p->M1, p->M2, twm, (const float2 *)p->tw_ly.p, s));
+        else
+            HIP_TRY(launch_large_pass1_fused(a, shifts, y1, y2, p->M1, p->M2, twm, s));
+        HIP_TRY(launch_large_pass2_phased(a, y1, y2, pp, p->M1, p->M2, twl2, twm, raw, ng, c0 > 0 ? 1 : 0,
+                                          plain, s));
         if (raw && p->M2 != 64) {
             HIP_TRY(launch_irfft_rows_quantise(a, (const float2 *)p->d_cb.p, cn, p->M1, p->M2,
                                                (const float2 *)p->tw_l1.p, twl2, (const float2 *)p->tw_lm.p,
@@ -1750,10 +1812,17 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                 hipStream_t s) {
     const float2 *twl1 = (const float2 *)(p->M1 == 128 ? p->tw_l1.p : p->tw_l2.p);
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
-    if (large_fused_ok(p)) {
+    if (large_fused_ok(p) && fused_for(p, nf)) {
         const int ng = large_fused_groups(p);
         const int64_t span = fused_param_span(p);
         int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
+        const bool plain = p->desc.precision == FXC_PRECISION_PLAIN_FP32;
+        // plain XCF: the chains of whole chunks, link-major
+        const bool chain = xcf_uses_chain(p);
+        const int64_t cspan = chain ? chain_span(nf, p->chunk_use, (size_t)base.ov * 8, base.ov) : 0;
+        const int64_t cld = chain_links_ld(std::min(cspan, nf));
+        if (chain) GROW(p, p->d_chain, (size_t)((base.ov + 7) & ~7) * cld * 8, s, "phase chains");
+        int64_t cspan0 = -1;
         for (int64_t c0 = 0; c0 < nf; c0 += p->chunk_use) {
             const int64_t cn = std::min(p->chunk_use, nf - c0);
             SectorArgs a = base;
@@ -1769,13 +1838,26 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                             (int64_t *)p->d_lshifts.p, s));
                 span0 = c0;
             }
+            if (chain) {
+                a.chain_ld = (int)cld;
+                if (cspan0 < 0 || c0 >= cspan0 + cspan) {
+                    SectorArgs ca = a;
+                    ca.nf = std::min(cspan, nf - c0);
+                    HIP_TRY(launch_phase_chain_links(ca, CHAIN_XCF, (float *)p->d_chain.p, s));
+                    cspan0 = c0;
+                }
+                a.chain = (const float *)p->d_chain.p + 2 * (c0 - cspan0);
+            }
             const FrameParam *params = (const FrameParam *)((const uint8_t *)p->d_params.p +
                                                             (size_t)(c0 - span0) * frame_param_bytes());
             const int64_t *shifts = (const int64_t *)p->d_lshifts.p + 2 * (c0 - span0);
-            HIP_TRY(launch_large_pass1_fused(a, shifts, (float2 *)p->d_z[0].p, (float2 *)p->d_z[1].p,
-                                             p->M1, p->M2, (const float2 *)p->tw_lm.p, s));
-            HIP_TRY(launch_large_pass2_mac(a, (const float2 *)p->d_z[0].p, (const float2 *)p->d_z[1].p,
-                                           params, p->M1, p->M2, twl2, ng, c0 > 0 ? 1 : 0, s));
+            float2 *y1 = (float2 *)p->d_z[0].p, *y2 = (float2 *)p->d_z[1].p;
+            const float2 *twm = (const float2 *)p->tw_lm.p;
+            if (plain)
+                HIP_TRY(launch_large_pass1_f32(a, shifts, y1, y2, p->M1, p->M2, twm, (const float2 *)p->tw_ly.p, s));
+            else
+                HIP_TRY(launch_large_pass1_fused(a, shifts, y1, y2, p->M1, p->M2, twm, s));
+            HIP_TRY(launch_large_pass2_mac(a, y1, y2, params, p->M1, p->M2, twl2, ng, c0 > 0 ? 1 : 0, plain, s));
         }
         HIP_TRY(launch_reduce_pairs((const double *)p->part.p, ng, p->half, p->M1, p->M2, base.flags,
                                     d_acc, s));
@@ -1828,6 +1910,30 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
     return FXC_OK;
 }
 
+// Plan timing: the events around a sector's kernels (fxc_plan_get_timing)
+static fxc_status timing_begin(fxc_plan *p, hipStream_t s, std::pair<hipEvent_t, hipEvent_t> &ev) {
+    if (!p->timing) return FXC_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+        return fail(FXC_ERR_INVALID_ARG, "plan timing is not available inside a graph capture");
+    if (!p->pool.empty()) {
+        ev = p->pool.back();
+        p->pool.pop_back();
+    } else {
+        HIP_TRY(hipEventCreate(&ev.first));
+        HIP_TRY(hipEventCreate(&ev.second));
+    }
+    HIP_TRY(hipEventRecord(ev.first, s));
+    return FXC_OK;
+}
+
+static fxc_status timing_end(fxc_plan *p, hipStream_t s, const std::pair<hipEvent_t, hipEvent_t> &ev) {
+    if (!p->timing) return FXC_OK;
+    HIP_TRY(hipEventRecord(ev.second, s));
+    p->pending.push_back(ev);
+    return FXC_OK;
+}
+
 static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8_t *d_raw2,
                                  int64_t first_frame, int64_t nf, const fxc_delay_cfg &dc,
                                  double *d_acc, uint8_t *d_raw_out, hipStream_t s) {
@@ -1851,10 +1957,17 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     a.raw2 = d_raw2;
     a.first_frame = first_frame;
     a.nf = nf;
-    if (phased && phased_fused_ok(p)) return enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s);
+    if (phased && phased_fused_ok(p) && fused_for(p, nf))
+        return enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s);
     if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
-    if (p->fft_form == 2 || large_fused_ok(p)) return enqueue_large(p, a, nf, d_acc, s);
+    if (p->fft_form == 2 || (large_fused_ok(p) && p->desc.precision == FXC_PRECISION_CHOSEN))
+        return enqueue_large(p, a, nf, d_acc, s);
+    if (large_fused_ok(p) && fused_for(p, nf)) {   // plain N = 16384: timed as on the Stockham kernel
+        std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
+        if ((st = timing_begin(p, s, ev)) != FXC_OK || (st = enqueue_large(p, a, nf, d_acc, s)) != FXC_OK) return st;
+        return timing_end(p, s, ev);
+    }
     const bool wave = wave_for(p, nf);
     const int wg_cap = std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div);
     // Plain XCF over more than kChainMinOverlap bins: slabs of frames whose
@@ -1876,19 +1989,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     a.frames_per_wg = fpw;
     a.part = (double *)p->part.p;
     std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
-    if (p->timing) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (s && hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
-            return fail(FXC_ERR_INVALID_ARG, "plan timing is not available inside a graph capture");
-        if (!p->pool.empty()) {
-            ev = p->pool.back();
-            p->pool.pop_back();
-        } else {
-            HIP_TRY(hipEventCreate(&ev.first));
-            HIP_TRY(hipEventCreate(&ev.second));
-        }
-        HIP_TRY(hipEventRecord(ev.first, s));
-    }
+    if ((st = timing_begin(p, s, ev)) != FXC_OK) return st;
     for (int64_t c0 = 0; c0 < nf; c0 += slab) {
         const int64_t cn = std::min(slab, nf - c0);
         SectorArgs b = a;
@@ -1911,10 +2012,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         else if (wave) HIP_TRY(launch_sector_wave(b, p->desc.precision, wgs, s));
         else HIP_TRY(launch_sector(b, p->desc.precision, wgs, s));
     }
-    if (p->timing) {
-        HIP_TRY(hipEventRecord(ev.second, s));
-        p->pending.push_back(ev);
-    }
+    if ((st = timing_end(p, s, ev)) != FXC_OK) return st;
     HIP_TRY(launch_reduce((const double *)p->part.p, n_wg, p->half, a.flags, d_acc, s));
     return FXC_OK;
 }

@@ -42,17 +42,11 @@ __device__ __forceinline__ float chain_next(float v, float qx, float c) {
     return own + cross;
 }
 
-__global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, float *out) {
-    const int nch = kind == CHAIN_XCF ? 1 : a.chains;
-    const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
-    const int64_t i = (int64_t)blockIdx.x * (blockDim.x / 2) + (threadIdx.x >> 1);   // chain
-    const bool im = threadIdx.x & 1;
-    if (i >= a.nf * nch) return;   // both lanes of a pair together
-    const int64_t f = i / nch;
-    const int s = (int)(i - f * nch);
+// Link 0 and the step of a frame's chain (phased: station s's)
+__device__ __forceinline__ void chain_start(const SectorArgs &a, int kind, int64_t frame, int s, float2 &p,
+                                            float2 &step) {
     FrameDelayDev d;
-    compute_frame_delay(a.first_frame + f, a.dly, d, nullptr, nullptr);
-    float2 p, step;
+    compute_frame_delay(frame, a.dly, d, nullptr, nullptr);
     {
 #pragma clang fp contract(off)
         if (kind == CHAIN_XCF) {
@@ -68,6 +62,18 @@ __global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, floa
             step = polar1_f32((float)phase_step);
         }
     }
+}
+
+__global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, float *out) {
+    const int nch = kind == CHAIN_XCF ? 1 : a.chains;
+    const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
+    const int64_t i = (int64_t)blockIdx.x * (blockDim.x / 2) + (threadIdx.x >> 1);   // chain
+    const bool im = threadIdx.x & 1;
+    if (i >= a.nf * nch) return;   // both lanes of a pair together
+    const int64_t f = i / nch;
+    const int s = (int)(i - f * nch);
+    float2 p, step;
+    chain_start(a, kind, a.first_frame + f, s, p, step);
     // this part's row: a.chain_ld floats (a multiple of 16, >= len)
     float4 *o = reinterpret_cast<float4 *>(out + (2 * i + (im ? 1 : 0)) * (int64_t)a.chain_ld);
     const float qx = step.x, c = im ? step.y : -step.y;
@@ -84,6 +90,47 @@ __global__ __launch_bounds__(64) void k_phase_chain(SectorArgs a, int kind, floa
             v = chain_next(r.w, qx, c);
         }
     }
+}
+
+typedef __attribute__((address_space(1))) float global_float;
+typedef __attribute__((address_space(1))) char global_char;
+
+// The chains link-major (link k of frame f's chain c at (((k chains + c) ld +
+// f) 2 + im), ld = a.chain_ld >= the frames, links up to a multiple of 8): for
+// the second pass of the four-step, whose threads own a bin and walk the
+// frames.  A block's 32 frames store 256 contiguous bytes per link; 16 ns a
+// link against the rows' 12.7 (the store and its scalar address).  grid.y: the chain.
+__global__ __launch_bounds__(64) void k_phase_chain_links(SectorArgs a, int kind, float *out) {
+    const int64_t f = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 1);
+    const bool im = threadIdx.x & 1;
+    if (f >= a.nf) return;   // both lanes of a pair together
+    const int len = kind == CHAIN_XCF ? a.ov : a.M + 1;
+    const int ch = (int)blockIdx.y;
+    float2 p, step;
+    chain_start(a, kind, a.first_frame + f, ch, p, step);
+    const float qx = step.x, c = im ? step.y : -step.y;
+    float v = im ? p.y : p.x;
+    // a uniform row pointer and the lane's offset: the walk's only vector work is the link
+    global_float *o = (global_float *)(out + 2 * (ch * (int64_t)a.chain_ld + (int64_t)blockIdx.x * 32));
+    const int64_t ld = 2 * (int64_t)gridDim.y * a.chain_ld;
+    unsigned off = threadIdx.x * 4u;
+    for (int k = 0; k < len; k += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u, o += ld) {
+            asm volatile("" : "+s"(o), "+v"(off));   // stay a scalar pair and a 32-bit offset
+            *(global_float *)((global_char *)o + off) = v;
+            v = chain_next(v, qx, c);
+        }
+    }
+}
+
+hipError_t launch_phase_chain_links(const SectorArgs &a, int kind, float *out, hipStream_t s) {
+    if (kind == CHAIN_PHASED && a.chains != 1 && a.chains != 2) return hipErrorInvalidValue;
+    if (a.nf <= 0) return hipSuccess;
+    if (a.chain_ld < a.nf) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((a.nf + 31) / 32), kind == CHAIN_XCF ? 1u : (unsigned)a.chains);
+    hipLaunchKernelGGL(k_phase_chain_links, grid, dim3(64), 0, s, a, kind, out);
+    return hipGetLastError();
 }
 
 hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t s) {

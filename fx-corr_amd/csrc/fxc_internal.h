@@ -223,6 +223,9 @@ hipError_t launch_scale_add_xcf(double *ac, const double *re, const double *im, 
 // fxc_chain.hip: frames [0, a.nf) of the launch, rows of 2 a.chain_ld
 // floats, real parts then imaginary parts (one XCF chain of a.ov bins, or two phased
 // chains of M+1 bins, per frame).
+// the same chains link-major: link k of frame f's chain c at
+// (((k chains + c) a.chain_ld + f) 2), links up to a multiple of 8
+hipError_t launch_phase_chain_links(const SectorArgs &a, int kind, float *out, hipStream_t stream);
 hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t stream);
 
 // fxc_large.hip: N = 32768, 65536 through HBM scratch (four-step M = M1 x M2)
@@ -279,11 +282,15 @@ hipError_t launch_rfft_mfma(const SectorArgs &a, const float *in, int64_t nframe
 hipError_t launch_large_pass1_fused(const SectorArgs &a, const int64_t *shifts, float2 *out0,
                                     float2 *out1, int M1, int M2, const float2 *tw_m,
                                     hipStream_t s);
+// plain: the same first pass in FP32 (fxc_large.hip); tw_y: W_M^{m2 k1} at
+// [k1][m2]
+hipError_t launch_large_pass1_f32(const SectorArgs &a, const int64_t *shifts, float2 *out0, float2 *out1,
+                                  int M1, int M2, const float2 *tw_m, const float2 *tw_y, hipStream_t s);
 hipError_t launch_reduce_pairs(const double *part, int n_wg, int half, int M1, int M2, int flags,
                                double *out, hipStream_t stream);
 hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                   const FrameParam *params, int M1, int M2, const float2 *tw_m2,
-                                  int n_groups, int accumulate, hipStream_t s);
+                                  int n_groups, int accumulate, bool plain, hipStream_t s);
 // the phased sum on the fused second pass; pp: the chunk's phased parameters
 // (launch_phased_params).  raw, M2 = 64 (N = 16384): also the first half of
 // the inverse FFT into a.cb_out (M per frame), finished by
@@ -292,7 +299,7 @@ hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const f
 hipError_t launch_large_pass2_phased(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                      const void *pp, int M1, int M2, const float2 *tw_m2,
                                      const float2 *tw_m, bool raw, int n_groups, int accumulate,
-                                     hipStream_t s);
+                                     bool plain, hipStream_t s);
 hipError_t launch_irfft_cols_quantise(const SectorArgs &a, const float2 *in, int64_t nframes,
                                       uint8_t *out, bool negate_odd, const float2 *tw_m,
                                       hipStream_t s);

@@ -313,6 +313,124 @@ __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// ------------------------------------ FP32 first pass fused with the decode
+// The plain form's first pass of the fused four-step (M1 = 128): workgroup
+// (frame, part p) takes the columns m2 in [64 p, 64 p + 64) of all 128 rows
+// m1 (element m = m2 + M2 m1).  The rows' packed words are staged in LDS as
+// k_large_pass1_fused does; thread (column n, j) decodes inputs m1 = j + 8 r,
+// takes the DFT-16 over r (index e) times W_128^{j e}, and after an LDS
+// transpose (over the words) the DFT-8 over j for e = 2 j and 2 j + 1, giving
+// k1 = e + 16 b; the output twiddle W_M^{m2 k1} comes from a table in store
+// order.  Against the decode kernel and the LDS Stockham pass it replaces
+// (FP32 samples to memory and back, then the columns), 2^27 samples of both
+// stations at N = 32768: 311 + 690 us to 424.
+template <int BITS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_large_pass1_f32(
+    SectorArgs a, int station, const int64_t *shifts, float2 *out, int M2, int parts,
+    const float2 *tw_m, const float2 *tw_y) {
+    __shared__ float2 zb[128 * 64];
+    __shared__ float2 w128[128];
+    __shared__ float lev[256];
+    uint32_t *words = reinterpret_cast<uint32_t *>(zb);   // 128 rows x K words, one zero word after them
+    const StationDev &st = a.st[station];
+    const int bits = BITS ? BITS : st.bits;
+    const int K = 4 * bits + 1, rw = M2 * bits / 16;      // 128 K + 1 <= 8321 words (16 bits)
+    const int M = a.M;
+    const int tid = threadIdx.x;
+    const int n = tid & 63;
+    const int jw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // a contiguous run of (frame, part) per XCD, as k_large_pass1_fused
+    const int nb = (int)gridDim.x, xcd = (int)blockIdx.x & 7, kb = (int)blockIdx.x >> 3;
+    const int lb = xcd * (nb >> 3) + min(xcd, nb & 7) + kb;
+    const int64_t f = lb / parts;
+    const int part = lb % parts;
+    if (f >= a.nf) return;   // uniform per workgroup
+    if (tid < 128) w128[tid] = tw_m[tid * M2];
+    if (st.bits >= 2 && st.bits <= 8 && tid >= 256)
+        lev[tid - 256] = (tid - 256 <= (int)st.code_mask) ? st.levels[tid - 256] : 0.0f;
+    const int sh = clamp_shift(shifts[f * 2 + station], a.N);
+    const int base0 = ((128 * part - sh) * bits) >> 5;   // arithmetic shift: floor
+    {
+        const uint8_t *frame = (station == 0 ? a.raw1 : a.raw2) + f * st.bpf;
+        const int nst = 128 * K;
+        for (int i0 = 0; i0 < nst; i0 += 512 * 4) {   // four loads in flight per thread
+            uint32_t v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int idx = i0 + tid + 512 * u;
+                const int m1 = idx / K;
+                v[u] = idx < nst ? frame_word(frame, st, m1 * rw + base0 + (idx - m1 * K)) : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int idx = i0 + tid + 512 * u;
+                if (idx < nst) words[idx] = v[u];
+            }
+        }
+        if (tid == 0) words[nst] = 0u;
+    }
+    __syncthreads();
+    // LSB flip (odd samples of the unshifted frame): sample 2m - sh is odd iff sh is
+    const uint32_t fm0 = (st.lsb && (sh & 1)) ? 0x80000000u : 0u;
+    const uint32_t fm1 = (st.lsb && !(sh & 1)) ? 0x80000000u : 0u;
+    const int m2 = 64 * part + n;
+    float2 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int m1 = jw + 8 * r;
+        const int src0 = 2 * (m2 + M2 * m1) - sh;
+        const int bp = src0 * bits;
+        v[r] = decode_pair_local<BITS>(words, st, lev, src0, (bp >> 5) - base0 + m1 * (K - rw),
+                                       (uint32_t)bp & 31u, a.N, fm0, fm1);
+    }
+    dft16(v);
+#pragma unroll
+    for (int e = 1; e < 16; ++e) v[e] = c_mul(v[e], w128[jw * e]);
+    float2 ty[2][8];   // output twiddles, loaded across the barriers
+    const float2 *ty0 = tw_y + m2;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int b = 0; b < 8; ++b) ty[h][b] = ty0[(2 * jw + h + 16 * b) * M2];
+    __syncthreads();   // every thread is done with the words
+#pragma unroll
+    for (int e = 0; e < 16; ++e) zb[(e * 8 + jw) * 64 + n] = v[e];
+    __syncthreads();
+    float2 *dst = out + f * (int64_t)M + m2;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int e = 2 * jw + h;
+        float2 u[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) u[q] = zb[(e * 8 + q) * 64 + n];
+        dftR<8>(u);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) dst[(e + 16 * b) * M2] = c_mul(u[b], ty[h][b]);
+    }
+}
+
+hipError_t launch_large_pass1_f32(const SectorArgs &a, const int64_t *shifts, float2 *out0, float2 *out1,
+                                  int M1, int M2, const float2 *tw_m, const float2 *tw_y, hipStream_t s) {
+    if (tw_y == nullptr || M1 != 128 || (M2 != 64 && M2 != 128 && M2 != 256) || M1 * M2 != a.M)
+        return hipErrorInvalidValue;
+    if (a.nf <= 0) return hipSuccess;
+    const int parts = M2 / 64;
+    for (int st = 0; st < 2; ++st) {
+        const int bits = a.st[st].bits;
+        if (bits < 1 || bits > 16) return hipErrorInvalidValue;
+        auto kern = bits == 1   ? k_large_pass1_f32<1>
+                    : bits == 2 ? k_large_pass1_f32<2>
+                    : bits == 4 ? k_large_pass1_f32<4>
+                    : bits == 8 ? k_large_pass1_f32<8>
+                                : k_large_pass1_f32<0>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)(a.nf * parts)), dim3(512), 0, s, a, st, shifts,
+                           st == 0 ? out0 : out1, M2, parts, tw_m, tw_y);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // ------------------------------------ second pass fused with the products
 // Chosen form, both stations' bins on the same rows of the four-step (the
 // band shift a multiple of M1).  Z[k1 + M1 k2] is row k1's DFT over m2 of
@@ -355,14 +473,43 @@ __device__ __forceinline__ void store_pair_sums(double *out, int half, int g, co
     }
 }
 
+// The plain form's phase chains for the second pass: link kk of the frames
+// of the span side by side (a.chain_ld per link), so that a thread, which
+// owns a bin and walks the frames, reads its frames' links as one run.  (Rows
+// of one frame's links, k_phase_chain's, would have each lane read 4 bytes of
+// its own line, M1 links apart, twice a frame.)  M2 = 64 / 128 take them two
+// frames at a time, the next two on their way; all eight in registers spill.
+__device__ __forceinline__ const float2 *chain_link(const SectorArgs &a, int kk, int64_t f) {
+    return reinterpret_cast<const float2 *>(a.chain) + (int64_t)kk * a.chain_ld + f;
+}
+template <int F>
+struct ChainLinks {
+    float2 v[F];
+    __device__ __forceinline__ void load(const float2 *p) {   // F frames (the row's padding included)
+#pragma unroll
+        for (int i = 0; i < F; ++i) v[i] = p[i];
+    }
+    // phased: rotations of station st's bin; a station without a chain
+    // (a.chains = 1, the second) is not rotated
+    __device__ __forceinline__ void load_rot(const SectorArgs &a, int bin, int st, int64_t f) {
+        if (st < a.chains) load(chain_link(a, bin * a.chains + st, f));
+        else
+#pragma unroll
+            for (int i = 0; i < F; ++i) v[i] = make_float2(1.f, 0.f);
+    }
+};
+
 // One bin of a row pair for the second pass: bin g = row + M1 k2
 // of row ra (rb_sel false) or rb, or bin M (nyq: row 0, k2 = M2); the
 // untangle of both stations and the ACF/XCF products (k_mac_large's arithmetic).
-template <int M2, int LP>
+// PLAIN: the reference's own f32 phase, chv (a link of the frame's chain),
+// after the fringe phasor frmix.
+template <int M2, int LP, bool PLAIN>
 __device__ __forceinline__ void row_bin(const float2 (*zb)[LP], const float2 (*twp)[M2], bool rb_sel,
                                         int k2, bool nyq, int M, int M1, int ra, int rb, int gs, int ov,
                                         int sbo, int jo, int grid, bool do_acf, bool do_xcf,
-                                        bool ov_only, double dth, double phw, double (&acc)[4]) {
+                                        bool ov_only, double dth, double phw, float2 frmix, float2 chv,
+                                        double (&acc)[4]) {
     const int row = nyq ? 0 : (rb_sel ? rb : ra);
     if (nyq) k2 = M2;
     const int g = nyq ? M : row + M1 * k2;
@@ -387,11 +534,16 @@ __device__ __forceinline__ void row_bin(const float2 (*zb)[LP], const float2 (*t
         acc[1] += (double)(grid == 0 ? poth : pgrid);
     }
     if (in_ov && do_xcf) {
-        const float r = (float)wrap_turns(fma((double)(g - gs), dth, phw));
-        const float2 phf = make_float2(__builtin_amdgcn_cosf(r), __builtin_amdgcn_sinf(r));
+        float2 phf = chv;
+        if constexpr (!PLAIN) {
+            const float r = (float)wrap_turns(fma((double)(g - gs), dth, phw));
+            phf = make_float2(__builtin_amdgcn_cosf(r), __builtin_amdgcn_sinf(r));
+        }
         const float2 X1 = (grid == 0) ? Xg : Xo;
         const float2 X2 = (grid == 0) ? Xo : Xg;
-        const float2 v2 = c_mul(c_mul(X1, c_conj(X2)), phf);
+        float2 v2 = c_mul(X1, c_conj(X2));
+        if constexpr (PLAIN) v2 = c_mul(v2, frmix);
+        v2 = c_mul(v2, phf);
         acc[2] += (double)v2.x;
         acc[3] += (double)v2.y;
     }
@@ -401,12 +553,13 @@ __device__ __forceinline__ void row_bin(const float2 (*zb)[LP], const float2 (*t
 // arithmetic, main.rs:2264-2302): both stations' untangled bins, each
 // rotated by exp(2 pi i b th) from the FP64 phase and by its fringe phasor,
 // cb = w1 c1 + w2 c2, |cb|^2 into the FP64 sum.  Returns cb as the inverse
-// FFT takes it (DC and Nyquist imaginary parts zeroed).
-template <int M2, int LP>
+// FFT takes it (DC and Nyquist imaginary parts zeroed).  PLAIN: rotated by
+// the reference's own f32 values rg (this bin) and ro (the other station's).
+template <int M2, int LP, bool PLAIN>
 __device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float2 (*twp)[M2], bool rb_sel,
                                              int k2, bool nyq, int M, int M1, int ra, int rb, int gs,
                                              int ov, int sbo, int jo, int grid, const PhasedParam &P,
-                                             float w1, float w2, double &acc) {
+                                             float w1, float w2, float2 rg, float2 ro, double &acc) {
     const int row = nyq ? 0 : (rb_sel ? rb : ra);
     if (nyq) k2 = M2;
     const int g = nyq ? M : row + M1 * k2;
@@ -418,7 +571,7 @@ __device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float
     const bool in_ov = g >= gs && g < gs + ov;
     const double thg = grid == 0 ? P.th1 : P.th2, tho = grid == 0 ? P.th2 : P.th1;
     const float2 frg = grid == 0 ? P.fr1 : P.fr2, fro = grid == 0 ? P.fr2 : P.fr1;
-    float2 sg = c_mul(Xg, phasor_turns((double)g * thg));
+    float2 sg = c_mul(Xg, PLAIN ? rg : phasor_turns((double)g * thg));
     if (g == M) sg.y = 0.0f;                              // Nyquist (utils.rs:118-123)
     const float2 cg = c_mul(sg, frg);
     float2 co = make_float2(0.0f, 0.0f);
@@ -427,7 +580,8 @@ __device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float
         const int khm = row == 0 ? (M2 - kh) & (M2 - 1) : M2 - 1 - kh;
         const float2 Oh = zb[2 + bg][pad(kh & (M2 - 1))];
         const float2 Om = zb[2 + bm][pad(khm & (M2 - 1))];
-        float2 so = c_mul(untangle_ab(Oh, Om, h, M, twp[bg][kh & (M2 - 1)]), phasor_turns((double)h * tho));
+        float2 so = c_mul(untangle_ab(Oh, Om, h, M, twp[bg][kh & (M2 - 1)]),
+                          PLAIN ? ro : phasor_turns((double)h * tho));
         if (h == M) so.y = 0.0f;
         co = c_mul(so, fro);
     }
@@ -443,6 +597,20 @@ __device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float
     return cb;
 }
 
+// Bin M's phased bin (pair 0's first threads), its rotations read here
+template <int M2, int LP, bool PLAIN>
+__device__ __forceinline__ float2 nyq_bin_ph(const SectorArgs &a, const float2 (*zb)[LP], const float2 (*twp)[M2],
+                                             int M1, int ra, int rb, int gs, int sbo, int jo,
+                                             const PhasedParam &P, float w1, float w2, int64_t f, double &acc) {
+    ChainLinks<1> rg = {}, ro = {};
+    if constexpr (PLAIN) {
+        rg.load_rot(a, a.M, a.grid, f);
+        if (a.M >= gs && a.M < gs + a.ov) ro.load_rot(a, a.M + sbo, 1 - a.grid, f);
+    }
+    return row_bin_ph<M2, LP, PLAIN>(zb, twp, false, 0, true, a.M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid, P, w1, w2,
+                                     rg.v[0], ro.v[0], acc);
+}
+
 // The same second pass at M2 = 256 with two radix-16 passes per row: each
 // wave transforms one frame's four rows (lane = 16 q + j: row q, butterfly
 // j) -- the first pass from registers, its outputs multiplied by the second
@@ -452,8 +620,8 @@ __device__ __forceinline__ float2 row_bin_ph(const float2 (*zb)[LP], const float
 // frees the rows.  The twiddles are read from LDS, which leaves registers
 // (and, with rows of 271 entries, LDS) for four workgroups per CU instead of
 // three: 2^27 samples 703 -> 683 us.
-template <int MODE>
-__global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const float2 *y1,
+template <int MODE, bool PLAIN>
+__global__ __launch_bounds__(256, PLAIN ? 3 : 4) void k_large_pass2_r16(SectorArgs a, const float2 *y1,
                                                          const float2 *y2, const void *params, int M1, const float2 *tw_m2, int64_t fpg,
                                                          int accumulate) {
     constexpr int M2 = 256, LP = 271;   // pad(255) + 1
@@ -497,6 +665,12 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const 
         for (int r = 0; r < 16; ++r)
             cur[r] = f < g1 ? src_row[f * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
     }
+    bool in_ov[2];   // the thread's bins (rows ra / rb) lie in the overlap
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int kk = (i ? rb : ra) + M1 * tid - gs;
+        in_ov[i] = kk >= 0 && kk < a.ov;
+    }
     __syncthreads();   // twiddles staged
     float2 *z = zr[w][q];
     for (int64_t it = g0; it < g1; it += 4) {
@@ -505,6 +679,17 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const 
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 16 * r] : make_float2(0.f, 0.f);
+        ChainLinks<PLAIN ? 4 : 1> cg[2] = {}, co[2] = {};
+#pragma unroll
+        for (int i = 0; PLAIN && i < 2; ++i) {
+            const int g = (i ? rb : ra) + M1 * tid;
+            if constexpr (MODE == P2_PRODUCTS) {
+                if (do_xcf && in_ov[i]) cg[i].load(chain_link(a, g - gs, it));
+            } else {
+                cg[i].load_rot(a, g, a.grid, it);
+                if (in_ov[i]) co[i].load_rot(a, g + sbo, 1 - a.grid, it);
+            }
+        }
         if (f < g1) {
             dft16(cur);                                  // pass 1: inputs j + 16 r
 #pragma unroll
@@ -521,32 +706,44 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const 
         }
         __syncthreads();   // the iteration's rows are ready
         const int nfr = (int)((g1 - it) < 4 ? (g1 - it) : 4);
-        for (int s2 = 0; s2 < nfr; ++s2) {
+        auto bins = [&](int s2) {
             if constexpr (MODE != P2_PRODUCTS) {
                 const PhasedParam P = static_cast<const PhasedParam *>(params)[it + s2];
                 float2 *cbo = MODE == P2_PHASED_CB ? a.cb_out + (it + s2) * half : nullptr;
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov,
-                                                         sbo, jo, a.grid, P, w1, w2, acc[i][0]);
+                    const float2 cb = row_bin_ph<M2, LP, PLAIN>(
+                        zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid, P, w1, w2,
+                        cg[i].v[PLAIN ? s2 : 0], co[i].v[PLAIN ? s2 : 0], acc[i][0]);
                     if constexpr (MODE == P2_PHASED_CB) cbo[(i ? rb : ra) * M2 + tid] = cb;
                 }
                 if (nyq) {
-                    const float2 cn = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov,
-                                                         sbo, jo, a.grid, P, w1, w2, acc[2][0]);
+                    const float2 cn = nyq_bin_ph<M2, LP, PLAIN>(a, zr[s2], twp, M1, ra, rb, gs, sbo, jo, P, w1, w2,
+                                                                it + s2, acc[2][0]);
                     if constexpr (MODE == P2_PHASED_CB) cbo[M] = cn;
                 }
             } else {
                 const FrameParam &F = static_cast<const FrameParam *>(params)[it + s2];
-                const double dth = F.dth, phw = F.phw;
+                const double dth = PLAIN ? 0.0 : F.dth, phw = PLAIN ? 0.0 : F.phw;
+                const float2 frmix = PLAIN ? F.frmix : make_float2(0.f, 0.f);
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    row_bin<M2, LP>(zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                                    do_acf, do_xcf, ov_only, dth, phw, acc[i]);
-                if (nyq)
-                    row_bin<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                                    do_acf, do_xcf, ov_only, dth, phw, acc[2]);
+                    row_bin<M2, LP, PLAIN>(zr[s2], twp, i == 1, tid, false, M, M1, ra, rb, gs, a.ov, sbo, jo,
+                                           a.grid, do_acf, do_xcf, ov_only, dth, phw, frmix, cg[i].v[PLAIN ? s2 : 0], acc[i]);
+                if (nyq) {
+                    const bool cn = PLAIN && do_xcf && M >= gs && M - gs < a.ov;
+                    row_bin<M2, LP, PLAIN>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo,
+                                           a.grid, do_acf, do_xcf, ov_only, dth, phw, frmix,
+                                           cn ? *chain_link(a, M - gs, it + s2) : make_float2(0.f, 0.f), acc[2]);
+                }
             }
+        };
+        if constexpr (PLAIN) {   // the frames' links in registers
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2)
+                if (s2 < nfr) bins(s2);
+        } else {
+            for (int s2 = 0; s2 < nfr; ++s2) bins(s2);
         }
         __syncthreads();   // every thread is done with the rows
 #pragma unroll
@@ -584,12 +781,13 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r16(SectorArgs a, const 
 // here 48 and 53.  M2 = 128 keeps the twiddles in LDS: in registers they
 // spill at four waves per SIMD (746 us for 2^27 samples against 699; 735
 // with three waves and no spill).
-template <int M2, int MODE>
-__global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
+template <int M2, int MODE, bool PLAIN>
+__global__ __launch_bounds__(256, PLAIN ? (MODE == P2_PRODUCTS ? 4 : 3) : M2 == 64 ? 5 : 4) void k_large_pass2_r8(
     SectorArgs a, const float2 *y1, const float2 *y2, const void *params, int M1, const float2 *tw_m2,
     int64_t fpg, int accumulate) {
     constexpr int E = M2 / 8, LP = M2 + M2 / 16 + 2;
     constexpr int FS = 128 / M2;                        // threads per bin
+    constexpr int FT = 8 / FS;                          // frames per thread and iteration
     constexpr int NA = MODE == P2_PRODUCTS ? 4 : 1;
     __shared__ float2 zr[8][4][LP];   // [frame of the iteration][grid ra, grid rb, other ra, other rb]
     __shared__ float2 twp[2][M2];     // tw_post[row + M1 k2], rows ra / rb
@@ -630,6 +828,16 @@ __global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
     double acc[NA], nacc[NA];
 #pragma unroll
     for (int c = 0; c < NA; ++c) acc[c] = nacc[c] = 0.0;
+    const int kk = (rb_sel ? rb : ra) + M1 * k2 - gs;   // overlap index of this thread's bin
+    const bool in_ov = kk >= 0 && kk < a.ov;
+    auto links = [&](ChainLinks<2> &cg, ChainLinks<2> &co, int64_t f) {   // plain: this bin's, frames f, f + 1
+        if constexpr (MODE == P2_PRODUCTS) {
+            if (do_xcf && in_ov) cg.load(chain_link(a, kk, f));
+        } else {
+            cg.load_rot(a, kk + gs, a.grid, f);
+            if (in_ov) co.load_rot(a, kk + gs + sbo, 1 - a.grid, f);
+        }
+    };
     const int slot = 2 * w + fw;   // this lane's frame of the iteration
     float2 cur[E];
     {
@@ -646,6 +854,8 @@ __global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
 #pragma unroll
         for (int r = 0; r < E; ++r)
             nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
+        ChainLinks<2> cg = {}, co = {};   // plain: the first pair's links, loaded behind the rows' transforms
+        if constexpr (PLAIN) links(cg, co, it + fsel * FT);
         if (f < g1) {
             dftR<E>(cur);                                // pass 1: inputs j + 8 r
 #pragma unroll
@@ -668,27 +878,41 @@ __global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
         }
         __syncthreads();   // the iteration's rows are ready
         const int nfr = (int)((g1 - it) < 8 ? (g1 - it) : 8);
-        for (int s2 = fsel; s2 < nfr; s2 += FS) {
+        auto bins = [&](int s2, float2 chv, float2 cho) {
             if constexpr (MODE == P2_PRODUCTS) {
                 const FrameParam &F = static_cast<const FrameParam *>(params)[it + s2];
-                const double dth = F.dth, phw = F.phw;
-                row_bin<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                                do_acf, do_xcf, ov_only, dth, phw, acc);
-                if (nyq)
-                    row_bin<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo, a.grid,
-                                    do_acf, do_xcf, ov_only, dth, phw, nacc);
+                const double dth = PLAIN ? 0.0 : F.dth, phw = PLAIN ? 0.0 : F.phw;
+                const float2 frmix = PLAIN ? F.frmix : make_float2(0.f, 0.f);
+                row_bin<M2, LP, PLAIN>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov, sbo, jo,
+                                       a.grid, do_acf, do_xcf, ov_only, dth, phw, frmix, chv, acc);
+                if (nyq) {
+                    const bool cn = PLAIN && do_xcf && M >= gs && M - gs < a.ov;
+                    row_bin<M2, LP, PLAIN>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo,
+                                           a.grid, do_acf, do_xcf, ov_only, dth, phw, frmix,
+                                           cn ? *chain_link(a, M - gs, it + s2) : make_float2(0.f, 0.f), nacc);
+                }
             } else {
                 const PhasedParam P = static_cast<const PhasedParam *>(params)[it + s2];
                 float2 *cbo = MODE == P2_PHASED_CB ? a.cb_out + (it + s2) * half : nullptr;
-                const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov,
-                                                     sbo, jo, a.grid, P, w1, w2, acc[0]);
+                const float2 cb = row_bin_ph<M2, LP, PLAIN>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs,
+                                                            a.ov, sbo, jo, a.grid, P, w1, w2, chv, cho, acc[0]);
                 if constexpr (MODE == P2_PHASED_CB) cbo[(rb_sel ? rb : ra) * M2 + k2] = cb;
                 if (nyq) {
-                    const float2 cn = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov,
-                                                         sbo, jo, a.grid, P, w1, w2, nacc[0]);
+                    const float2 cn = nyq_bin_ph<M2, LP, PLAIN>(a, zr[s2], twp, M1, ra, rb, gs, sbo, jo, P, w1, w2,
+                                                                it + s2, nacc[0]);
                     if constexpr (MODE == P2_PHASED_CB) cbo[M] = cn;
                 }
             }
+        };
+        if constexpr (PLAIN) {   // consecutive frames, their links in pairs, the next pair on its way
+            for (int i = 0; i < FT && fsel * FT + i < nfr; i += 2) {
+                const ChainLinks<2> ng = cg, no = co;
+                if (i + 2 < FT) links(cg, co, it + fsel * FT + i + 2);
+                bins(fsel * FT + i, ng.v[0], no.v[0]);
+                if (fsel * FT + i + 1 < nfr) bins(fsel * FT + i + 1, ng.v[1], no.v[1]);
+            }
+        } else {
+            for (int s2 = fsel; s2 < nfr; s2 += FS) bins(s2, make_float2(0.f, 0.f), make_float2(0.f, 0.f));
         }
         __syncthreads();   // every thread is done with the rows
 #pragma unroll
@@ -729,7 +953,8 @@ __global__ __launch_bounds__(256, M2 == 64 ? 5 : 4) void k_large_pass2_r8(
 // the wave's own row buffers as scratch), times W_M^{n2 k1}, stored as row
 // k1 of the frame's 128 x 64 block in a.cb_out (M entries per frame).
 // k_irfft_cols_quantise finishes the transform over k1 and quantises.
-__global__ __launch_bounds__(256, 4) void k_large_pass2_r8_ph(SectorArgs a, const float2 *y1,
+template <bool PLAIN>
+__global__ __launch_bounds__(256, PLAIN ? 3 : 4) void k_large_pass2_r8_ph(SectorArgs a, const float2 *y1,
                                                            const float2 *y2, const PhasedParam *pp,
                                                            int M1, const float2 *tw_m2,
                                                            const float2 *tw_m, int64_t fpg,
@@ -788,6 +1013,12 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r8_ph(SectorArgs a, cons
 #pragma unroll
         for (int r = 0; r < 8; ++r)
             nxt[r] = fn < g1 ? src_row[fn * (int64_t)M + 8 * r] : make_float2(0.f, 0.f);
+        ChainLinks<PLAIN ? 4 : 1> cg = {}, co = {};   // this thread's frames it + 4 fsel ..
+        if constexpr (PLAIN) {
+            const int g = (rb_sel ? rb : ra) + M1 * k2;
+            cg.load_rot(a, g, a.grid, it + 4 * fsel);
+            if (g >= gs && g < gs + a.ov) co.load_rot(a, g + sbo, 1 - a.grid, it + 4 * fsel);
+        }
         if (f < g1) {
             dftR<8>(cur);                                // pass 1: inputs j + 8 r
 #pragma unroll
@@ -804,14 +1035,19 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r8_ph(SectorArgs a, cons
         }
         __syncthreads();   // the iteration's rows are ready
         const int nfr = (int)((g1 - it) < 8 ? (g1 - it) : 8);
-        for (int s2 = fsel; s2 < nfr; s2 += 2) {
+        auto bins = [&](int s2, float2 rg, float2 ro) {
             const PhasedParam P = pp[it + s2];
-            const float2 cb = row_bin_ph<M2, LP>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov,
-                                                 sbo, jo, a.grid, P, w1, w2, acc);
-            cbl[s2][rb_sel][k2] = cb;
+            cbl[s2][rb_sel][k2] = row_bin_ph<M2, LP, PLAIN>(zr[s2], twp, rb_sel, k2, false, M, M1, ra, rb, gs, a.ov,
+                                                            sbo, jo, a.grid, P, w1, w2, rg, ro, acc);
             if (nyq)
-                cbn[s2] = row_bin_ph<M2, LP>(zr[s2], twp, false, 0, true, M, M1, ra, rb, gs, a.ov, sbo, jo,
-                                             a.grid, P, w1, w2, nacc);
+                cbn[s2] = nyq_bin_ph<M2, LP, PLAIN>(a, zr[s2], twp, M1, ra, rb, gs, sbo, jo, P, w1, w2, it + s2, nacc);
+        };
+        if constexpr (PLAIN) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * fsel + i < nfr) bins(4 * fsel + i, cg.v[i], co.v[i]);
+        } else {
+            for (int s2 = fsel; s2 < nfr; s2 += 2) bins(s2, make_float2(0.f, 0.f), make_float2(0.f, 0.f));
         }
         __syncthreads();   // every thread is done with the rows; cb complete
         {
@@ -889,35 +1125,47 @@ __global__ __launch_bounds__(256, 4) void k_large_pass2_r8_ph(SectorArgs a, cons
 hipError_t launch_large_pass2_phased(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                      const void *pp, int M1, int M2, const float2 *tw_m2,
                                      const float2 *tw_m, bool raw, int n_groups, int accumulate,
-                                     hipStream_t s) {
+                                     bool plain, hipStream_t s) {
     const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
     if (M1 * M2 != a.M || sbo % M1 != 0 || (M2 != 64 && M2 != 128 && M2 != 256) || M1 != 128 ||
         (raw && !a.cb_out))
         return hipErrorInvalidValue;
-    const int64_t fpg = (a.nf + n_groups - 1) / n_groups;
+    int64_t fpg = (a.nf + n_groups - 1) / n_groups;
+    if (plain) {   // whole iterations, so that the chain runs start on their 64-byte lines
+        if (a.chain == nullptr || a.chain_ld < a.nf + 8) return hipErrorInvalidValue;
+        fpg = (fpg + 7) & ~(int64_t)7;
+    }
     const dim3 grid((unsigned)(M1 / 2), (unsigned)n_groups);
     if (raw && M2 == 64) {
-        hipLaunchKernelGGL(k_large_pass2_r8_ph, grid, dim3(256), 0, s, a, y1, y2, (const PhasedParam *)pp,
-                           M1, tw_m2, tw_m, fpg, accumulate);
+        auto kern = plain ? k_large_pass2_r8_ph<true> : k_large_pass2_r8_ph<false>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, y1, y2, (const PhasedParam *)pp, M1, tw_m2, tw_m,
+                           fpg, accumulate);
         return hipGetLastError();
     }
-    auto kern = M2 == 64    ? k_large_pass2_r8<64, P2_PHASED>
-                : M2 == 128 ? (raw ? k_large_pass2_r8<128, P2_PHASED_CB> : k_large_pass2_r8<128, P2_PHASED>)
-                            : (raw ? k_large_pass2_r16<P2_PHASED_CB> : k_large_pass2_r16<P2_PHASED>);
+    auto pick = [raw](auto cb, auto power) { return raw ? cb : power; };
+    auto kern = M2 == 64    ? (plain ? k_large_pass2_r8<64, P2_PHASED, true> : k_large_pass2_r8<64, P2_PHASED, false>)
+                : M2 == 128 ? (plain ? pick(k_large_pass2_r8<128, P2_PHASED_CB, true>, k_large_pass2_r8<128, P2_PHASED, true>)
+                                     : pick(k_large_pass2_r8<128, P2_PHASED_CB, false>, k_large_pass2_r8<128, P2_PHASED, false>))
+                            : (plain ? pick(k_large_pass2_r16<P2_PHASED_CB, true>, k_large_pass2_r16<P2_PHASED, true>)
+                                     : pick(k_large_pass2_r16<P2_PHASED_CB, false>, k_large_pass2_r16<P2_PHASED, false>));
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, y1, y2, pp, M1, tw_m2, fpg, accumulate);
     return hipGetLastError();
 }
 
 hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                   const FrameParam *params, int M1, int M2, const float2 *tw_m2,
-                                  int n_groups, int accumulate, hipStream_t s) {
+                                  int n_groups, int accumulate, bool plain, hipStream_t s) {
     const int sbo = (a.grid == 0) ? (a.a2s - a.a1s) : (a.a1s - a.a2s);
     if (M1 * M2 != a.M || sbo % M1 != 0 || (M2 != 64 && M2 != 128 && M2 != 256)) return hipErrorInvalidValue;
-    const int64_t fpg = (a.nf + n_groups - 1) / n_groups;
+    int64_t fpg = (a.nf + n_groups - 1) / n_groups;
+    if (plain) {   // whole iterations, so that the chain runs start on their 64-byte lines
+        if ((a.flags & FLAG_XCF) && (a.chain == nullptr || a.chain_ld < a.nf + 8)) return hipErrorInvalidValue;
+        fpg = (fpg + 7) & ~(int64_t)7;
+    }
     const dim3 grid((unsigned)(M1 / 2), (unsigned)n_groups);
-    auto kern = M2 == 64    ? k_large_pass2_r8<64, P2_PRODUCTS>
-                : M2 == 128 ? k_large_pass2_r8<128, P2_PRODUCTS>
-                            : k_large_pass2_r16<P2_PRODUCTS>;
+    auto kern = M2 == 64    ? (plain ? k_large_pass2_r8<64, P2_PRODUCTS, true> : k_large_pass2_r8<64, P2_PRODUCTS, false>)
+                : M2 == 128 ? (plain ? k_large_pass2_r8<128, P2_PRODUCTS, true> : k_large_pass2_r8<128, P2_PRODUCTS, false>)
+                            : (plain ? k_large_pass2_r16<P2_PRODUCTS, true> : k_large_pass2_r16<P2_PRODUCTS, false>);
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, y1, y2, (const void *)params, M1, tw_m2, fpg,
                        accumulate);
     return hipGetLastError();

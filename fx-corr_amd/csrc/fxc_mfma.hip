@@ -2352,54 +2352,6 @@ __global__ __launch_bounds__(64 * R) void k_fft_pass1_mfma(const IN *in, float2 
     }
 }
 
-// One element (two consecutive samples, the first at src0 = 2m - shift of
-// the shifted frame) from words staged per four-step row: lw is the local
-// index of the word holding bit src0 * bits and off its bit offset.  The
-// code width is fixed at compile time for 1, 2, 4 and 8 bits (0: the
-// station's run-time width, at most 16 so that both codes fit one funnel
-// shift).  Branch-free: the LSB flip is a sign mask per sample parity (fm0
-// for the first sample, fm1 for the second; the parity of src0 is the
-// shift's), and samples outside the frame are zero.
-template <int BITS>
-__device__ __forceinline__ float2 decode_pair_local(const uint32_t *words, const StationDev &st,
-                                                    const float *lev_lds, int src0, int lw,
-                                                    uint32_t off, int N, uint32_t fm0,
-                                                    uint32_t fm1) {
-    const uint32_t v = __builtin_amdgcn_alignbit(words[lw + 1], words[lw], off);
-    float x0, x1;
-    if constexpr (BITS == 1) {
-        x0 = (v & 1u) ? st.lev4[1] : st.lev4[0];
-        x1 = (v & 2u) ? st.lev4[1] : st.lev4[0];
-    } else if constexpr (BITS == 2 || BITS == 4 || BITS == 8) {
-        constexpr uint32_t mask = (1u << BITS) - 1u;
-        x0 = lev_lds[v & mask];
-        x1 = lev_lds[(v >> BITS) & mask];
-    } else {
-        x0 = level_of(v & st.code_mask, st, lev_lds);
-        x1 = level_of((v >> st.bits) & st.code_mask, st, lev_lds);
-    }
-    x0 = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x0) ^ fm0);
-    x1 = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x1) ^ fm1);
-    return make_float2((unsigned)src0 < (unsigned)N ? x0 : 0.0f,
-                       (unsigned)(src0 + 1) < (unsigned)N ? x1 : 0.0f);
-}
-
-// Word gw of a frame (little-endian, shuffle applied); zero outside it.
-__device__ __forceinline__ uint32_t frame_word(const uint8_t *frame, const StationDev &st, int gw) {
-    if (gw < 0 || gw >= st.nwords) return 0u;
-    uint32_t v = 0;
-    if (st.aligned) {
-        v = reinterpret_cast<const uint32_t *>(frame)[gw];
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int b = 4 * gw + j;
-            if (b < st.bpf) v |= (uint32_t)frame[b] << (8 * j);
-        }
-    }
-    return shuffle_word(v, st);
-}
-
 // The same first pass with the frame decode fused in (chosen form, sector
 // path, M1 = 128 = 32 x 4).  Workgroup (frame, part p) takes the columns
 // m2 in [64 p, 64 p + 64) of all 128 rows m1 (element m = m2 + M2 m1): it
