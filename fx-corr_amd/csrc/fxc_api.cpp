@@ -1140,6 +1140,12 @@ static fxc_status grow(fxc_plan *p, DevBuf &b, size_t bytes, hipStream_t s, cons
         return fail(FXC_ERR_NOMEM, "%s: device allocation of %zu bytes failed", what, bytes);
     return FXC_OK;
 }
+// Whether a call may use `bytes` of the buffer: it holds them or may grow.  The
+// paths that need more scratch than the general ones are left for those where
+// it may not, so that a call a capture or a live graph accepts stays accepted.
+static bool can_hold(const fxc_plan *p, const DevBuf &b, size_t bytes, hipStream_t s) {
+    return bytes <= b.cap || !(p->live_graphs > 0 || stream_capturing(s));
+}
 #define GROW(p, buf, bytes, s, what)                                  \
     do {                                                              \
         fxc_status g_ = grow((p), (buf), (bytes), (s), (what));       \
@@ -1426,6 +1432,7 @@ constexpr int kChainSpanMinLen = 4096;
 
 // Frames (whole chunks, at least one) whose chains (`len` links, `row_bytes`
 // per frame) one launch computes for a sector of nf frames.
+static bool phased_fused_ok(const fxc_plan *p);
 static int64_t chain_span(int64_t nf, int64_t chunk, size_t row_bytes, int len) {
     if (len < kChainSpanMinLen) return chunk;
     const int64_t fit = std::max<int64_t>(1, (int64_t)(kChainSpanBytes / row_bytes) / chunk);
@@ -1471,6 +1478,30 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
     return FXC_OK;
 }
 
+// The general phased path's chunk, chain span and scratch for nf frames.  Per
+// frame: two rotation chains and, for the .raw output, the combined half
+// spectrum (the inverse FFT quantises its time series from LDS; the N * 4 term
+// keeps the chunking of the staged form).  The chunk does not depend on
+// whether .raw is written, so |cb|^2 sums in the same order either way.
+struct PhasedScratch {
+    int64_t chunk, span;
+    size_t chain_bytes, cb_bytes;
+};
+static PhasedScratch phased_scratch(const fxc_plan *p, int64_t nf) {
+    const size_t half = (size_t)p->half, row = 2 * (size_t)chain_ld_for((int)half) * 8;
+    PhasedScratch r;
+    if (p->fft_form == 2) {   // the fused four-step's smaller chunks are not the general path's
+        r.chunk = phased_fused_ok(p) ? p->chunk : p->chunk_use;
+    } else {
+        const size_t per_frame = row + half * 8 + (size_t)p->N * 4;
+        r.chunk = std::max<int64_t>(1, std::min<int64_t>(nf, (int64_t)(((size_t)256 << 20) / per_frame)));
+    }
+    r.span = chain_span(nf, r.chunk, row, (int)half);
+    r.chain_bytes = p->desc.precision == FXC_PRECISION_CHOSEN ? 0 : (size_t)r.span * row;
+    r.cb_bytes = (size_t)r.chunk * half * 8;
+    return r;
+}
+
 // Phased sum on the wave kernel: equal chunks whose combined spectra (.raw) and
 // rotation chains (plain) fit kPhasedWaveBytes, so that the kernels after them
 // read both from the Infinity Cache.  A delay model with the geometric table
@@ -1479,7 +1510,7 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
 constexpr size_t kPhasedWaveBytes = (size_t)192 << 20;
 
 static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64_t nf,
-                                      uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
+                                      uint8_t *d_raw_out, double *d_acc, hipStream_t s, bool *done) {
     const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
     const size_t half = (size_t)p->half;
     const int64_t bpf_o = plan_bpf_out(p);
@@ -1491,9 +1522,17 @@ static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64
     if (per_frame) chunk = std::min<int64_t>(chunk, (int64_t)(kPhasedWaveBytes / per_frame));
     const int64_t nchunks = (nf + chunk - 1) / chunk;
     chunk = (nf + nchunks - 1) / nchunks;
-    if (nch) GROW(p, p->d_chain, (size_t)chunk * nch * ld * 8, s, "phased rotation chains");
-    if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
-    GROW(p, p->d_wparams, (size_t)chunk * sizeof(WkPhased), s, "frame parameters");
+    // the general path's scratch too, which a later captured call may need
+    const PhasedScratch g = phased_scratch(p, nf);
+    const size_t chain_b = nch ? std::max((size_t)chunk * nch * ld * 8, g.chain_bytes) : 0;
+    const size_t cb_b = raw ? std::max((size_t)chunk * half * 8, g.cb_bytes) : 0;
+    const size_t par_b = (size_t)chunk * sizeof(WkPhased);
+    if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s) || !can_hold(p, p->d_wparams, par_b, s))
+        return FXC_OK;
+    *done = true;
+    if (nch) GROW(p, p->d_chain, chain_b, s, "phased rotation chains");
+    if (raw) GROW(p, p->d_cb, cb_b, s, "phased spectra");
+    GROW(p, p->d_wparams, par_b, s, "frame parameters");
     const int64_t fpw = frames_per_wg(p, chunk, wave_wg_cap(), true);
     const int n_wg = (int)((chunk + fpw - 1) / fpw);
     for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
@@ -1525,23 +1564,21 @@ static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64
 static fxc_status enqueue_phased(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                  uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
     if (p->fft_form == 1) return enqueue_phased_mf3(p, base, nf, d_raw_out, d_acc, s);
-    if (wave_for(p, nf)) return enqueue_phased_wave(p, base, nf, d_raw_out, d_acc, s);
+    if (wave_for(p, nf)) {
+        bool done = false;   // not where its scratch may not grow
+        const fxc_status st = enqueue_phased_wave(p, base, nf, d_raw_out, d_acc, s, &done);
+        if (done || st != FXC_OK) return st;
+    }
     const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
     const size_t half = (size_t)p->half;
     const int64_t bpf_o = plan_bpf_out(p);
-    // per-frame scratch: two rotation chains and, for the .raw output, the
-    // combined half spectrum (the inverse FFT quantises its time series from
-    // LDS; the N * 4 term keeps the chunking of the staged form).  The chunk
-    // does not depend on whether .raw is written, so |cb|^2 sums in the same
-    // order either way.
     // chosen form: rotations from FP64 phases in the kernel, no chain table
     const int prec = p->desc.precision == FXC_PRECISION_CHOSEN ? 1 : 0;
     const int ld = chain_ld_for((int)half);
-    const size_t per_frame = 2 * (size_t)ld * 8 + half * 8 + (size_t)p->N * 4;
-    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(nf, (int64_t)(((size_t)256 << 20) / per_frame)));
-    const int64_t span = chain_span(nf, chunk, 2 * (size_t)ld * 8, (int)half);
-    if (!prec) GROW(p, p->d_chain, (size_t)span * 2 * ld * 8, s, "phased rotation chains");
-    if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
+    const PhasedScratch g = phased_scratch(p, nf);
+    const int64_t chunk = g.chunk, span = g.span;
+    if (!prec) GROW(p, p->d_chain, g.chain_bytes, s, "phased rotation chains");
+    if (raw) GROW(p, p->d_cb, g.cb_bytes, s, "phased spectra");
     const int64_t fpw = frames_per_wg(p, chunk, p->max_wg);
     const int n_wg = (int)((chunk + fpw - 1) / fpw);
     int64_t span0 = -1;    // first frame (of this sector) of the computed chains
@@ -1594,10 +1631,10 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
     const float2 *twm = (const float2 *)p->tw_lm.p;
     const int prec = p->desc.precision == FXC_PRECISION_CHOSEN ? 1 : 0;
     const int ld = chain_ld_for((int)half);
-    const int64_t chunk = p->chunk_use;
-    const int64_t span = chain_span(nf, chunk, 2 * (size_t)ld * 8, (int)half);
-    if (!prec) GROW(p, p->d_chain, (size_t)span * 2 * ld * 8, s, "phased rotation chains");
-    if (raw) GROW(p, p->d_cb, (size_t)chunk * half * 8, s, "phased spectra");
+    const PhasedScratch g = phased_scratch(p, nf);
+    const int64_t chunk = g.chunk, span = g.span;
+    if (!prec) GROW(p, p->d_chain, g.chain_bytes, s, "phased rotation chains");
+    if (raw) GROW(p, p->d_cb, g.cb_bytes, s, "phased spectra");
     int64_t span0 = -1;    // first frame (of this sector) of the computed chains
     for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
         const int64_t cn = std::min(chunk, nf - c0);
@@ -1649,13 +1686,12 @@ static fxc_status enqueue_phased_large(fxc_plan *p, const SectorArgs &base, int6
 // N = 32768 / 65536: chunks of frames through HBM scratch; the product
 // kernel's kLargeGroups frame-group partial slots accumulate over the chunks
 // in order, then one fixed-order reduce.
-// The chosen form's fused four-step (decode in the first pass; the second
-// pass, untangle and products in one kernel) applies when both stations'
-// bins of a product lie on the same rows (band shift a multiple of M1) and
-// both code widths are at most 16 bits (two codes per funnel shift).
-// The fused four-step runs at M1 = 128 (variant 1 of the large form).
-// The fused four-step (M1 = 128): N = 32768 / 65536 (the large form's
-// default), and N = 16384 (M2 = 64) as variant 1 of the Stockham form.
+// The fused four-step (decode in the first pass; the second pass, untangle
+// and products in one kernel) applies when both stations' bins of a product
+// lie on the same rows (band shift a multiple of M1 = 128) and both code
+// widths are at most 16 bits (two codes per funnel shift).  It is variant 1:
+// the default at N = 32768 / 65536, and of the Stockham form at N = 16384
+// (M2 = 64).
 // The plain form takes it with an FP32 first pass and, for the XCF, the
 // phase chains link-major (an XCF over few bins, which uses no chains, stays
 // on the Stockham kernel / the four-step through HBM): 2^27 samples of both
@@ -1739,7 +1775,7 @@ static int64_t chain_links_ld(int64_t frames) { return ((frames + 8 + 15) & ~(in
 // phased spectra as rows, the inverse's first pass takes the rows as they
 // are, its second ends in natural order with the quantiser.
 static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int64_t nf,
-                                       uint8_t *d_raw_out, double *d_acc, hipStream_t s) {
+                                       uint8_t *d_raw_out, double *d_acc, hipStream_t s, bool *done) {
     const bool raw = (p->desc.products & FXC_PRODUCT_RAW_OUT) && d_raw_out != nullptr;
     const int64_t bpf_o = plan_bpf_out(p);
     // the .raw second pass holds four waves per SIMD (the power-only one
@@ -1752,10 +1788,18 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
     const int nch = base.dly.table != nullptr ? 1 : 2;
     const int64_t cspan = plain ? chain_span(nf, p->chunk_use, (size_t)nch * p->half * 8, (int)p->half) : 0;
     const int64_t cld = chain_links_ld(std::min(cspan, nf));
-    if (plain) GROW(p, p->d_chain, (((size_t)p->half + 7) & ~(size_t)7) * nch * cld * 8, s, "phased rotation chains");
+    size_t chain_b = 0, cb_b = raw ? (size_t)p->chunk_use * p->half * 8 : 0;
+    if (plain) {   // with the general path's scratch, which a later captured call may need
+        const PhasedScratch g = phased_scratch(p, nf);
+        chain_b = std::max((((size_t)p->half + 7) & ~(size_t)7) * nch * cld * 8, g.chain_bytes);
+        if (raw) cb_b = std::max(cb_b, g.cb_bytes);
+        if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s)) return FXC_OK;
+        GROW(p, p->d_chain, chain_b, s, "phased rotation chains");
+    }
+    *done = true;
     int64_t cspan0 = -1;
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
-    if (raw) GROW(p, p->d_cb, (size_t)p->chunk_use * p->half * 8, s, "phased spectra");
+    if (raw) GROW(p, p->d_cb, cb_b, s, "phased spectra");
     const int64_t span = fused_param_span(p);
     int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
     for (int64_t c0 = 0; c0 < nf; c0 += p->chunk_use) {
@@ -1808,20 +1852,42 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
     return FXC_OK;
 }
 
-static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf, double *d_acc,
+// Frames of one slab of the sector kernels' phase chains, and of one span of
+// the four-step through HBM (whole chunks, not the fused path's smaller ones)
+static int64_t chain_slab(const fxc_plan *p, int64_t nf) {
+    const size_t row = (size_t)chain_ld_for((int)(p->desc.a1e - p->desc.a1s)) * 8;
+    return std::min<int64_t>(nf, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / row)));
+}
+static int64_t large_chunk(const fxc_plan *p) { return large_fused_ok(p) ? p->chunk : p->chunk_use; }
+
+// Plain XCF on the fused four-step: the chains of whole chunks, link-major,
+// and the table's size, at least the general path's (a later captured call
+// may need that).
+static int64_t fused_chain_span(const fxc_plan *p, int64_t nf) {
+    const int ov = (int)(p->desc.a1e - p->desc.a1s);
+    return xcf_uses_chain(p) ? chain_span(nf, p->chunk_use, (size_t)ov * 8, ov) : 0;
+}
+static size_t fused_chain_bytes(const fxc_plan *p, int64_t nf) {
+    if (!xcf_uses_chain(p)) return 0;
+    const int ov = (int)(p->desc.a1e - p->desc.a1s);
+    const size_t row = (size_t)chain_ld_for(ov) * 8;
+    const int64_t rows = p->fft_form == 2 ? chain_span(nf, large_chunk(p), row, ov) : chain_slab(p, nf);
+    return std::max((size_t)((ov + 7) & ~7) * chain_links_ld(std::min(fused_chain_span(p, nf), nf)) * 8,
+                    (size_t)rows * row);
+}
+
+static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf, double *d_acc, bool fused,
                                 hipStream_t s) {
     const float2 *twl1 = (const float2 *)(p->M1 == 128 ? p->tw_l1.p : p->tw_l2.p);
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
-    if (large_fused_ok(p) && fused_for(p, nf)) {
+    if (fused) {
         const int ng = large_fused_groups(p);
         const int64_t span = fused_param_span(p);
         int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
         const bool plain = p->desc.precision == FXC_PRECISION_PLAIN_FP32;
-        // plain XCF: the chains of whole chunks, link-major
         const bool chain = xcf_uses_chain(p);
-        const int64_t cspan = chain ? chain_span(nf, p->chunk_use, (size_t)base.ov * 8, base.ov) : 0;
-        const int64_t cld = chain_links_ld(std::min(cspan, nf));
-        if (chain) GROW(p, p->d_chain, (size_t)((base.ov + 7) & ~7) * cld * 8, s, "phase chains");
+        const int64_t cspan = fused_chain_span(p, nf), cld = chain_links_ld(std::min(cspan, nf));
+        if (chain) GROW(p, p->d_chain, fused_chain_bytes(p, nf), s, "phase chains");
         int64_t cspan0 = -1;
         for (int64_t c0 = 0; c0 < nf; c0 += p->chunk_use) {
             const int64_t cn = std::min(p->chunk_use, nf - c0);
@@ -1863,16 +1929,17 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
                                     d_acc, s));
         return FXC_OK;
     }
+    const int64_t chunk = large_chunk(p);
     const bool chain = xcf_uses_chain(p);
     const int ld = chain ? chain_ld_for(base.ov) : 0;
     int64_t span = 0;      // frames whose chains one launch computes: whole chunks
     if (chain) {
-        span = chain_span(nf, p->chunk_use, (size_t)ld * 8, base.ov);
+        span = chain_span(nf, chunk, (size_t)ld * 8, base.ov);
         GROW(p, p->d_chain, (size_t)span * ld * 8, s, "phase chains");
     }
     int64_t span0 = -1;    // first frame (of this sector) of the computed chains
-    for (int64_t c0 = 0; c0 < nf; c0 += p->chunk_use) {
-        const int64_t cn = std::min(p->chunk_use, nf - c0);
+    for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
+        const int64_t cn = std::min(chunk, nf - c0);
         SectorArgs a = base;
         a.raw1 = base.raw1 + c0 * p->st[0].bpf;
         a.raw2 = base.raw2 + c0 * p->st[1].bpf;
@@ -1957,18 +2024,24 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     a.raw2 = d_raw2;
     a.first_frame = first_frame;
     a.nf = nf;
-    if (phased && phased_fused_ok(p) && fused_for(p, nf))
-        return enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s);
+    if (phased && phased_fused_ok(p) && fused_for(p, nf)) {
+        bool done = false;   // plain: not where its scratch may not grow
+        st = enqueue_phased_fused(p, a, nf, d_raw_out, d_acc, s, &done);
+        if (done || st != FXC_OK) return st;
+    }
     if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
-    if (p->fft_form == 2 || (large_fused_ok(p) && p->desc.precision == FXC_PRECISION_CHOSEN))
-        return enqueue_large(p, a, nf, d_acc, s);
-    if (large_fused_ok(p) && fused_for(p, nf)) {   // plain N = 16384: timed as on the Stockham kernel
+    // plain: not where its chain table may not grow
+    const bool fused = large_fused_ok(p) && fused_for(p, nf) && can_hold(p, p->d_chain, fused_chain_bytes(p, nf), s);
+    if (p->fft_form == 2 || (fused && p->desc.precision == FXC_PRECISION_CHOSEN))
+        return enqueue_large(p, a, nf, d_acc, fused, s);
+    if (fused) {   // plain N = 16384: timed as on the Stockham kernel
         std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
-        if ((st = timing_begin(p, s, ev)) != FXC_OK || (st = enqueue_large(p, a, nf, d_acc, s)) != FXC_OK) return st;
+        if ((st = timing_begin(p, s, ev)) != FXC_OK || (st = enqueue_large(p, a, nf, d_acc, fused, s)) != FXC_OK) return st;
         return timing_end(p, s, ev);
     }
-    const bool wave = wave_for(p, nf);
+    const size_t par_b = (size_t)std::min(nf, kWaveSlab) * sizeof(WkParam);
+    const bool wave = wave_for(p, nf) && can_hold(p, p->d_wparams, par_b, s);
     const int wg_cap = std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div);
     // Plain XCF over more than kChainMinOverlap bins: slabs of frames whose
     // f32 phase chains fit the chain scratch; the slabs add into the same
@@ -1976,14 +2049,13 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     const bool chain = p->fft_form == 0 && xcf_uses_chain(p);
     const int ld = chain ? chain_ld_for(a.ov) : 0;
     int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
-    if (chain)
-        slab = std::min<int64_t>(slab, std::max<int64_t>(kFrameBatch, (int64_t)(kChainSlabBytes / ((size_t)ld * 8))));
+    if (chain) {
+        slab = std::min(slab, chain_slab(p, nf));
+        GROW(p, p->d_chain, (size_t)chain_slab(p, nf) * ld * 8, s, "phase chains");
+    }
     // slabs of equal length (a short last one would leave most workgroups idle)
     slab = (nf + (nf + slab - 1) / slab - 1) / ((nf + slab - 1) / slab);
-    if (chain) {
-        GROW(p, p->d_chain, (size_t)slab * ld * 8, s, "phase chains");
-    }
-    if (wave) GROW(p, p->d_wparams, (size_t)slab * sizeof(WkParam), s, "frame parameters");
+    if (wave) GROW(p, p->d_wparams, par_b, s, "frame parameters");
     const int64_t fpw = frames_per_wg(p, slab, wg_cap, wave);
     const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;

@@ -12,6 +12,11 @@
 //   4. k_mac_large      realfft untangle and ACF/XCF products, one output
 //                       bin per thread looping over a group of frames, FP64
 //                       accumulators (any band shift)
+//
+// Where both stations' bins share the four-step's rows, the fused four-step
+// (also N = 16384): the plain form's first pass with the decode in it
+// (k_large_pass1_f32; the chosen form's is in fxc_mfma.hip) and the second
+// passes with the untangle and the products or the phased bin in them.
 #include "fxc_dev.h"
 
 namespace fxc {
@@ -432,8 +437,8 @@ hipError_t launch_large_pass1_f32(const SectorArgs &a, const int64_t *shifts, fl
 }
 
 // ------------------------------------ second pass fused with the products
-// Chosen form, both stations' bins on the same rows of the four-step (the
-// band shift a multiple of M1).  Z[k1 + M1 k2] is row k1's DFT over m2 of
+// Both stations' bins on the same rows of the four-step (the band shift a
+// multiple of M1).  Z[k1 + M1 k2] is row k1's DFT over m2 of
 // Y[k1][m2], and bin M - k lies in row M1 - k1 (row 0 and row M1/2 are their
 // own mirrors), so the untangle of a bin needs only its row pair.
 // Workgroup (pair p, frame group): rows ra = p, rb = M1 - p (p = 0: rows 0

@@ -91,3 +91,56 @@ def test_wave_phased_both_stations_delayed(n, nf, shift, grid, form):
     # power: the forms' bars; codes: a byte holds two, each may flip at a decision boundary (1e-4 of codes)
     assert np.max(np.abs(g["acc_ph"] / o["acc_ph"] - 1)) < (1e-5 if plain else 1e-4)
     assert np.count_nonzero(g["raw_out"] != o["raw_out"]) <= 2e-4 * o["raw_out"].size + 2
+
+
+@pytest.mark.parametrize("n,form,products,small,large", [
+    (4096, "chosen", ACF | XCF, 0, 3000), (1024, "plain", ACF | XCF, 700, 5000), (4096, "plain", XCF, 3000, 1500),
+    (2048, "chosen", F.PRODUCT_PHASED, 0, 3000), (1024, "plain", F.PRODUCT_PHASED | F.PRODUCT_RAW_OUT, 9000, 2500),
+    (16384, "plain", ACF | XCF, 900, 600), (16384, "plain", F.PRODUCT_PHASED, 700, 600)])
+def test_capture_without_room_to_grow(n, form, products, small, large):
+    """A captured call runs where the plan's scratch may not grow: as the
+    plan's first call (small = 0) or after an eager call of another length;
+    also while the graph is alive.  Against an eager call on a fresh plan."""
+    fs, m = 64e6, n // 2
+    raw = bool(products & F.PRODUCT_RAW_OUT)
+    c = make_case(n=n, fs=fs, nf=max(small, large), rho=0.3, seed=n, no_table=True, net_d1_base=4.4 / fs,
+                  total_rate1_base=1e-9, band=(0, 0, m, 0) if n > 4096 else (1, 0, m - 1, 1))
+    cfg, prec = F.make_delay_cfg(c["table"], **c["delay"]), (F.PRECISION_PLAIN_FP32 if form == "plain" else
+                                                             F.PRECISION_CHOSEN)
+    s = F.Stream()
+    r1, r2 = F.DeviceBuffer(c["raw1"].size), F.DeviceBuffer(c["raw2"].size)
+    r1.upload(c["raw1"])
+    r2.upload(c["raw2"])
+
+    def plan():
+        return F.Plan(n, bits=c["bits"], levels=c["levels"], band=c["band"], df_hz=fs / n, products=products,
+                      bit_out=2, precision=prec)
+
+    keep = []   # buffers stay until the end
+
+    def run(p, nf):
+        acc, out = F.DeviceBuffer(F.N_PRODUCTS * p.half * 8), F.DeviceBuffer(max(8, nf * n // 4))
+        keep.extend((acc, out))
+        return acc, lambda: p.sector_run_device(r1.ptr, r2.ptr, 0, nf, cfg, acc.ptr,
+                                                     **(dict(d_raw_out=out.ptr) if raw else {}), stream=s.ptr)
+
+    p, q = plan(), plan()
+    acc_q, call_q = run(q, large)
+    call_q()
+    if small:
+        run(p, small)[1]()
+    s.sync()
+    want = acc_q.download(np.zeros(F.N_PRODUCTS * q.half))
+    acc, call = run(p, large)
+    g = F.Graph(s)
+    call()
+    g.end()
+    acc2, eager = run(p, large)
+    for _ in range(2):
+        g.launch()
+        eager()
+        s.sync()
+        for a in (acc, acc2):   # either path: the form's bar on the spectrum's scale
+            got = a.download(np.zeros(F.N_PRODUCTS * p.half))
+            assert np.max(np.abs(got - want)) < (1e-5 if form == "plain" else 1e-4) * np.max(np.abs(want))
+    g.close()
