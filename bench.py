@@ -74,18 +74,17 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_1024msps_2bit_fft1024
 # pass in profiles/sector_kernels_1024msps_2bit_fft1024_kernel_stats.md:
 # (VALU instructions, matrix-busy cycles).  A wave64 VALU instruction takes
 # 4 cycles of its SIMD; MI355X has 1,024 SIMDs at up to 2.4 GHz.
-ISSUE_PER_FRAME = {"k_sector_mf3": (664.8, 512.0), "k_sector_mf3<FP32 batches>": (618.0, 512.0),
-                   "k_sector<8, 64, 0>": (2973.0, 0.0)}
+ISSUE_PER_FRAME = {"k_sector_mf3": (664.8, 512.0), "k_sector_mf3<FP32 batches>": (618.0, 512.0)}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 COUNTS_FILE = "profiles/sector_kernels_1024msps_2bit_fft1024_kernel_stats.md"
 # fused kernel of each form (the MFMA form by kernel organization variant)
 KERNEL_KEYS = {("chosen", 0): "k_sector_mf2", ("chosen", 1): "k_sector_mf3",
-               ("chosen", 2): "k_sector_mf3<FP32 batches>", ("plain", 0): "k_sector<8, 64, 0>"}
+               ("chosen", 2): "k_sector_mf3<FP32 batches>", ("plain", 0): "k_sector_wave"}
 KERNEL_LABELS = {"k_sector_mf2": "fused decode+shift+MFMA four-step FFT+MAC, whole-frame waves",
                  "k_sector_mf3": "fused decode+shift+MFMA four-step FFT+MAC, producer/consumer waves",
                  "k_sector_mf3<FP32 batches>": "fused decode+shift+MFMA four-step FFT+MAC, "
                                                "producer/consumer waves, FP32 batch sums",
-                 "k_sector<8, 64, 0>": "fused decode+shift+FFT+MAC (plain FP32)"}
+                 "k_sector_wave": "fused decode+shift+FFT+MAC, wave-private transforms (plain FP32)"}
 
 
 def _pmc_rows(d):
@@ -310,7 +309,7 @@ def load_traffic(key):
     return None
 
 
-FORM_NAMES = {0: "FP32 Stockham", 1: "FP16-MFMA four-step", 2: "FP32 four-step through HBM"}
+FORM_NAMES = {0: "FP32 wave kernel (N = 256..8192, longer sectors) or Stockham", 1: "FP16-MFMA four-step", 2: "FP32 four-step through HBM"}
 
 
 def form_name(info):
@@ -320,7 +319,7 @@ def form_name(info):
     if info.fft_form == 2 and info.fft_mfma:
         return "four-step through HBM, FP16-MFMA DFT-32 first pass"
     if info.fft_form == 0 and info.fft_mfma:
-        return "Stockham, FP16-MFMA DFT-32 first pass"
+        return "wave kernel, FP16-MFMA DFT-32 columns" if info.fft_len <= 8192 else "Stockham, FP16-MFMA DFT-32 first pass"
     return FORM_NAMES[info.fft_form]
 
 

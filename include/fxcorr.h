@@ -229,7 +229,7 @@ fxc_status fxc_sector_run_device(fxc_plan *plan, const uint8_t *d_raw1,
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The call allocates and frees nothing and never synchronises;
- * its scratch (geometric table, workgroup partial sums, reduction sums) is
+ * its scratch (geometric table, frame parameters, workgroup partial sums) is
  * one static device array of FXC_NOALLOC_SCRATCH_BYTES per device, held
  * until the process ends.  Same arguments and d_acc layout as
  * fxc_sector_run_device, for ACF/XCF plans of fft_len <= 16384 whose XCF
@@ -432,15 +432,18 @@ fxc_status fxc_plan_device_bytes(const fxc_plan *plan, uint64_t *bytes);
  * the spectrum's scale) for the FP32-batch organization. */
 typedef struct {
     int32_t candidates;
-    int32_t variant;           /* Stockham: 0 default passes, 1 radix-16 passes
-                                  (N = 2048..8192) or, chosen form at N = 16384, the
-                                  fused four-step (split_m1 = 128, the default there;
+    int32_t variant;           /* Stockham: 0 default (the wave kernel, N = 256..8192
+                                  and longer sectors, else Stockham), 1 Stockham with
+                                  radix-16 passes (N = 2048..8192) or, at N = 16384,
+                                  the fused four-step (split_m1 = 128, the default
+                                  there; the plain form takes it from 512 frames;
                                   also for phased plans through fxc_plan_set_tuning,
-                                  0 then selects the Stockham phased kernel);
+                                  0 then selects the Stockham kernels);
                                   MFMA: 1 producer/consumer (default), 2 producer/consumer
                                   with FP32 sums over batches of 128 frames added to FP64
                                   totals, 0 whole-frame waves (2 and 0: N = 1024 only);
-                                  N >= 32768: 1 fused four-step, 0 through HBM */
+                                  N >= 32768: 1 fused four-step (plain: from 512
+                                  frames), 0 through HBM */
     int32_t grid_divisor;      /* workgroups = default / grid_divisor */
     int32_t split_m1;          /* four-step forms: column DFT length M1 (else 0) */
     int64_t chunk_frames;      /* four-step forms: frames per chunk (else 0) */
