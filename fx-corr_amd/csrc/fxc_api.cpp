@@ -965,6 +965,10 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
             hipMemcpy(p->out_lev.p, lv.data(), lv.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(fail(FXC_ERR_HIP, "level upload failed"));
     }
+    auto upload_twf = [&twf](DevBuf &b) {   // W_M^k for the four-step plans' output twiddles
+        return b.ensure(twf.size() * 4) == hipSuccess &&
+               hipMemcpy(b.p, twf.data(), twf.size() * 4, hipMemcpyHostToDevice) == hipSuccess;
+    };
     const int cus = num_cus();
     if (mfma_eligible(p)) {
         std::vector<uint8_t> tab = mfma_tables(p);
@@ -996,7 +1000,7 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
         };
         const size_t C = (size_t)p->chunk;
         p->chunk_use = p->chunk;
-        if (!table(p->tw_l1, 128) || !table(p->tw_l2, 256) || !table(p->tw_lm, (int)M) ||
+        if (!table(p->tw_l1, 128) || !table(p->tw_l2, 256) || !upload_twf(p->tw_lm) ||
             p->d_x[0].ensure(C * N * 4) != hipSuccess || p->d_x[1].ensure(C * N * 4) != hipSuccess ||
             p->d_y.ensure(C * M * 8) != hipSuccess || p->d_z[0].ensure(C * M * 8) != hipSuccess ||
             p->d_z[1].ensure(C * M * 8) != hipSuccess ||
@@ -1050,12 +1054,14 @@ extern "C" fxc_status fxc_plan_create(const fxc_plan_desc *desc, fxc_plan **out)
                        hipMemcpy(b.p, t.data(), t.size() * 4, hipMemcpyHostToDevice) == hipSuccess;
             };
             p->chunk_use = fused_chunk_default(p);
-            if (!table(p->tw_l0, 64) || !table(p->tw_lm, (int)M) ||
-                p->d_z[0].ensure(C * M * 8) != hipSuccess || p->d_z[1].ensure(C * M * 8) != hipSuccess ||
-                p->d_params.ensure(param_frames(C) * pb) != hipSuccess ||
-                p->d_lshifts.ensure(param_frames(C) * 16) != hipSuccess)
-                return cleanup(fail(FXC_ERR_NOMEM, "fused four-step scratch allocation failed"));
             p->param_cap = (int64_t)param_frames(C);
+            // plain: at the first call that takes this path (fused_reserve)
+            const bool now = desc->precision == FXC_PRECISION_CHOSEN;
+            if (!table(p->tw_l0, 64) || !upload_twf(p->tw_lm) ||
+                (now && (p->d_z[0].ensure(C * M * 8) != hipSuccess || p->d_z[1].ensure(C * M * 8) != hipSuccess ||
+                         p->d_params.ensure(param_frames(C) * pb) != hipSuccess ||
+                         p->d_lshifts.ensure(param_frames(C) * 16) != hipSuccess)))
+                return cleanup(fail(FXC_ERR_NOMEM, "fused four-step scratch allocation failed"));
         }
         if (desc->precision == FXC_PRECISION_PLAIN_FP32) {
             std::vector<float> t(2 * (size_t)M);
@@ -1761,6 +1767,26 @@ static bool fused_for(const fxc_plan *p, int64_t nf) {
     return p->desc.precision == FXC_PRECISION_CHOSEN || nf >= kPlainFusedFrames;
 }
 
+// The plain form's Y and parameter buffers at N = 16384, which short sectors
+// never use: held or able to grow, and their growth.
+static bool fused_ready(const fxc_plan *p, hipStream_t s) {
+    if (p->fft_form == 2 || p->desc.precision == FXC_PRECISION_CHOSEN) return true;
+    const size_t zb = (size_t)p->chunk_use * p->M * 8;
+    return can_hold(p, p->d_z[0], zb, s) && can_hold(p, p->d_z[1], zb, s) &&
+           can_hold(p, p->d_params, (size_t)p->param_cap * std::max(frame_param_bytes(), phased_param_bytes()), s) &&
+           can_hold(p, p->d_lshifts, (size_t)p->param_cap * 16, s);
+}
+static fxc_status fused_reserve(fxc_plan *p, hipStream_t s) {
+    if (p->fft_form == 2 || p->desc.precision == FXC_PRECISION_CHOSEN) return FXC_OK;
+    const size_t zb = (size_t)p->chunk_use * p->M * 8;
+    GROW(p, p->d_z[0], zb, s, "fused four-step rows");
+    GROW(p, p->d_z[1], zb, s, "fused four-step rows");
+    GROW(p, p->d_params, (size_t)p->param_cap * std::max(frame_param_bytes(), phased_param_bytes()), s,
+         "frame parameters");
+    GROW(p, p->d_lshifts, (size_t)p->param_cap * 16, s, "frame shifts");
+    return FXC_OK;
+}
+
 // Link-major chains: a link's row holds the span's frames and eight more (the
 // last iteration's reads), on an odd number of 64-byte lines.
 static int64_t chain_links_ld(int64_t frames) { return ((frames + 8 + 15) & ~(int64_t)15) | 8; }
@@ -1793,7 +1819,10 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
         const PhasedScratch g = phased_scratch(p, nf);
         chain_b = std::max((((size_t)p->half + 7) & ~(size_t)7) * nch * cld * 8, g.chain_bytes);
         if (raw) cb_b = std::max(cb_b, g.cb_bytes);
-        if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s)) return FXC_OK;
+        if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s) || !fused_ready(p, s))
+            return FXC_OK;
+        const fxc_status st = fused_reserve(p, s);
+        if (st != FXC_OK) return st;
         GROW(p, p->d_chain, chain_b, s, "phased rotation chains");
     }
     *done = true;
@@ -1881,6 +1910,8 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
     const float2 *twl1 = (const float2 *)(p->M1 == 128 ? p->tw_l1.p : p->tw_l2.p);
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
     if (fused) {
+        const fxc_status st = fused_reserve(p, s);
+        if (st != FXC_OK) return st;
         const int ng = large_fused_groups(p);
         const int64_t span = fused_param_span(p);
         int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
@@ -2031,8 +2062,9 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     }
     if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
-    // plain: not where its chain table may not grow
-    const bool fused = large_fused_ok(p) && fused_for(p, nf) && can_hold(p, p->d_chain, fused_chain_bytes(p, nf), s);
+    // plain: not where its scratch may not grow
+    const bool fused = large_fused_ok(p) && fused_for(p, nf) && fused_ready(p, s) &&
+                       can_hold(p, p->d_chain, fused_chain_bytes(p, nf), s);
     if (p->fft_form == 2 || (fused && p->desc.precision == FXC_PRECISION_CHOSEN))
         return enqueue_large(p, a, nf, d_acc, fused, s);
     if (fused) {   // plain N = 16384: timed as on the Stockham kernel

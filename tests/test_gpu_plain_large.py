@@ -23,6 +23,7 @@ LINE = 512   # frames
     (16384, 0, 33, (4, 2), (PERM, None), (True, False), -4096, 0, 33.2, ACF | XCF | OV),
     (16384, -1, 1024, (2, 4), (None, SWAP), (False, False), 0, 1, 16500.0, XCF),
     (16384, 9, 131, (8, 1), (SWAP, PERM), (True, True), -128, 1, 1.5, ACF),
+    (16384, 2, 300, (3, 5), (PERM, None), (False, True), 0, 0, 12.2, ACF | XCF),
     (32768, 3, 512, (2, 2), (None, None), (False, False), 0, 0, -31.7, ACF | XCF),
     (32768, 41, 99, (4, 1), (SWAP, PERM), (True, True), -256, 1, 64.9, ACF | XCF),
     (32768, 0, 100, (8, 2), (None, PERM), (False, True), 15744, 0, 2.5, XCF),

@@ -96,7 +96,7 @@ def test_wave_phased_both_stations_delayed(n, nf, shift, grid, form):
 @pytest.mark.parametrize("n,form,products,small,large", [
     (4096, "chosen", ACF | XCF, 0, 3000), (1024, "plain", ACF | XCF, 700, 5000), (4096, "plain", XCF, 3000, 1500),
     (2048, "chosen", F.PRODUCT_PHASED, 0, 3000), (1024, "plain", F.PRODUCT_PHASED | F.PRODUCT_RAW_OUT, 9000, 2500),
-    (16384, "plain", ACF | XCF, 900, 600), (16384, "plain", F.PRODUCT_PHASED, 700, 600)])
+    (16384, "plain", ACF | XCF, 900, 600), (16384, "plain", ACF, 0, 600), (16384, "plain", F.PRODUCT_PHASED, 700, 600)])
 def test_capture_without_room_to_grow(n, form, products, small, large):
     """A captured call runs where the plan's scratch may not grow: as the
     plan's first call (small = 0) or after an eager call of another length;
