@@ -73,7 +73,7 @@ struct WkShared {
     uint32_t slut[2][4 * 256];
     alignas(16) uint16_t dlut[2][kWkDlutHalves];
     float2 w2[S::A > 1 ? S::M2 : 1];
-    P pp[S::F];   // this round's frames
+    P pp[S::F];   // the iteration's frames
 };
 
 // Slot of element (row k1, position a B + b) of the wave's station-frame q.
@@ -604,7 +604,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
     const Par *params = reinterpret_cast<const Par *>(a.wk_params);
     for (int64_t fr = f_begin; fr < f_end; fr += F) {
         {
-            const int nf = (int)((f_end - fr) < F ? (f_end - fr) : F);   // frames of this round
+            const int nf = (int)((f_end - fr) < F ? (f_end - fr) : F);   // frames of this iteration
             const int lr = loop_local(l), tr = loop_local(t);   // see loop_local
             int sht[MF ? 4 : 1];
 #pragma unroll
