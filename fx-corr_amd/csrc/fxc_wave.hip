@@ -599,6 +599,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
 #pragma unroll
     for (int u = 0; u < 16; ++u) w[u] = 0u;
     wk_load<LOGM>(raw + (f_begin + fw) * bpf, nvalid(f_begin), bits, t, w);
+    __syncthreads();   // the tables are filled by all waves, and read by each on its own from here on
     float2 *zw = &sh.z[s][fw][0];
 
     const Par *params = reinterpret_cast<const Par *>(a.wk_params);
