@@ -184,6 +184,34 @@ __device__ __forceinline__ float2 sincos_turns(float r) {
                        __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, si) ^ ((uint32_t)(qi & 2) << 30)));
 }
 
+// A uniform constant kept in scalar registers: the compiler holds FP64
+// literals in vector registers and copies them ahead of every multiply-add.
+__device__ __forceinline__ double in_sgpr(double x) {
+    asm("" : "+s"(x));
+    return x;
+}
+
+// exp(2 pi i x), x in turns, in FP64, for phasors that are rounded to f32
+// once, at the bin: quadrant reduction to |t| <= 1/8 turn and polynomials in
+// t^2 fitted by Remez exchange there (within 5e-11).
+__device__ __forceinline__ cd phasor_turns_f64(double x) {
+    const double q = rint(4.0 * x);
+    const double t = fma(-0.25, q, x);
+    const double u = t * t;
+    double s = fma(u, in_sgpr(41.47294862148435), in_sgpr(-76.69786995599631));
+    s = fma(u, s, in_sgpr(81.60520474626004));
+    s = fma(u, s, in_sgpr(-41.341702153504954));
+    s = fma(u, s, in_sgpr(6.283185307152453));
+    s *= t;
+    double c = fma(u, in_sgpr(59.220407311205165), in_sgpr(-85.44285212185385));
+    c = fma(u, c, in_sgpr(64.9393162084543));
+    c = fma(u, c, in_sgpr(-19.73920865035794));
+    c = fma(u, c, in_sgpr(0.9999999999526005));
+    const int qi = (int)q & 3;
+    const double co = (qi & 1) ? s : c, si = (qi & 1) ? c : s;
+    return cd{((qi + 1) & 2) ? -co : co, (qi & 2) ? -si : si};
+}
+
 __device__ __forceinline__ float2 c_scale(float2 a, float w) { return make_float2(a.x * w, a.y * w); }
 
 struct FrameParam {

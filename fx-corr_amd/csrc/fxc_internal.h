@@ -181,14 +181,14 @@ __host__ __device__ inline WkTables wk_tables(const void *tab, int M) {
 }
 inline int wave_frames(int N) { return 8192 / N; }   // frames a workgroup's round holds (N <= 8192)
 // Per-frame values: the XCF phasor of overlap index k is
-// (1 + lam0 + k lam) exp(2 pi i (phw + k dth)), the fringe phasors included
-// (chosen: lam0 = lam = 0), or frmix times the chain's link.
+// (l0 + k lam) exp(2 pi i (phw + k dth)), the fringe phasors included (chosen:
+// l0 = 1, lam = 0), or frmix times the chain's link.
 struct WkParam {
     double phw, dth;
-    float2 C;            // exp(2 pi i (2 phw + (M - 2 gs) dth)): mirror bins
-    float2 F1;           // exp(2 pi i 256 dth): a thread's next pair
+    double l0, lam;
+    double2 C;           // exp(2 pi i (2 phw + (M - 2 gs) dth)): mirror bins
+    float2 F1;           // exp(2 pi i 256 dth): a thread's next pair (chosen)
     float2 frmix;
-    float lam0, lam;
     int16_t s1, s2;      // integer shifts clamped to [-N, N]
     int32_t pad;
 };

@@ -463,7 +463,8 @@ __global__ __launch_bounds__(64) void k_wave_params(SectorArgs a, int precision,
     const int64_t idx = a.first_frame + f;
     WkParam p;
     const int gs = a.grid == 0 ? a.a1s : a.a2s;
-    p.lam0 = p.lam = 0.0f;
+    p.l0 = 1.0;
+    p.lam = 0.0;
     FrameDelayDev d;
     compute_frame_delay(idx, a.dly, d, nullptr, nullptr);
     p.s1 = (int16_t)clamp_shift(d.int1, a.N);
@@ -491,11 +492,12 @@ __global__ __launch_bounds__(64) void k_wave_params(SectorArgs a, int precision,
         const double inv = 0.5 / FXC_PI;
         p.phw = atan2(s.y, s.x) * inv;
         p.dth = atan2((double)sp.y, (double)sp.x) * inv;
-        // ln |x| of values within 1e-7 of 1
-        p.lam0 = (float)(0.5 * (s.x * s.x + s.y * s.y - 1.0));
-        p.lam = (float)(0.5 * ((double)sp.x * sp.x + (double)sp.y * sp.y - 1.0));
+        // |start| |step|^k to first order in ln |.|, for values within 1e-7 of 1
+        p.l0 = 0.5 * (s.x * s.x + s.y * s.y + 1.0);
+        p.lam = 0.5 * ((double)sp.x * sp.x + (double)sp.y * sp.y - 1.0);
     }
-    p.C = sincos_turns((float)wrap_turns(2.0 * p.phw + (double)(a.M - 2 * gs) * p.dth));
+    const cd C = phasor_turns_f64(2.0 * p.phw + (double)(a.M - 2 * gs) * p.dth);
+    p.C = make_double2(C.x, C.y);
     p.F1 = sincos_turns((float)wrap_turns(256.0 * p.dth));
     out[f] = p;
 }
@@ -543,8 +545,9 @@ __device__ __forceinline__ float2 wk_untangle1(float2 a, float2 b, float2 w) {
 // pair are p + sb and M - p + sb, untangled one by one.  PH: the phased sum
 // in place of the ACF / XCF products: per bin the stations' rotations (the
 // reference's f32 chains, or phasors of the FP64 phases), fringe phasors, the
-// weighted sum cb, |cb|^2 and, for the .raw output, cb.
-template <int LOGM, bool MF, bool SHIFT, bool PH>
+// weighted sum cb, |cb|^2 and, for the .raw output, cb.  CHAIN: the XCF takes
+// its phases from the reference's chains (overlaps above 512 bins, plain form).
+template <int LOGM, bool MF, bool SHIFT, bool PH, bool CHAIN>
 __global__ __launch_bounds__(wk::Shape<LOGM>::NT)
 __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
     using Par = std::conditional_t<PH, WkPhased, WkParam>;
@@ -764,6 +767,15 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                 }
             } else {
                 // ---- products of the round's frames (main.rs:2491-2568)
+                // FP64 phasor u of overlap index k with the f32 step's magnitude, rounded to f32
+                auto scaled = [](cd u, const Par &P, int k) {
+                    const double l = fma((double)k, P.lam, P.l0);
+                    return make_float2((float)(u.x * l), (float)(u.y * l));
+                };
+                auto phasor = [&](const Par &P, int k) {   // zero outside the overlap, whose sums are dropped
+                    if ((unsigned)k >= (unsigned)a.ov) return make_float2(0.f, 0.f);
+                    return scaled(phasor_turns_f64(fma((double)k, P.dth, P.phw)), P, k);
+                };
     #pragma unroll 1
                 for (int f = grp; f < nf; f += G) {
                     const Par &P = sh.pp[f];
@@ -771,10 +783,17 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                     // rows of the wave's station-frame q are XORed by q in the
                     // single-pass swizzle
                     const int qx = S::A == 1 ? ((f % S::SPW) & (S::RB - 1)) * S::M2 : 0;
+                    // XCF phasors.  MFMA instances (chosen form): f32 from the
+                    // reduced FP64 phase on.  The others hold them in FP64 to
+                    // the bin, as the plain form's powers of the f32 step are
+                    // rounded there: parts within 2^-25, where an f32
+                    // polynomial, step and mirror product gave up to 1.8e-7.
+                    // 2^27 samples of both stations, plain N = 1024: 386 us
+                    // against 377 (FP64 literals in vector registers and the
+                    // phasor ahead of the untangle: 404)
                     float2 U = make_float2(1.f, 0.f);
-                    const bool chain = a.chain != nullptr;
-                    if (do_xcf && !chain)
-                        U = sincos_turns((float)wrap_turns(fma((double)(pt - gs), P.dth, P.phw)));
+                    if constexpr (MF)
+                        if (do_xcf) U = sincos_turns((float)wrap_turns(fma((double)(pt - gs), P.dth, P.phw)));
     #pragma unroll
                     for (int j = 0; j < PPT; ++j) {
                         const int p = pt + NT * j;
@@ -794,18 +813,22 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                         }
                         if (do_xcf) {
                             float2 Pp, Pm;
-                            if (chain) {
+                            if constexpr (CHAIN) {
                                 const int kp = p - gs, km = M - p - gs;
                                 Pp = c_mul(P.frmix, chain_at(a, fr + f, kp < 0 ? 0 : (kp >= a.ov ? a.ov - 1 : kp)));
                                 Pm = c_mul(P.frmix, chain_at(a, fr + f, km < 0 ? 0 : (km >= a.ov ? a.ov - 1 : km)));
-                            } else {
+                            } else if constexpr (MF) {
                                 Pp = U;
-                                Pm = c_mul(P.C, c_conj(U));
-                                if constexpr (!MF) {   // plain form: the f32 step's magnitude
-                                    Pp = c_scale(Pp, 1.0f + fmaf((float)(p - gs), P.lam, P.lam0));
-                                    Pm = c_scale(Pm, 1.0f + fmaf((float)(M - p - gs), P.lam, P.lam0));
-                                }
+                                Pm = c_mul(make_float2((float)P.C.x, (float)P.C.y), c_conj(U));
                                 if (j + 1 < PPT) U = c_mul(U, P.F1);
+                            } else if constexpr (PPT == 1) {
+                                const cd Ud = phasor_turns_f64(fma((double)(pt - gs), P.dth, P.phw));
+                                const cd Um = d_mul(cd{P.C.x, P.C.y}, cd{Ud.x, -Ud.y});
+                                Pp = scaled(Ud, P, p - gs);
+                                Pm = scaled(Um, P, M - p - gs);
+                            } else {   // overlaps of at most 512 bins: each bin's own
+                                Pp = phasor(P, p - gs);
+                                Pm = phasor(P, M - p - gs);
                             }
                             // station 1 times conj(station 2)
                             const float2 vp = c_mul(gst == 0 ? c_mul(gp, c_conj(xp)) : c_mul(xp, c_conj(gp)), Pp);
@@ -835,12 +858,9 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
                     const int k = M / 2 - gs;
                     if (do_xcf && k >= 0 && k < a.ov) {
                         float2 ph;
-                        if (a.chain != nullptr) {
-                            ph = c_mul(P.frmix, chain_at(a, fr + f, k));
-                        } else {
-                            ph = sincos_turns((float)wrap_turns(fma((double)k, P.dth, P.phw)));
-                            ph = c_scale(ph, 1.0f + fmaf((float)k, P.lam, P.lam0));
-                        }
+                        if constexpr (CHAIN) ph = c_mul(P.frmix, chain_at(a, fr + f, k));
+                        else if constexpr (MF) ph = sincos_turns((float)wrap_turns(fma((double)k, P.dth, P.phw)));
+                        else ph = phasor(P, k);
                         const float2 v = c_mul(gst == 0 ? c_mul(g2, c_conj(x2)) : c_mul(x2, c_conj(g2)), ph);
                         mid[2] += (double)v.x;
                         mid[3] += (double)v.y;
@@ -908,13 +928,13 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void k_sector_wave(SectorArgs a) {
     }
 }
 
-template <int LOGM, bool MF, bool PH>
+template <int LOGM, bool MF, bool PH, bool CHAIN = false>
 static hipError_t launch_wave_t(const SectorArgs &a, int n_wg, hipStream_t s) {
     constexpr size_t lds = sizeof(WkShared<LOGM, std::conditional_t<PH, WkPhased, WkParam>>);
     static_assert(2 * lds <= 160 * 1024 && wk::Shape<LOGM>::NT == 256, "two workgroups per CU");
     const dim3 grid(n_wg), block(wk::Shape<LOGM>::NT);
-    if (a.a1s == a.a2s) hipLaunchKernelGGL((k_sector_wave<LOGM, MF, false, PH>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((k_sector_wave<LOGM, MF, true, PH>), grid, block, lds, s, a);
+    if (a.a1s == a.a2s) hipLaunchKernelGGL((k_sector_wave<LOGM, MF, false, PH, CHAIN>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((k_sector_wave<LOGM, MF, true, PH, CHAIN>), grid, block, lds, s, a);
     return hipGetLastError();
 }
 
@@ -937,13 +957,18 @@ static hipError_t launch_wave_n(const SectorArgs &a, int precision, int n_wg, hi
     if (a.wk_tab == nullptr || a.wk_params == nullptr || a.frames_per_wg % wave_frames(a.N) != 0)
         return hipErrorInvalidValue;
     const bool mf = precision != 0 && a.mf_tab != nullptr;   // the DFT-32 operand table (scale 1)
+    const bool chain = !PH && a.chain != nullptr;            // the phased sum's instances hold both
+    if (chain && (mf || a.N < 2048)) return hipErrorInvalidValue;   // at most 512 bins
     switch (a.N) {
     case 256: return launch_wave_t<7, false, PH>(a, n_wg, s);
     case 512: return launch_wave_t<8, false, PH>(a, n_wg, s);
     case 1024: return mf ? launch_wave_t<9, true, PH>(a, n_wg, s) : launch_wave_t<9, false, PH>(a, n_wg, s);
-    case 2048: return mf ? launch_wave_t<10, true, PH>(a, n_wg, s) : launch_wave_t<10, false, PH>(a, n_wg, s);
-    case 4096: return mf ? launch_wave_t<11, true, PH>(a, n_wg, s) : launch_wave_t<11, false, PH>(a, n_wg, s);
-    case 8192: return mf ? launch_wave_t<12, true, PH>(a, n_wg, s) : launch_wave_t<12, false, PH>(a, n_wg, s);
+    case 2048: return mf ? launch_wave_t<10, true, PH>(a, n_wg, s)
+                    : chain ? launch_wave_t<10, false, PH, !PH>(a, n_wg, s) : launch_wave_t<10, false, PH>(a, n_wg, s);
+    case 4096: return mf ? launch_wave_t<11, true, PH>(a, n_wg, s)
+                    : chain ? launch_wave_t<11, false, PH, !PH>(a, n_wg, s) : launch_wave_t<11, false, PH>(a, n_wg, s);
+    case 8192: return mf ? launch_wave_t<12, true, PH>(a, n_wg, s)
+                    : chain ? launch_wave_t<12, false, PH, !PH>(a, n_wg, s) : launch_wave_t<12, false, PH>(a, n_wg, s);
     default: return hipErrorInvalidValue;
     }
 }
