@@ -1439,9 +1439,9 @@ constexpr int kChainSpanMinLen = 4096;
 // Frames (whole chunks, at least one) whose chains (`len` links, `row_bytes`
 // per frame) one launch computes for a sector of nf frames.
 static bool phased_fused_ok(const fxc_plan *p);
-static int64_t chain_span(int64_t nf, int64_t chunk, size_t row_bytes, int len) {
+static int64_t chain_span(int64_t nf, int64_t chunk, size_t row_bytes, int len, size_t cap = kChainSpanBytes) {
     if (len < kChainSpanMinLen) return chunk;
-    const int64_t fit = std::max<int64_t>(1, (int64_t)(kChainSpanBytes / row_bytes) / chunk);
+    const int64_t fit = std::max<int64_t>(1, (int64_t)(cap / row_bytes) / chunk);
     const int64_t need = (nf + chunk - 1) / chunk;
     return std::min(fit, need) * chunk;
 }
@@ -1892,9 +1892,15 @@ static int64_t large_chunk(const fxc_plan *p) { return large_fused_ok(p) ? p->ch
 // Plain XCF on the fused four-step: the chains of whole chunks, link-major,
 // and the table's size, at least the general path's (a later captured call
 // may need that).
+// N = 16384 holds at most kFusedChainBytes: the walk of 8192 links (131 us) then
+// takes as long as writing its table at 4.1 TB/s, so longer spans gain nothing
+// (a second of 1024 Msps, 62,500 frames, would be 4.1 GB).
+constexpr size_t kFusedChainBytes = (size_t)512 << 20;
 static int64_t fused_chain_span(const fxc_plan *p, int64_t nf) {
     const int ov = (int)(p->desc.a1e - p->desc.a1s);
-    return xcf_uses_chain(p) ? chain_span(nf, p->chunk_use, (size_t)ov * 8, ov) : 0;
+    return xcf_uses_chain(p) ? chain_span(nf, p->chunk_use, (size_t)ov * 8, ov,
+                                          p->fft_form == 2 ? kChainSpanBytes : kFusedChainBytes)
+                             : 0;
 }
 static size_t fused_chain_bytes(const fxc_plan *p, int64_t nf) {
     if (!xcf_uses_chain(p)) return 0;

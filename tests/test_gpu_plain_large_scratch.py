@@ -1,0 +1,38 @@
+"""Device memory of the plain form at N = 16384: the chain table's bound."""
+import numpy as np
+import pytest
+
+import fxcorr as F
+from _synth import LEVELS_2BIT
+
+pytestmark = pytest.mark.gpu
+N, FS = 16384, 256e6
+HALF = N // 2 + 1
+KW = dict(bits=(2, 2), levels=[LEVELS_2BIT, LEVELS_2BIT], df_hz=FS / N, precision=F.PRECISION_PLAIN_FP32)
+
+
+def setup(nf):
+    s = F.Stream()
+    r = [F.DeviceBuffer(nf * N // 4) for _ in range(2)]
+    for st in range(2):
+        F.synth_station_device(r[st].ptr, nf * N, 2, None, False, 5, st, 0.2, 3, s.ptr)
+    cfg = F.make_delay_cfg(np.zeros(8), frame_dt=N / FS, fs=FS, delay_user_samples=3.3, lo1_hz=1e9, lo2_hz=1e9)
+    return s, r, cfg
+
+
+def spectra(p, s, r, cfg, nf):
+    acc = F.DeviceBuffer(F.N_PRODUCTS * HALF * 8)
+    p.sector_run_device(r[0].ptr, r[1].ptr, 0, nf, cfg, acc.ptr, stream=s.ptr)
+    s.sync()
+    return acc.download(np.zeros(F.N_PRODUCTS * HALF))
+
+
+def test_chain_table_bound():
+    nf = 12_000
+    s, r, cfg = setup(nf)
+    p = F.Plan(N, **KW)
+    base = F.plan_device_bytes(p)
+    spectra(p, s, r, cfg, nf)
+    # two Y buffers of 1024 frames, 512 MiB of chains (a link's row: 9 to 24 frames of padding), parameters
+    y, chains = 2 * 1024 * (N // 2) * 8, (8192 + 24) * (N // 2) * 8
+    assert y + chains // 2 < F.plan_device_bytes(p) - base < y + chains + (16 << 20)
