@@ -153,6 +153,7 @@ struct fxc_plan {
     bool mf_b1 = false;   // fft_form 0 / 2: mf_tab holds the DFT-32 operand table (scale 1)
                           // and the FFT's first pass runs on FP16 MFMA
     bool wave = false;    // fft_form 0: variant 0 is the wave kernel (wk_tab holds its tables)
+    bool lean = false;    // no scratch beyond the general paths' (fxc_internal_plan_lean)
     // large-N scratch (fft_form 2): chunk of `chunk` frames
     int M1 = 0, M2 = 0;
     int64_t chunk = 0;       // allocated chunk (frames)
@@ -1146,11 +1147,17 @@ static fxc_status grow(fxc_plan *p, DevBuf &b, size_t bytes, hipStream_t s, cons
         return fail(FXC_ERR_NOMEM, "%s: device allocation of %zu bytes failed", what, bytes);
     return FXC_OK;
 }
-// Whether a call may use `bytes` of the buffer: it holds them or may grow.  The
-// paths that need more scratch than the general ones are left for those where
-// it may not, so that a call a capture or a live graph accepts stays accepted.
-static bool can_hold(const fxc_plan *p, const DevBuf &b, size_t bytes, hipStream_t s) {
-    return bytes <= b.cap || !(p->live_graphs > 0 || stream_capturing(s));
+// Scratch of the paths that need more than the general ones: whether the
+// buffer holds `bytes`, grown to them where it may grow.  Such a path is left
+// for the general one where this says no -- during a capture, under a live
+// graph, in a lean plan, or where the device has no room -- so that a call
+// which runs on the general path's scratch is never refused for more.
+static bool hold(fxc_plan *p, DevBuf &b, size_t bytes, hipStream_t s) {
+    if (bytes <= b.cap) return true;
+    if (p->lean || p->live_graphs > 0 || stream_capturing(s)) return false;
+    if (b.ensure(bytes) == hipSuccess) return true;
+    (void)hipGetLastError();   // the general path's launches check for errors of their own
+    return false;
 }
 #define GROW(p, buf, bytes, s, what)                                  \
     do {                                                              \
@@ -1533,12 +1540,9 @@ static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64
     const size_t chain_b = nch ? std::max((size_t)chunk * nch * ld * 8, g.chain_bytes) : 0;
     const size_t cb_b = raw ? std::max((size_t)chunk * half * 8, g.cb_bytes) : 0;
     const size_t par_b = (size_t)chunk * sizeof(WkPhased);
-    if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s) || !can_hold(p, p->d_wparams, par_b, s))
+    if (!hold(p, p->d_chain, chain_b, s) || !hold(p, p->d_cb, cb_b, s) || !hold(p, p->d_wparams, par_b, s))
         return FXC_OK;
     *done = true;
-    if (nch) GROW(p, p->d_chain, chain_b, s, "phased rotation chains");
-    if (raw) GROW(p, p->d_cb, cb_b, s, "phased spectra");
-    GROW(p, p->d_wparams, par_b, s, "frame parameters");
     const int64_t fpw = frames_per_wg(p, chunk, wave_wg_cap(), true);
     const int n_wg = (int)((chunk + fpw - 1) / fpw);
     for (int64_t c0 = 0; c0 < nf; c0 += chunk) {
@@ -1767,24 +1771,26 @@ static bool fused_for(const fxc_plan *p, int64_t nf) {
     return p->desc.precision == FXC_PRECISION_CHOSEN || nf >= kPlainFusedFrames;
 }
 
-// The plain form's Y and parameter buffers at N = 16384, which short sectors
-// never use: held or able to grow, and their growth.
-static bool fused_ready(const fxc_plan *p, hipStream_t s) {
-    if (p->fft_form == 2 || p->desc.precision == FXC_PRECISION_CHOSEN) return true;
-    const size_t zb = (size_t)p->chunk_use * p->M * 8;
-    return can_hold(p, p->d_z[0], zb, s) && can_hold(p, p->d_z[1], zb, s) &&
-           can_hold(p, p->d_params, (size_t)p->param_cap * std::max(frame_param_bytes(), phased_param_bytes()), s) &&
-           can_hold(p, p->d_lshifts, (size_t)p->param_cap * 16, s);
+// The plain form's Y and parameter buffers at N = 16384, which only this path
+// uses (short sectors never): their sizes, and hold() of them all.
+struct FusedScratch {
+    DevBuf *buf;
+    size_t bytes;
+};
+static std::array<FusedScratch, 4> fused_scratch(fxc_plan *p) {
+    if (p->fft_form == 2 || p->desc.precision == FXC_PRECISION_CHOSEN) return {};   // held from creation on
+    const size_t zb = (size_t)p->chunk_use * p->M * 8, pb = std::max(frame_param_bytes(), phased_param_bytes());
+    return {{{&p->d_z[0], zb}, {&p->d_z[1], zb}, {&p->d_params, p->param_cap * pb},
+             {&p->d_lshifts, (size_t)p->param_cap * 16}}};
 }
-static fxc_status fused_reserve(fxc_plan *p, hipStream_t s) {
-    if (p->fft_form == 2 || p->desc.precision == FXC_PRECISION_CHOSEN) return FXC_OK;
-    const size_t zb = (size_t)p->chunk_use * p->M * 8;
-    GROW(p, p->d_z[0], zb, s, "fused four-step rows");
-    GROW(p, p->d_z[1], zb, s, "fused four-step rows");
-    GROW(p, p->d_params, (size_t)p->param_cap * std::max(frame_param_bytes(), phased_param_bytes()), s,
-         "frame parameters");
-    GROW(p, p->d_lshifts, (size_t)p->param_cap * 16, s, "frame shifts");
-    return FXC_OK;
+static bool fused_hold(fxc_plan *p, hipStream_t s) {
+    const std::array<FusedScratch, 4> need = fused_scratch(p);
+    bool ok = true;
+    for (const FusedScratch &f : need) ok = ok && (!f.buf || hold(p, *f.buf, f.bytes, s));
+    if (!ok && p->live_graphs == 0 && !stream_capturing(s))   // no use for a part of it
+        for (const FusedScratch &f : need)
+            if (f.buf) f.buf->release();
+    return ok;
 }
 
 // Link-major chains: a link's row holds the span's frames and eight more (the
@@ -1819,11 +1825,7 @@ static fxc_status enqueue_phased_fused(fxc_plan *p, const SectorArgs &base, int6
         const PhasedScratch g = phased_scratch(p, nf);
         chain_b = std::max((((size_t)p->half + 7) & ~(size_t)7) * nch * cld * 8, g.chain_bytes);
         if (raw) cb_b = std::max(cb_b, g.cb_bytes);
-        if (!can_hold(p, p->d_chain, chain_b, s) || !can_hold(p, p->d_cb, cb_b, s) || !fused_ready(p, s))
-            return FXC_OK;
-        const fxc_status st = fused_reserve(p, s);
-        if (st != FXC_OK) return st;
-        GROW(p, p->d_chain, chain_b, s, "phased rotation chains");
+        if (!hold(p, p->d_chain, chain_b, s) || !hold(p, p->d_cb, cb_b, s) || !fused_hold(p, s)) return FXC_OK;
     }
     *done = true;
     int64_t cspan0 = -1;
@@ -1916,15 +1918,12 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
     const float2 *twl1 = (const float2 *)(p->M1 == 128 ? p->tw_l1.p : p->tw_l2.p);
     const float2 *twl2 = (const float2 *)(p->M2 == 64 ? p->tw_l0.p : p->M2 == 128 ? p->tw_l1.p : p->tw_l2.p);
     if (fused) {
-        const fxc_status st = fused_reserve(p, s);
-        if (st != FXC_OK) return st;
         const int ng = large_fused_groups(p);
         const int64_t span = fused_param_span(p);
         int64_t span0 = -1;   // first frame (of this sector) of the computed parameters
         const bool plain = p->desc.precision == FXC_PRECISION_PLAIN_FP32;
         const bool chain = xcf_uses_chain(p);
         const int64_t cspan = fused_chain_span(p, nf), cld = chain_links_ld(std::min(cspan, nf));
-        if (chain) GROW(p, p->d_chain, fused_chain_bytes(p, nf), s, "phase chains");
         int64_t cspan0 = -1;
         for (int64_t c0 = 0; c0 < nf; c0 += p->chunk_use) {
             const int64_t cn = std::min(p->chunk_use, nf - c0);
@@ -2014,6 +2013,22 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
     return FXC_OK;
 }
 
+// The job server's view of the ACF/XCF paths above: the bytes a plan may still
+// grow by for them, and whether it may (a lean plan stays on the general ones
+// where its buffers are too small).
+extern "C" uint64_t fxc_internal_plan_optional_bytes(fxc_plan *p) {
+    uint64_t t = 0;
+    auto add = [&t](const DevBuf &b, size_t bytes) { t += bytes > b.cap ? bytes - b.cap : 0; };
+    if (p->wave && p->variant == 0) add(p->d_wparams, (size_t)kWaveSlab * sizeof(WkParam));
+    if (large_fused_ok(p) && p->fft_form == 0 && p->desc.precision == FXC_PRECISION_PLAIN_FP32) {
+        for (const FusedScratch &f : fused_scratch(p))
+            if (f.buf) add(*f.buf, f.bytes);
+        add(p->d_chain, fused_chain_bytes(p, INT64_MAX / 2));
+    }
+    return t;
+}
+extern "C" void fxc_internal_plan_lean(fxc_plan *p, int lean) { p->lean = lean != 0; }
+
 // Plan timing: the events around a sector's kernels (fxc_plan_get_timing)
 static fxc_status timing_begin(fxc_plan *p, hipStream_t s, std::pair<hipEvent_t, hipEvent_t> &ev) {
     if (!p->timing) return FXC_OK;
@@ -2069,8 +2084,8 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     if (phased && p->fft_form == 2) return enqueue_phased_large(p, a, nf, d_raw_out, d_acc, s);
     if (phased) return enqueue_phased(p, a, nf, d_raw_out, d_acc, s);
     // plain: not where its scratch may not grow
-    const bool fused = large_fused_ok(p) && fused_for(p, nf) && fused_ready(p, s) &&
-                       can_hold(p, p->d_chain, fused_chain_bytes(p, nf), s);
+    const bool fused = large_fused_ok(p) && fused_for(p, nf) && hold(p, p->d_chain, fused_chain_bytes(p, nf), s) &&
+                       fused_hold(p, s);
     if (p->fft_form == 2 || (fused && p->desc.precision == FXC_PRECISION_CHOSEN))
         return enqueue_large(p, a, nf, d_acc, fused, s);
     if (fused) {   // plain N = 16384: timed as on the Stockham kernel
@@ -2079,7 +2094,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         return timing_end(p, s, ev);
     }
     const size_t par_b = (size_t)std::min(nf, kWaveSlab) * sizeof(WkParam);
-    const bool wave = wave_for(p, nf) && can_hold(p, p->d_wparams, par_b, s);
+    const bool wave = wave_for(p, nf) && hold(p, p->d_wparams, par_b, s);
     const int wg_cap = std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div);
     // Plain XCF over more than kChainMinOverlap bins: slabs of frames whose
     // f32 phase chains fit the chain scratch; the slabs add into the same
@@ -2093,7 +2108,6 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     }
     // slabs of equal length (a short last one would leave most workgroups idle)
     slab = (nf + (nf + slab - 1) / slab - 1) / ((nf + slab - 1) / slab);
-    if (wave) GROW(p, p->d_wparams, par_b, s, "frame parameters");
     const int64_t fpw = frames_per_wg(p, slab, wg_cap, wave);
     const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;

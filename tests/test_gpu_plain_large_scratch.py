@@ -1,4 +1,5 @@
-"""Device memory of the plain form at N = 16384: the chain table's bound."""
+"""Device memory of the plain form at N = 16384: the chain table's bound, and the
+general kernels where the fused four-step's scratch may not be taken."""
 import numpy as np
 import pytest
 
@@ -36,3 +37,19 @@ def test_chain_table_bound():
     # two Y buffers of 1024 frames, 512 MiB of chains (a link's row: 9 to 24 frames of padding), parameters
     y, chains = 2 * 1024 * (N // 2) * 8, (8192 + 24) * (N // 2) * 8
     assert y + chains // 2 < F.plan_device_bytes(p) - base < y + chains + (16 << 20)
+
+
+def test_lean_plan_runs_the_general_kernels():
+    nf = 700
+    s, r, cfg = setup(nf)
+    p, q = F.Plan(N, **KW), F.Plan(N, **KW)
+    F.plan_set_tuning(q, variant=0)
+    F.lib().fxc_internal_plan_lean(p.h, 1)
+    a, b = spectra(p, s, r, cfg, nf), spectra(q, s, r, cfg, nf)
+    assert np.array_equal(a, b)
+    # rows of the general path alone
+    assert F.plan_device_bytes(p) == F.plan_device_bytes(q)
+    F.lib().fxc_internal_plan_lean(p.h, 0)
+    c = spectra(p, s, r, cfg, nf)
+    assert not np.array_equal(a, c) and np.max(np.abs(a - c)) < 1e-5 * np.max(np.abs(a))
+    assert F.plan_device_bytes(p) > F.plan_device_bytes(q)
