@@ -28,6 +28,8 @@
 
 extern "C" fxc_status fxc_internal_fail(fxc_status s, const char *msg);
 extern "C" const int32_t *fxc_internal_plan_error_word(const fxc_plan *p);
+extern "C" uint64_t fxc_internal_plan_optional_bytes(fxc_plan *p);
+extern "C" void fxc_internal_plan_lean(fxc_plan *p, int lean);
 
 using fxc::kNumProducts;
 using fxc::launch_add_f64;
@@ -126,7 +128,13 @@ struct fxc_server {
     std::deque<uint64_t> pending;
     std::map<uint64_t, std::unique_ptr<Job>> jobs;
     std::multimap<std::string, fxc_plan *> idle_plans;
-    std::map<std::string, std::pair<uint64_t, fxc_plan_info>> key_info;   // plan bytes, info
+    // A plan description's device bytes: with the scratch its longest sectors
+    // may take, and without (a lean plan stays on the paths that need less).
+    struct KeyInfo {
+        uint64_t full, lean;
+        fxc_plan_info info;
+    };
+    std::map<std::string, KeyInfo> key_info;
     uint64_t idle_bytes = 0;
     uint64_t active_bytes = 0;
     int active = 0;
@@ -218,6 +226,15 @@ struct fxc_server {
         return b;
     }
 
+    // Bytes a job's plan is admitted with: the full ones, unless a job of
+    // `extra` bytes besides would then not fit an empty server.
+    uint64_t admit_bytes(fxc_plan *p, uint64_t extra) {
+        const uint64_t held = plan_bytes(p), more = fxc_internal_plan_optional_bytes(p);
+        const bool lean = held + more + extra > cfg.hbm_budget_bytes;
+        fxc_internal_plan_lean(p, lean);
+        return held + (lean ? 0 : more);
+    }
+
     void evict_idle(uint64_t need) {
         trim_pool(need);
         while (!idle_plans.empty() && in_use() + need > cfg.hbm_budget_bytes) {
@@ -231,7 +248,7 @@ struct fxc_server {
     void evict_idle_except(const std::string &key, uint64_t need) {
         trim_pool(need);
         for (auto it = idle_plans.begin(); it != idle_plans.end();) {
-            const uint64_t keep = idle_plans.count(key) ? key_info[key].first : 0;
+            const uint64_t keep = idle_plans.count(key) ? plan_bytes(idle_plans.find(key)->second) : 0;
             if (in_use() - keep + need <= cfg.hbm_budget_bytes) break;
             if (it->first == key) {
                 ++it;
@@ -291,12 +308,18 @@ struct fxc_server {
     bool try_admit(Job &j) {
         auto known = key_info.find(j.key);
         if (known != key_info.end()) {
-            const uint64_t need = known->second.first + job_extra(j, known->second.second);
-            const bool cached = idle_plans.count(j.key) != 0;
-            const uint64_t have = in_use() - (cached ? known->second.first : 0);
+            const KeyInfo &k = known->second;
+            const uint64_t extra = job_extra(j, k.info);
+            const uint64_t need = extra + (k.full + extra <= cfg.hbm_budget_bytes ? k.full : k.lean);
+            // a cached plan's bytes are in use already and part of the need
+            auto cached = [&] {
+                auto it = idle_plans.find(j.key);
+                return it != idle_plans.end() ? plan_bytes(it->second) : 0;
+            };
+            const uint64_t have = in_use() - cached();
             if (have + need > cfg.hbm_budget_bytes) {
                 evict_idle_except(j.key, need);
-                const uint64_t have2 = in_use() - (idle_plans.count(j.key) ? known->second.first : 0);
+                const uint64_t have2 = in_use() - cached();
                 if (have2 + need > cfg.hbm_budget_bytes) {
                     if (active == 0) {
                         fail_job(j, "job footprint exceeds the server's HBM budget");
@@ -307,14 +330,22 @@ struct fxc_server {
             }
         }
         fxc_plan *plan = nullptr;
+        fxc_plan_info info;
         uint64_t pb = 0;
         auto it = idle_plans.find(j.key);
         if (it != idle_plans.end()) {
             plan = it->second;
-            pb = plan_bytes(plan);
             idle_plans.erase(it);
-            idle_bytes -= pb;
-        } else {
+            idle_bytes -= plan_bytes(plan);
+            const uint64_t extra = job_extra(j, known->second.info);
+            pb = admit_bytes(plan, extra);
+            if (pb + extra > cfg.hbm_budget_bytes && known->second.lean < pb) {   // grown past this job: a fresh one
+                fxc_plan_destroy(plan);
+                plan = nullptr;
+            }
+        }
+        const bool fresh = plan == nullptr;
+        if (fresh) {
             fxc_plan_desc d = j.desc.plan;
             d.st[0].levels = j.lev[0].data();
             d.st[1].levels = j.lev[1].data();
@@ -322,11 +353,13 @@ struct fxc_server {
                 fail_job(j, std::string("plan: ") + fxc_last_error());
                 return true;
             }
-            pb = plan_bytes(plan);
         }
-        fxc_plan_info info;
         (void)fxc_plan_get_info(plan, &info);
-        key_info[j.key] = {pb, info};
+        if (fresh) {
+            const uint64_t held = plan_bytes(plan);
+            key_info[j.key] = {held + fxc_internal_plan_optional_bytes(plan), held, info};
+            pb = admit_bytes(plan, job_extra(j, info));
+        }
         j.half = (size_t)info.half;
         const uint64_t acc_bytes = (uint64_t)kNumProducts * j.half * sizeof(double);
         const uint64_t need = pb + job_extra(j, info);
@@ -470,10 +503,12 @@ struct fxc_server {
     void retire(Job &j, bool to_cache) {
         if (j.plan) {
             if (to_cache) {   // scratch may have grown in use: re-learn its size
-                const uint64_t pb = plan_bytes(j.plan);
-                key_info[j.key].first = pb;
+                const uint64_t full = plan_bytes(j.plan) + fxc_internal_plan_optional_bytes(j.plan);
+                KeyInfo &k = key_info[j.key];
+                if (k.lean == k.full) k.lean = full;
+                k.full = full;
                 idle_plans.emplace(j.key, j.plan);
-                idle_bytes += pb;
+                idle_bytes += plan_bytes(j.plan);
             } else {
                 fxc_plan_destroy(j.plan);
             }

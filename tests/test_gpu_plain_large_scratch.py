@@ -1,5 +1,6 @@
-"""Device memory of the plain form at N = 16384: the chain table's bound, and the
-general kernels where the fused four-step's scratch may not be taken."""
+"""Device memory of the plain form at N = 16384: the chain table's bound, the
+general kernels where the fused four-step's scratch may not be taken, and the
+job server's budget counting that scratch before a job's first long sector."""
 import numpy as np
 import pytest
 
@@ -53,3 +54,38 @@ def test_lean_plan_runs_the_general_kernels():
     c = spectra(p, s, r, cfg, nf)
     assert not np.array_equal(a, c) and np.max(np.abs(a - c)) < 1e-5 * np.max(np.abs(a))
     assert F.plan_device_bytes(p) > F.plan_device_bytes(q)
+
+
+@pytest.mark.parametrize("jobs_fit", [1, 0])
+def test_server_budget_counts_the_scratch(jobs_fit):
+    """jobs_fit = 1: the budget holds one job's plan with its scratch, not
+    two.  0: it holds no such plan; the jobs run on the general kernels."""
+    nf = 1200
+    s, r, cfg = setup(nf)
+    probe = F.Plan(N, **KW)
+    held = F.plan_device_bytes(probe)
+    want = spectra(probe, s, r, cfg, nf)
+    grown = F.plan_device_bytes(probe)
+    probe.close()
+    # a job's most: Y, parameters and the whole chain table
+    full = grown + (512 << 20) - 1200 * (N // 2) * 8
+    spectra_bytes = 2 * F.N_PRODUCTS * HALF * 8
+    budget = int(1.5 * full) if jobs_fit else 2 * (held + spectra_bytes) + (8 << 20)
+    sv = F.Server(hbm_budget_bytes=budget, max_active_jobs=4, n_streams=2)
+    jobs = []
+    for _ in range(3):
+        j = sv.submit(dict(KW, fft_len=N), cfg)
+        sv.push(j, r[0].ptr, r[1].ptr, nf)
+        jobs.append(j)
+    for j in jobs:
+        sv.close_job(j)
+    for j in jobs:
+        assert sv.wait(j, 120.0)
+    st = sv.stats()
+    got = [sv.result(j, HALF)[0] for j in jobs]
+    sv.close()
+    assert st.jobs_done == 3 and st.jobs_failed == 0
+    if jobs_fit:
+        assert st.max_concurrent_jobs == 1 and st.peak_hbm_bytes <= budget
+    for g in got:
+        assert np.array_equal(g, got[0]) and np.max(np.abs(g - want)) < 1e-5 * np.max(np.abs(want))
