@@ -789,10 +789,11 @@ static bool wave_eligible(const fxc_plan *p) {
 // 20; plain 1024, 256 frames 19 / 20, 2048 frames 39 / 24; phased plain 512,
 // 512 frames 21 / 28, 4096 frames 45 / 33).  Four frames per CU for the phased
 // sum and from N = 4096 on, two otherwise.
-static bool wave_for(const fxc_plan *p, int64_t nf) {
+static bool wave_long(const fxc_plan *p, int64_t nf) {
     const bool phased = (p->desc.products & (FXC_PRODUCT_PHASED | FXC_PRODUCT_RAW_OUT)) != 0;
-    return p->wave && p->variant == 0 && nf > (int64_t)num_cus() * (p->N <= 2048 && !phased ? 2 : 4);
+    return p->wave && nf > (int64_t)num_cus() * (p->N <= 2048 && !phased ? 2 : 4);
 }
+static bool wave_for(const fxc_plan *p, int64_t nf) { return p->variant == 0 && wave_long(p, nf); }
 
 // The wave kernel's tables (WkTables): twf holds W_M^k.
 static std::vector<uint8_t> wave_tables(const fxc_plan *p, const std::vector<float> &twf) {
@@ -2189,6 +2190,11 @@ extern "C" fxc_status fxc_plan_autotune(fxc_plan *p, const uint8_t *d_raw1, cons
         else
             cands.push_back({1, 1, 0, 0});
     }
+    // A sample so short that the plan's kernel for longer sectors does not run
+    // on it: a candidate would time the general kernels alone, and fixing it
+    // would take that kernel from the longer sectors, unmeasured (up to 2x).
+    // The default, which is the first candidate, stays.
+    if ((p->wave && !wave_long(p, nf)) || (large_fused_possible(p) && !fused_for(p, nf))) cands.resize(1);
     const int save_variant = p->variant, save_div = p->grid_div, save_m1 = p->M1, save_m2 = p->M2;
     const int64_t save_chunk = p->chunk_use;
     const bool save_timing = p->timing;

@@ -429,7 +429,12 @@ fxc_status fxc_plan_device_bytes(const fxc_plan *plan, uint64_t *bytes);
  * producer/consumer waves with FP32 batch sums; N = 2048 has the
  * producer/consumer organization only).  Results are the same sums up to
  * FP64 summation order, or FP32 rounding of the batch sums (about 1e-7 of
- * the spectrum's scale) for the FP32-batch organization. */
+ * the spectrum's scale) for the FP32-batch organization.
+ * A sample too short for the plan's kernel of longer sectors (two or four
+ * frames per compute unit for the wave kernel, 512 for the plain form's fused
+ * four-step) leaves the default, the only candidate then: tune on a sector of
+ * the length that is run.  A report fixes the kernel it names for sectors of
+ * every length, also one kept from before a kernel was added. */
 typedef struct {
     int32_t candidates;
     int32_t variant;           /* Stockham: 0 default (the wave kernel, N = 256..8192
