@@ -1418,8 +1418,21 @@ static bool xcf_uses_chain(const fxc_plan *p) {
 }
 constexpr size_t kChainSlabBytes = (size_t)256 << 20;   // chain scratch of the fused plain path
 
-// Frames of one wave-kernel launch: its parameter table stays below 32 MB.
-constexpr int64_t kWaveSlab = (int64_t)1 << 19;
+// Frames of one wave-kernel launch: at most 2^19, whose parameters (72 bytes a
+// frame) take 38 MB, and 2^30 samples of a station, so that the parameters
+// leave the allocation-free entry's fixed scratch to the partial slots: all 512
+// of them up to N = 4096, 351 at 8192 (with 2^19 frames at every N: 357 at 4096,
+// 178 at 8192).  Each slab costs its workgroups' ramp and tail: slabs of 2^28
+// samples took 2^30 samples at N = 8192, chosen, from 5358 to 5634 us.
+static int64_t wave_slab_max(const fxc_plan *p) {
+    return std::min<int64_t>((int64_t)1 << 19, ((int64_t)1 << 30) / p->N);
+}
+// A sector's slabs of at most `cap` frames, of equal length (a short last one
+// would leave most workgroups idle).
+static int64_t equal_slabs(int64_t nf, int64_t cap) {
+    const int64_t n = (nf + cap - 1) / cap;
+    return (nf + n - 1) / n;
+}
 
 // Frames per workgroup of the fused kernels for a launch of nf frames on at
 // most wg_cap workgroups.  Stockham kernels (one frame pair at a time per
@@ -1532,7 +1545,7 @@ static fxc_status enqueue_phased_wave(fxc_plan *p, const SectorArgs &base, int64
     const int nch = prec ? 0 : (base.dly.table != nullptr ? 1 : 2);
     const int ld = chain_ld_for((int)half);
     const size_t per_frame = (raw ? half * 8 : 0) + (size_t)nch * ld * 8;
-    int64_t chunk = std::min(nf, kWaveSlab);
+    int64_t chunk = std::min(nf, wave_slab_max(p));
     if (per_frame) chunk = std::min<int64_t>(chunk, (int64_t)(kPhasedWaveBytes / per_frame));
     const int64_t nchunks = (nf + chunk - 1) / chunk;
     chunk = (nf + nchunks - 1) / nchunks;
@@ -2020,7 +2033,7 @@ static fxc_status enqueue_large(fxc_plan *p, const SectorArgs &base, int64_t nf,
 extern "C" uint64_t fxc_internal_plan_optional_bytes(fxc_plan *p) {
     uint64_t t = 0;
     auto add = [&t](const DevBuf &b, size_t bytes) { t += bytes > b.cap ? bytes - b.cap : 0; };
-    if (p->wave && p->variant == 0) add(p->d_wparams, (size_t)kWaveSlab * sizeof(WkParam));
+    if (p->wave && p->variant == 0) add(p->d_wparams, (size_t)wave_slab_max(p) * sizeof(WkParam));
     if (large_fused_ok(p) && p->fft_form == 0 && p->desc.precision == FXC_PRECISION_PLAIN_FP32) {
         for (const FusedScratch &f : fused_scratch(p))
             if (f.buf) add(*f.buf, f.bytes);
@@ -2094,7 +2107,7 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
         if ((st = timing_begin(p, s, ev)) != FXC_OK || (st = enqueue_large(p, a, nf, d_acc, fused, s)) != FXC_OK) return st;
         return timing_end(p, s, ev);
     }
-    const size_t par_b = (size_t)std::min(nf, kWaveSlab) * sizeof(WkParam);
+    const size_t par_b = (size_t)std::min(nf, wave_slab_max(p)) * sizeof(WkParam);
     const bool wave = wave_for(p, nf) && hold(p, p->d_wparams, par_b, s);
     const int wg_cap = std::max(1, (wave ? wave_wg_cap() : p->max_wg) / p->grid_div);
     // Plain XCF over more than kChainMinOverlap bins: slabs of frames whose
@@ -2102,13 +2115,12 @@ static fxc_status enqueue_sector(fxc_plan *p, const uint8_t *d_raw1, const uint8
     // workgroup slots in order.
     const bool chain = p->fft_form == 0 && xcf_uses_chain(p);
     const int ld = chain ? chain_ld_for(a.ov) : 0;
-    int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
+    int64_t slab = wave ? std::min(nf, wave_slab_max(p)) : nf;
     if (chain) {
         slab = std::min(slab, chain_slab(p, nf));
         GROW(p, p->d_chain, (size_t)chain_slab(p, nf) * ld * 8, s, "phase chains");
     }
-    // slabs of equal length (a short last one would leave most workgroups idle)
-    slab = (nf + (nf + slab - 1) / slab - 1) / ((nf + slab - 1) / slab);
+    slab = equal_slabs(nf, slab);
     const int64_t fpw = frames_per_wg(p, slab, wg_cap, wave);
     const int n_wg = (int)((slab + fpw - 1) / fpw);
     a.frames_per_wg = fpw;
@@ -2367,7 +2379,7 @@ extern "C" fxc_status fxc_internal_sector_noalloc(fxc_plan *p, const uint8_t *d_
     const size_t per_wg = slot + (p->fft_form == 1 ? kMfConsumerAccBytes : 0);
     // wave kernel: one slab's frame parameters
     const bool wave = wave_for(p, nf);
-    const int64_t slab = wave ? std::min(nf, kWaveSlab) : nf;
+    const int64_t slab = wave ? equal_slabs(nf, wave_slab_max(p)) : nf;   // the plan's
     const size_t par = wave ? ((size_t)slab * sizeof(WkParam) + 255) & ~(size_t)255 : 0;
     const size_t head = table_bytes + par + 256;   // + alignment of the totals
     const int64_t slots = scratch_bytes > head ? (int64_t)((scratch_bytes - head) / per_wg) : 0;
