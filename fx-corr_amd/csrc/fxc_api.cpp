@@ -794,6 +794,8 @@ static bool wave_long(const fxc_plan *p, int64_t nf) {
     return p->wave && nf > (int64_t)num_cus() * (p->N <= 2048 && !phased ? 2 : 4);
 }
 static bool wave_for(const fxc_plan *p, int64_t nf) { return p->variant == 0 && wave_long(p, nf); }
+// for the tests, which run both sides of the line
+extern "C" int fxc_internal_wave_for(const fxc_plan *p, int64_t nf) { return wave_for(p, nf); }
 
 // The wave kernel's tables (WkTables): twf holds W_M^k.
 static std::vector<uint8_t> wave_tables(const fxc_plan *p, const std::vector<float> &twf) {

@@ -3,18 +3,33 @@ the oracle: every size, both stage-1 forms, code widths, shuffles and LSB
 input, shifts inside and past the staging padding and past the frame, band
 offsets on both grids, product subsets, ragged last rounds, and the frame
 counts on both sides of its line against the Stockham kernel."""
+import ctypes
+import functools
+
 import numpy as np
 import pytest
 
 import fxcorr as F
 import fxref as R
 from _cases import gpu_run, make_case, oracle_run, spectra_err
+from _synth import LEVELS_2BIT
 
 pytestmark = pytest.mark.gpu
-LINE = {256: 512, 512: 512, 1024: 512, 2048: 512, 4096: 1024, 8192: 1024}   # frames on 256 CUs
 ACF, XCF, OV = F.PRODUCT_ACF, F.PRODUCT_XCF, F.PRODUCT_ACF_OVERLAP_ONLY
 PERM = np.random.default_rng(4).permutation(32).astype(np.int32)
 SWAP = np.arange(32, dtype=np.int32) ^ 1
+
+
+@functools.lru_cache(None)
+def line(n):
+    """Longest ACF/XCF sector (frames) that stays on the Stockham kernel on this device."""
+    p = F.Plan(n, levels=[LEVELS_2BIT, LEVELS_2BIT], df_hz=64e6 / n)
+    lo, hi = 0, 1 << 16
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if F.lib().fxc_internal_wave_for(p.h, ctypes.c_int64(mid)) else (mid, hi)
+    assert 0 < lo < 1 << 15
+    return lo
 
 
 def check(c, form):
@@ -29,16 +44,16 @@ def check(c, form):
 
 @pytest.mark.parametrize("form", ["plain", "chosen"])
 @pytest.mark.parametrize("n,extra", [(256, 0), (256, 1), (256, 70), (512, 13), (1024, 1), (1024, 260), (2048, 3),
-                                     (4096, 1), (4096, 2), (8192, 1), (8192, 0)])
+                                     (4096, 1), (4096, 2), (8192, 1), (8192, 0), (8192, 515)])
 def test_wave_sizes(n, extra, form):
     # band offset of one bin: also the chosen form leaves the producer/consumer kernels
-    c = make_case(n=n, fs=64e6, nf=LINE[n] + extra, rho=0.2, seed=n + extra, band=(1, 0, n // 2 - 1, 1),
+    c = make_case(n=n, fs=64e6, nf=line(n) + extra, rho=0.2, seed=n + extra, band=(1, 0, n // 2 - 1, 1),
                   delay_user_samples=5.3, extra_delay_rate_sps=3e-8, lo1_hz=6.7e9, lo2_hz=6.7e9)
     check(c, form)
 
 
 @pytest.mark.parametrize("form", ["plain", "chosen"])
-@pytest.mark.parametrize("n", [256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("n", [256, 512, 1024, 2048, 4096, 8192])
 @pytest.mark.parametrize("bits,shuffles,lsb,shift,grid,delay,products", [
     ((1, 8), (None, PERM), (False, True), 0, 0, -70.6, ACF | XCF),
     ((8, 2), (PERM, None), (True, False), 5, 1, 33.2, ACF | XCF),
@@ -50,19 +65,35 @@ def test_wave_options(n, bits, shuffles, lsb, shift, grid, delay, products, form
     m = n // 2
     a1s = max(0, -shift)
     band = (shift, a1s, min(m, m - shift), a1s + shift)
-    c = make_case(n=n, fs=64e6, nf=LINE[n] + 9, bits=bits, shuffles=shuffles, lsb=lsb, band=band, grid=grid,
+    c = make_case(n=n, fs=64e6, nf=line(n) + 9, bits=bits, shuffles=shuffles, lsb=lsb, band=band, grid=grid,
                   products=products, rho=0.3, seed=n, delay_samples=3.0, delay_user_samples=delay,
                   lo1_hz=1.2e9, lo2_hz=1.2e9)
     check(c, form)
 
 
-@pytest.mark.parametrize("n", [256, 2048, 4096])
+@pytest.mark.parametrize("n", [256, 2048, 4096, 8192])
 def test_wave_shift_past_the_frame(n):
     """Station 1 shifted out of most frames: the sweep crosses +-N."""
     fs = 64e6
-    c = make_case(n=n, fs=fs, nf=LINE[n] + 5, rho=0.3, seed=3, delay_user_samples=-1.2 * n, lo1_hz=1e9, lo2_hz=1e9,
-                  extra_delay_rate_sps=2.4 * n / fs / ((LINE[n] + 5) * n / fs))
+    c = make_case(n=n, fs=fs, nf=line(n) + 5, rho=0.3, seed=3, delay_user_samples=-1.2 * n, lo1_hz=1e9, lo2_hz=1e9,
+                  extra_delay_rate_sps=2.4 * n / fs / ((line(n) + 5) * n / fs))
     check(c, "plain")
+
+
+@pytest.mark.parametrize("n,form", [(256, "plain"), (1024, "plain"), (2048, "plain"), (4096, "chosen"), (8192, "plain"),
+                                    (8192, "chosen")])
+def test_wave_grid_divisors(n, form):
+    """The autotuner's configurations of this kernel (variant 0), and the
+    Stockham kernel's radix-16 variant on the same sector."""
+    plain = form == "plain"
+    c = make_case(n=n, fs=64e6, nf=2 * line(n) + 77, rho=0.3, seed=n, delay_user_samples=2.3, lo1_hz=3e9)
+    o = oracle_run(c, R.MODE_F32 if plain else R.MODE_F64)
+    for variant, div in ((0, 1), (0, 2), (0, 4)) + (((1, 1),) if n >= 2048 else ()):
+        p = F.Plan(n, bits=c["bits"], levels=c["levels"], band=c["band"], df_hz=c["fs"] / n, products=c["products"],
+                   precision=F.PRECISION_PLAIN_FP32 if plain else F.PRECISION_CHOSEN)
+        F.plan_set_tuning(p, variant=variant, grid_divisor=div)
+        errs = spectra_err(gpu_run(c, plan=p), o)
+        assert all(e < (1e-5 if plain else 1e-4) for e in errs.values()), (variant, div, errs)
 
 
 @pytest.mark.parametrize("form", ["plain", "chosen"])
