@@ -17,6 +17,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline] [
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import math
 import os
@@ -73,8 +74,10 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_1024msps_2bit_fft1024
 # Issue counts per frame pair of the fused sector kernels, from the counter
 # pass in profiles/sector_kernels_1024msps_2bit_fft1024_kernel_stats.md:
 # (VALU instructions, matrix-busy cycles).  A wave64 VALU instruction takes
-# 4 cycles of its SIMD; MI355X has 1,024 SIMDs at up to 2.4 GHz.
-ISSUE_PER_FRAME = {"k_sector_mf3": (664.8, 512.0), "k_sector_mf3<FP32 batches>": (618.0, 512.0)}
+# 4 cycles of its SIMD; MI355X has 1,024 SIMDs at up to 2.4 GHz (2.2..2.35 under
+# these kernels: the fractions of the cycles actually run are larger, see there).
+ISSUE_PER_FRAME = {"k_sector_mf3": (664.6, 512.0), "k_sector_mf3<FP32 batches>": (618.0, 512.0),
+                   "k_sector_wave": (1263.8, 0.0)}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 COUNTS_FILE = "profiles/sector_kernels_1024msps_2bit_fft1024_kernel_stats.md"
 # fused kernel of each form (the MFMA form by kernel organization variant)
@@ -296,8 +299,9 @@ def issue_fractions(key, frames, launch_ms):
             "issue_counts_source": COUNTS_FILE}
 
 
-def load_traffic(key):
-    """Bytes per launch of a fused kernel from the committed summary."""
+def load_traffic(key, sectors):
+    """Bytes per sector of a fused kernel from the committed summary (one step
+    of `sectors` sectors; a sector may be several launches)."""
     try:
         with open(TRAFFIC_FILE) as fh:
             kern = json.load(fh)["kernels"]
@@ -305,22 +309,23 @@ def load_traffic(key):
         return None
     for name, e in kern.items():
         if key in name:
-            return e.get("traffic_bytes")
+            return e["traffic_bytes"] * e["dispatches"] / sectors
     return None
 
 
-FORM_NAMES = {0: "FP32 wave kernel (N = 256..8192, longer sectors) or Stockham", 1: "FP16-MFMA four-step", 2: "FP32 four-step through HBM"}
-
-
-def form_name(info):
-    """The FFT a plan runs (fxc_plan_info.fft_form / fft_mfma)."""
-    if info.fft_mfma and info.variant == 1 and (info.fft_form == 2 or info.fft_len == 16384):
-        return "fused four-step: decode + FP16-MFMA DFT-128 columns, row DFTs + products"
-    if info.fft_form == 2 and info.fft_mfma:
-        return "four-step through HBM, FP16-MFMA DFT-32 first pass"
-    if info.fft_form == 0 and info.fft_mfma:
-        return "wave kernel, FP16-MFMA DFT-32 columns" if info.fft_len <= 8192 else "Stockham, FP16-MFMA DFT-32 first pass"
-    return FORM_NAMES[info.fft_form]
+def form_name(p, nf):
+    """The FFT a plan runs on a sector of nf frames (fxc_plan_info; equal bands)."""
+    info = p.info
+    if info.variant == 1 and (info.fft_form == 2 or info.fft_len == 16384):
+        columns = "FP16-MFMA" if info.fft_mfma else "FP32"
+        return f"fused four-step: decode + {columns} DFT-128 columns, row DFTs + products"
+    if info.fft_form == 1:
+        return "FP16-MFMA four-step"
+    if info.fft_form == 2:
+        return "four-step through HBM, " + ("FP16-MFMA DFT-32 first pass" if info.fft_mfma else "FP32")
+    if F.lib().fxc_internal_wave_for(p.h, ctypes.c_int64(nf)):
+        return "wave kernel, " + ("FP16-MFMA" if info.fft_mfma else "FP32") + " DFT-32 columns"
+    return "Stockham, " + ("FP16-MFMA DFT-32 first pass" if info.fft_mfma else "FP32")
 
 
 def size_sweep(stream, samples_per_station=1 << 28, reps=5):
@@ -350,7 +355,7 @@ def size_sweep(stream, samples_per_station=1 << 28, reps=5):
             stream.sync()
             el = (time.perf_counter() - t0) / reps
             row[name] = round(nf * n / el / 1e6, 1)
-            row[name + "_fft"] = form_name(p.info)
+            row[name + "_fft"] = form_name(p, nf)
             acc.free()
             p.close()
         d1.free()
@@ -1025,7 +1030,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(r["tflops"], 3),
                      "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(r["tflops"] / FP32_PEAK_TFLOPS, 4),
-                     "traffic": load_traffic(r["kernel"]),
+                     "traffic": load_traffic(r["kernel"], len(sectors)),
                      "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT),
                      "kernel": f"{KERNEL_LABELS[r['kernel']]} ({r['kernel']})",
                      "hbm_frac": round(r["gbs"] / HBM_PEAK_GBS, 4),

@@ -1511,7 +1511,11 @@ static fxc_status enqueue_phased_mf3(fxc_plan *p, const SectorArgs &base, int64_
 // frame: two rotation chains and, for the .raw output, the combined half
 // spectrum (the inverse FFT quantises its time series from LDS; the N * 4 term
 // keeps the chunking of the staged form).  The chunk does not depend on
-// whether .raw is written, so |cb|^2 sums in the same order either way.
+// whether .raw is written, so on this path |cb|^2 sums in the same order either
+// way.  (The wave kernel, the producer/consumer kernel and the fused four-step
+// take chunks or grids of their own for .raw: there the two differ by FP64
+// rounding.  The wave kernel on .raw's chunks without .raw: power alone, 2^27
+// samples, plain N = 8192 824 -> 915 us, chosen 4096 551 -> 584.)
 struct PhasedScratch {
     int64_t chunk, span;
     size_t chain_bytes, cb_bytes;

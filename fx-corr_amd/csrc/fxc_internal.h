@@ -154,7 +154,7 @@ hipError_t launch_delay_eval(const DelayDev &d, int64_t first, int64_t n,
 // Inverse FFT and quantiser in one kernel (phased .raw output, N <= 16384).
 hipError_t launch_irfft_quantise(const SectorArgs &a, const float2 *in, int64_t nframes,
                                  uint8_t *out, bool negate_odd, hipStream_t s);
-// Quantiser over the HBM four-step inverse's complex output (N >= 32768).
+// Quantiser over scaled samples, N floats per frame.
 hipError_t launch_quantise_frames(const SectorArgs &a, const float *in,
                                   int64_t nframes, uint8_t *out,
                                   hipStream_t stream);
@@ -221,12 +221,12 @@ hipError_t launch_scale_add_xcf(double *ac, const double *re, const double *im, 
                                 hipStream_t stream);
 
 // fxc_chain.hip: frames [0, a.nf) of the launch, rows of 2 a.chain_ld
-// floats, real parts then imaginary parts (one XCF chain of a.ov bins, or two phased
-// chains of M+1 bins, per frame).
+// floats, real parts then imaginary parts (one XCF chain of a.ov bins, or
+// a.chains phased chains of M+1 bins, per frame).
+hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t stream);
 // the same chains link-major: link k of frame f's chain c at
 // (((k chains + c) a.chain_ld + f) 2), links up to a multiple of 8
 hipError_t launch_phase_chain_links(const SectorArgs &a, int kind, float *out, hipStream_t stream);
-hipError_t launch_phase_chain(const SectorArgs &a, int kind, float *out, hipStream_t stream);
 
 // fxc_large.hip: N = 32768, 65536 through HBM scratch (four-step M = M1 x M2)
 struct FrameParam;
@@ -295,7 +295,7 @@ hipError_t launch_large_pass2_mac(const SectorArgs &a, const float2 *y1, const f
 // (launch_phased_params).  raw, M2 = 64 (N = 16384): also the first half of
 // the inverse FFT into a.cb_out (M per frame), finished by
 // launch_irfft_cols_quantise (tw_m: W_M table); M2 = 128 / 256: the spectra
-// as rows into a.cb_out (M + 1 per frame), for launch_irfft_rows
+// as rows into a.cb_out (M + 1 per frame), for launch_irfft_rows_quantise
 hipError_t launch_large_pass2_phased(const SectorArgs &a, const float2 *y1, const float2 *y2,
                                      const void *pp, int M1, int M2, const float2 *tw_m2,
                                      const float2 *tw_m, bool raw, int n_groups, int accumulate,

@@ -309,15 +309,6 @@ __global__ __launch_bounds__(256) void k_mac_large(SectorArgs a, const float2 *z
     out[P_12I * half + g] = prev[3] + acc[3];
 }
 
-// Wave-synchronous Stockham FFT of L = 64 E points in LDS (one wave, no
-// workgroup barrier): v[r] = z[lane + 64 r] on entry, natural order in z on
-// return.  Radix E passes (E = 2 or 4), then a radix-2 pass when needed.
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ------------------------------------ FP32 first pass fused with the decode
 // The plain form's first pass of the fused four-step (M1 = 128): workgroup
 // (frame, part p) takes the columns m2 in [64 p, 64 p + 64) of all 128 rows
@@ -701,11 +692,11 @@ __global__ __launch_bounds__(256, PLAIN ? 3 : 4) void k_large_pass2_r16(SectorAr
             for (int r = 1; r < 16; ++r) cur[r] = c_mul(cur[r], twj[r][loop_local(j)]);
 #pragma unroll
             for (int r = 0; r < 16; ++r) z[pad(16 * j + r)] = cur[r];
-            wave_sync_lds();
+            wave_lds_sync();
 #pragma unroll
             for (int r = 0; r < 16; ++r) cur[r] = z[pad(j + 16 * r)];
             dft16(cur);                                  // pass 2
-            wave_sync_lds();
+            wave_lds_sync();
 #pragma unroll
             for (int r = 0; r < 16; ++r) z[pad(j + 16 * r)] = cur[r];   // X[j + 16 r]
         }
@@ -867,13 +858,13 @@ __global__ __launch_bounds__(256, PLAIN ? (MODE == P2_PRODUCTS ? 4 : 3) : M2 == 
             for (int r = 1; r < E; ++r) cur[r] = c_mul(cur[r], M2 == 64 ? tw[r] : twj[r][loop_local(j)]);
 #pragma unroll
             for (int r = 0; r < E; ++r) z[pad(8 * r + j)] = cur[r];
-            wave_sync_lds();
+            wave_lds_sync();
             float2 u[E / 8][8];
 #pragma unroll
             for (int h = 0; h < E / 8; ++h)
 #pragma unroll
                 for (int r = 0; r < 8; ++r) u[h][r] = z[pad(8 * (j + 8 * h) + r)];
-            wave_sync_lds();
+            wave_lds_sync();
 #pragma unroll
             for (int h = 0; h < E / 8; ++h) {
                 dftR<8>(u[h]);                           // pass 2
@@ -1030,11 +1021,11 @@ __global__ __launch_bounds__(256, PLAIN ? 3 : 4) void k_large_pass2_r8_ph(Sector
             for (int r = 1; r < 8; ++r) cur[r] = c_mul(cur[r], tw[r]);
 #pragma unroll
             for (int r = 0; r < 8; ++r) z[pad(8 * j + r)] = cur[r];
-            wave_sync_lds();
+            wave_lds_sync();
 #pragma unroll
             for (int r = 0; r < 8; ++r) cur[r] = z[pad(j + 8 * r)];
             dftR<8>(cur);                                // pass 2
-            wave_sync_lds();
+            wave_lds_sync();
 #pragma unroll
             for (int r = 0; r < 8; ++r) z[pad(j + 8 * r)] = cur[r];   // X[j + 8 r]
         }
@@ -1089,14 +1080,14 @@ __global__ __launch_bounds__(256, PLAIN ? 3 : 4) void k_large_pass2_r8_ph(Sector
                 for (int r = 1; r < 8; ++r) v[r] = c_mul(v[r], tw[r]);
 #pragma unroll
                 for (int r = 0; r < 8; ++r) zs[pad(8 * j + r)] = v[r];
-                wave_sync_lds();
+                wave_lds_sync();
 #pragma unroll
                 for (int r = 0; r < 8; ++r) v[r] = zs[pad(j + 8 * r)];
                 dftR<8>(v);                                  // pass 2: outputs n2 = j + 8 r
                 float2 *bo = a.cb_out + (it + s3) * (int64_t)M + row * M2;
 #pragma unroll
                 for (int r = 0; r < 8; ++r) bo[j + 8 * r] = c_mul(v[r], twr[b][j + 8 * r]);
-                wave_sync_lds();
+                wave_lds_sync();
             }
         }
 #pragma unroll

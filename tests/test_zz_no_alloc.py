@@ -48,9 +48,9 @@ def _acc(buf, half):
 CASES = [
     # fft, precision, bits, lsb2 + shuffle, frames of the two calls
     (1024, F.PRECISION_CHOSEN, 2, True, (120000, 37001)),     # fused k_sector_mf3
-    (1024, F.PRECISION_PLAIN_FP32, 2, True, (60000, 20003)),  # plain fused k_sector
-    (4096, F.PRECISION_CHOSEN, 2, False, (9000, 4001)),       # Stockham, MFMA first pass
-    (512, F.PRECISION_PLAIN_FP32, 4, False, (30000, 777)),    # plain, 4-bit
+    (1024, F.PRECISION_PLAIN_FP32, 2, True, (60000, 20003)),  # plain, wave kernel
+    (4096, F.PRECISION_CHOSEN, 2, False, (9000, 4001)),       # chosen, wave kernel
+    (512, F.PRECISION_PLAIN_FP32, 4, False, (30000, 777)),    # plain, wave kernel, 4-bit
 ]
 
 
