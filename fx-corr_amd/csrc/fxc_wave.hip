@@ -451,6 +451,11 @@ __device__ __forceinline__ void wk_fft(float2 *z, const int *sht, const float2 *
     }
 }
 
+// The chosen form's DFT-32 on MFMA: the operand table (scale 1), N >= 1024.
+__host__ __device__ inline bool wave_mfma(const SectorArgs &a, int precision) {
+    return precision != 0 && a.mf_tab != nullptr && a.N >= 1024;
+}
+
 // The frames' parameters, one thread each, ahead of the sector kernel: in it
 // the FP64 phases (eight sines and cosines and two arctangents in the plain
 // form) would be a serial stretch of a few lanes per workgroup.  k_sector's
@@ -496,8 +501,14 @@ __global__ __launch_bounds__(64) void k_wave_params(SectorArgs a, int precision,
         p.l0 = 0.5 * (s.x * s.x + s.y * s.y + 1.0);
         p.lam = 0.5 * ((double)sp.x * sp.x + (double)sp.y * sp.y - 1.0);
     }
-    const cd C = phasor_turns_f64(2.0 * p.phw + (double)(a.M - 2 * gs) * p.dth);
-    p.C = make_double2(C.x, C.y);
+    const double mirror = 2.0 * p.phw + (double)(a.M - 2 * gs) * p.dth;
+    if (wave_mfma(a, precision)) {   // taken as f32 (k_sector_wave)
+        const float2 C = sincos_turns((float)wrap_turns(mirror));
+        p.C = make_double2(C.x, C.y);
+    } else {
+        const cd C = phasor_turns_f64(mirror);
+        p.C = make_double2(C.x, C.y);
+    }
     p.F1 = sincos_turns((float)wrap_turns(256.0 * p.dth));
     out[f] = p;
 }
@@ -956,7 +967,7 @@ template <bool PH>
 static hipError_t launch_wave_n(const SectorArgs &a, int precision, int n_wg, hipStream_t s) {
     if (a.wk_tab == nullptr || a.wk_params == nullptr || a.frames_per_wg % wave_frames(a.N) != 0)
         return hipErrorInvalidValue;
-    const bool mf = precision != 0 && a.mf_tab != nullptr;   // the DFT-32 operand table (scale 1)
+    const bool mf = wave_mfma(a, precision);
     const bool chain = !PH && a.chain != nullptr;            // the phased sum's instances hold both
     if (chain && (mf || a.N < 2048)) return hipErrorInvalidValue;   // at most 512 bins
     switch (a.N) {
