@@ -28,16 +28,18 @@
 // zero-padded row that byte tables decode into, as in the MFMA kernels; the
 // integer shift is an offset into it.  The row shares the Z slot's memory.
 //
-// Bound by VALU issue: at N = 1024 1,231 VALU instructions per frame pair (the
-// Stockham kernel: 2,973; half of the 1,231 are the DFTs' additions), 73 % of
+// Bound by VALU issue: at N = 1024 1,264 VALU instructions per frame pair (the
+// Stockham kernel: 2,973; half of the 1,264 are the DFTs' additions), 75 % of
 // its SIMD cycles; HBM and the LDS are far from their rates.  Two waves per
 // SIMD, because 32 points, the FP64 sums and the twiddles of a lane take
-// 180..256 VGPRs.  2^27 samples per station, 2-bit, Stockham kernel -> this
-// one (microseconds; plain from N = 2048 with the phase chains): plain 256:
-// 1051 -> 369, 512: 973 -> 362, 1024: 776 -> 359, 2048: 1146 -> 638, 4096: 1510
-// -> 748, 8192: 1695 -> 911; chosen 4096: 709 -> 498, 8192: 908 -> 730; phased
-// power, plain 256: 1675 -> 656, 1024: 1264 -> 632, 4096: 1559 -> 809; chosen
-// 2048: 694 -> 468, 4096: 792 -> 548, 8192: 1067 -> 584.
+// 180..256 VGPRs; from N = 4096 on they leave a third to a half of the cycles
+// to LDS latency and, at 8192, the transform's barriers.  2^27 samples per
+// station, 2-bit, whole calls, Stockham kernel -> this one (microseconds; plain
+// from N = 2048 with the phase chains): plain 256: 1052 -> 399, 512: 975 ->
+// 378, 1024: 778 -> 390, 2048: 1456 -> 629, 4096: 1604 -> 750, 8192: 1340 ->
+// 899; chosen 4096: 710 -> 491, 8192: 912 -> 736; phased power, plain 256: 1677
+// -> 663, 1024: 1266 -> 637, 4096: 1560 -> 818; chosen 2048: 697 -> 472, 4096:
+// 791 -> 552, 8192: 1068 -> 584.
 #include <type_traits>
 
 #include "fxc_dev.h"

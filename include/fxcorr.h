@@ -513,7 +513,9 @@ fxc_status fxc_plan_check_device_error(fxc_plan *plan, void *stream);
 /* ----------------------------------------------------------------------- */
 typedef struct fxc_server fxc_server;
 typedef struct {
-    uint64_t hbm_budget_bytes;  /* admission budget for plans + input windows + spectra */
+    uint64_t hbm_budget_bytes;  /* admission budget for plans (with the scratch their longest
+                                   sectors take; a plan that fits only without it runs on
+                                   kernels that need none) + input windows + spectra */
     int32_t max_active_jobs;    /* concurrent job slots */
     int32_t n_streams;          /* HIP streams the jobs are spread over (1..4) */
 } fxc_server_cfg;
