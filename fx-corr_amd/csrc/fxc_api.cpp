@@ -1420,12 +1420,13 @@ static bool xcf_uses_chain(const fxc_plan *p) {
 }
 constexpr size_t kChainSlabBytes = (size_t)256 << 20;   // chain scratch of the fused plain path
 
-// Frames of one wave-kernel launch: at most 2^19, whose parameters (72 bytes a
-// frame) take 38 MB, and 2^30 samples of a station, so that the parameters
+// Frames of one wave-kernel launch: at most 2^19, whose parameters (80 bytes a
+// frame) take 42 MB, and 2^30 samples of a station, so that the parameters
 // leave the allocation-free entry's fixed scratch to the partial slots: all 512
-// of them up to N = 4096, 351 at 8192 (with 2^19 frames at every N: 357 at 4096,
-// 178 at 8192).  Each slab costs its workgroups' ramp and tail: slabs of 2^28
+// of them up to N = 4096, 345 at 8192 (with 2^19 frames at every N: 306 at 4096,
+// 153 at 8192).  Each slab costs its workgroups' ramp and tail: slabs of 2^28
 // samples took 2^30 samples at N = 8192, chosen, from 5358 to 5634 us.
+static_assert(sizeof(WkParam) <= 80 && sizeof(WkPhased) <= 80, "wave_slab_max's account");
 static int64_t wave_slab_max(const fxc_plan *p) {
     return std::min<int64_t>((int64_t)1 << 19, ((int64_t)1 << 30) / p->N);
 }

@@ -1029,7 +1029,8 @@ def test_large_chunking_is_a_sum():
 # ---------------------------------------------------------------- autotuner
 @pytest.mark.parametrize("n,variant,div", [(2048, 1, 1), (4096, 1, 2), (8192, 0, 4), (8192, 1, 1)])
 def test_tuning_candidates_keep_parity(n, variant, div):
-    """Every configuration the autotuner can pick gives the same spectra."""
+    """Every configuration the autotuner can pick gives the same spectra (a
+    sector below the wave kernel's line; above it: test_wave_grid_divisors)."""
     c = make_case(n=n, fs=128e6, nf=max(128, 2 ** 19 // n), rho=0.5, seed=n + variant,
                   delay_user_samples=2.3, lo1_hz=3e9)
     o64 = oracle_run(c, R.MODE_F64)
